@@ -32,6 +32,7 @@
 
 #include "nc_common.h"
 #include "nc_internal.h"
+#include "nc_group.h"
 #include "nc_kernels.h"
 
 using nc::fail;
@@ -191,7 +192,7 @@ struct NetMaps {
 // network's own first slot, slice and out-edge.  nc_sim_add relocates it
 // (host offsets for the per-neuron rows, k_relocate_edges for the edges).
 struct NetImage {
-  uint32_t nq = 0;
+  uint32_t nq = 0, max_mw = 0;  // slices; most active-mask words of a lane
   uint64_t S = 0, nslots = 0, nmwords = 0, mwords_step = 0;
   std::vector<uint32_t> slice_off, slice_moff;  // per slice: first slot, first mask word
   std::vector<float> slot_w;                    // nslots weights (0 on padding slots)
@@ -245,6 +246,7 @@ std::shared_ptr<const NetImage> build_image(const nc_net& net) {
       I.slice_moff[q] = (uint32_t)mo;
       o += L.slice_slots[q];
       mo += L.slice_mwords[q];
+      I.max_mw = std::max(I.max_mw, L.slice_mwords[q] / 64);
     }
   }
   uint64_t h = 1469598103934665603ull;
@@ -375,6 +377,7 @@ struct NetRec {
   uint64_t S = 0;
   uint32_t q0 = 0, nq = 0;
   uint64_t slot0 = 0, nslots = 0, out0 = 0, mask0 = 0, nmwords = 0;
+  uint32_t max_mw = 0;  // most active-mask words of a lane
   uint32_t act0 = 0;  // first record of this network in the active-slice list
   bool act_valid = false;    // the device active-slice list holds this network's records at act0
   uint64_t mwords_step = 0;  // active-mask words k_neuron reads per step
@@ -436,6 +439,7 @@ struct nc_sim {
   uint32_t* slice_moff = nullptr;  // per slice: first active-mask word
   uint32_t *slice_off = nullptr, *slice_net = nullptr;
   nc_slice_rec* active = nullptr;
+  nc_net_rec* net_recs = nullptr;  // live networks with neurons, for the workgroup-per-network form
   uint32_t *forced_in = nullptr, *forced_bg = nullptr;
   uint4* fired = nullptr;
   uint32_t* fired_cnt = nullptr;
@@ -453,6 +457,8 @@ struct nc_sim {
   uint32_t graph_key[5] = {0, 0, 0, 0, 0};
   nc_netdesc* d_nets = nullptr;
   float *t_pre = nullptr, *t_post = nullptr, *w_ap = nullptr;
+  uint64_t calls = 0;   // nc_sim_step calls, numbering the activity reports
+  bool busy = false;    // the last report read back (step_form)
   DevBuf<nc_group> d_groups;
   DevBuf<uint32_t> d_gfire;
   DevBuf<float> d_wbuf;       // packed weights of one network, for host reads
@@ -460,6 +466,7 @@ struct nc_sim {
   DevBuf<uint32_t> d_thr;
   DevBuf<uint32_t> d_ev_pos;
   DevBuf<uint8_t> d_ev_kind;
+  DevBuf<uint32_t> d_ev_step;
 
   // Drive group table and threshold tables: ranges per network, reused after
   // removal (freed groups point at the never-live network max_nets).
@@ -467,6 +474,8 @@ struct nc_sim {
   std::vector<uint32_t> thr;
   RangeAlloc a_groups, a_thr;
   std::vector<nc_slice_rec> active_host;
+  std::vector<nc_net_rec> net_recs_host;
+  uint32_t live_nq = 0, live_mw = 0;  // most slices of a live network; most mask words of a lane
   std::vector<uint32_t> slice_off_host, slice_moff_host;
   bool active_dirty = true;
   std::vector<uint32_t> slice_net_host;
@@ -478,6 +487,7 @@ struct nc_sim {
   std::vector<nc_netdesc> h_nds;
   std::vector<uint32_t> h_ev_pos;
   std::vector<uint8_t> h_ev_kind;
+  std::vector<uint32_t> h_ev_step;
   hipEvent_t upload_done = nullptr;
   bool upload_pending = false;
 };
@@ -568,8 +578,7 @@ nc_step_args base_args(nc_sim* sim) {
 // that record i is slice q0 + i and the kernels' per-neuron loads need not
 // wait for the record; otherwise every slice of every live network,
 // networks in id order (each network's slices are contiguous).
-nc_status rebuild_active(nc_sim* sim) {
-  if (!sim->active_dirty) return NC_OK;
+nc_status rebuild_slices(nc_sim* sim) {
   if (sim->upload_pending) {
     NC_HIP(hipEventSynchronize(sim->upload_done));
     sim->upload_pending = false;
@@ -601,7 +610,6 @@ nc_status rebuild_active(nc_sim* sim) {
     sim->act_q0 = qmin;
     NC_HIP(hipMemcpy(sim->active, sim->active_host.data(), sim->active_host.size() * sizeof(nc_slice_rec),
                      hipMemcpyHostToDevice));
-    sim->active_dirty = false;
     return NC_OK;
   }
   for (size_t i = 0; i < sim->nets.size(); ++i) {
@@ -619,6 +627,25 @@ nc_status rebuild_active(nc_sim* sim) {
   if (!sim->active_host.empty())
     NC_HIP(hipMemcpy(sim->active, sim->active_host.data(), sim->active_host.size() * sizeof(nc_slice_rec),
                      hipMemcpyHostToDevice));
+  return NC_OK;
+}
+
+nc_status rebuild_active(nc_sim* sim) {
+  if (!sim->active_dirty) return NC_OK;
+  nc_status st = rebuild_slices(sim);
+  if (st != NC_OK) return st;
+  sim->net_recs_host.clear();
+  sim->live_nq = sim->live_mw = 0;
+  for (size_t i = 0; i < sim->nets.size(); ++i) {
+    const NetRec& r = sim->nets[i];
+    if (!r.live || r.nq == 0) continue;
+    sim->net_recs_host.push_back(nc_net_rec{r.act0, r.nq, (uint32_t)i, 0u});
+    sim->live_nq = std::max(sim->live_nq, r.nq);
+    sim->live_mw = std::max(sim->live_mw, r.max_mw);
+  }
+  if (!sim->net_recs_host.empty())
+    NC_HIP(hipMemcpy(sim->net_recs, sim->net_recs_host.data(), sim->net_recs_host.size() * sizeof(nc_net_rec),
+                     hipMemcpyHostToDevice));
   sim->active_dirty = false;
   return NC_OK;
 }
@@ -629,13 +656,14 @@ nc_status reserve_events(nc_sim* sim) {
   size_t total = 0;
   for (const NetRec& r : sim->nets)
     if (r.live) total += r.events.size();
-  if (total <= sim->d_ev_pos.n && total <= sim->d_ev_kind.n) return NC_OK;
+  if (total <= sim->d_ev_pos.n && total <= sim->d_ev_kind.n && total <= sim->d_ev_step.n) return NC_OK;
   if (sim->upload_pending) {
     NC_HIP(hipEventSynchronize(sim->upload_done));
     sim->upload_pending = false;
   }
   nc_status st = grow(&sim->d_ev_pos, total, sim->stream);
   if (st == NC_OK) st = grow(&sim->d_ev_kind, total, sim->stream);
+  if (st == NC_OK) st = grow(&sim->d_ev_step, total, sim->stream);
   return st;
 }
 
@@ -769,6 +797,7 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
     H(hipMalloc(&sim->slice_off, Q * 4), "hipMalloc slice_off");
     H(hipMalloc(&sim->slice_net, Q * 4), "hipMalloc slice_net");
     H(hipMalloc(&sim->active, Q * sizeof(nc_slice_rec)), "hipMalloc active");
+    H(hipMalloc(&sim->net_recs, sim->max_nets * sizeof(nc_net_rec)), "hipMalloc network records");
     H(hipMalloc(&sim->forced_in, (P / 32) * 4), "hipMalloc forced_in");
     H(hipMalloc(&sim->forced_bg, (P / 32) * 4), "hipMalloc forced_bg");
     H(hipMalloc(&sim->fired, (Q + NC_FLISTS * 8ull) * NC_FSPLIT * sizeof(uint4)), "hipMalloc fired");
@@ -779,7 +808,8 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
     sim->ctr_rows = Q + 2;
     // word 0: chunk offset; word 32: grid-barrier arrivals of the call;
     // word 64: a grid barrier timed out (sticky until reported); word 128:
-    // zero, the group-spike-train word read when there are no groups
+    // zero, the group-spike-train word read when there are no groups; word
+    // 160: the activity report of the newest call
     H(hipMalloc(&sim->d_chunk_off, 1024), "hipMalloc chunk_off");
     H(hipMalloc(&sim->ctr, sim->ctr_rows * NC_NCTR * 8), "hipMalloc ctr");
     // one more, never written: the (never live) network of hole records
@@ -824,10 +854,10 @@ extern "C" void nc_sim_destroy(nc_sim* sim) {
   if (sim->stream) (void)hipStreamSynchronize(sim->stream);
   if (sim->graph) (void)hipGraphExecDestroy(sim->graph);
   void* ptrs[] = {sim->d_chunk_off, sim->amask, sim->asum, sim->slots, sim->V, sim->last_fire, sim->firings, sim->ndw,
-                  sim->nid, sim->out_row, sim->edges, sim->pend0, sim->pend1, sim->pend_cnt, sim->bcnt, sim->bent, sim->acache, sim->slice_moff, sim->id_pos, sim->id_row, sim->slice_off, sim->slice_net, sim->active, sim->forced_in,
+                  sim->nid, sim->out_row, sim->edges, sim->pend0, sim->pend1, sim->pend_cnt, sim->bcnt, sim->bent, sim->acache, sim->slice_moff, sim->id_pos, sim->id_row, sim->slice_off, sim->slice_net, sim->active, sim->net_recs, sim->forced_in,
                   sim->forced_bg, sim->fired, sim->fired_cnt, sim->raster, sim->raster_cnt,
                   sim->ctr, sim->d_nets, sim->t_pre, sim->t_post, sim->w_ap, sim->d_groups.p,
-                  sim->d_thr.p, sim->d_ev_pos.p, sim->d_ev_kind.p, sim->d_gfire.p, sim->d_wbuf.p, sim->d_stage.p};
+                  sim->d_thr.p, sim->d_ev_pos.p, sim->d_ev_kind.p, sim->d_ev_step.p, sim->d_gfire.p, sim->d_wbuf.p, sim->d_stage.p};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : sim->ev_pool) (void)hipEventDestroy(e);
@@ -933,6 +963,7 @@ extern "C" nc_status nc_sim_add(nc_sim* sim, const nc_net* net, const nc_params*
   r.out0 = o0;
   r.mask0 = mk0;
   r.nmwords = I.nmwords;
+  r.max_mw = I.max_mw;
   r.lr = p.learning_rate;
   r.pre_f = p.pre_factor;
   r.post_f = p.post_factor;
@@ -1141,6 +1172,61 @@ extern "C" nc_status nc_sim_remove(nc_sim* sim, int32_t net_id) try {
 }
 NC_ABI_CATCH
 
+namespace {
+// The form of the step kernels a call takes.  A launch shape the caller chose
+// is used as it is, and the device counters are k_neuron's; at the default
+// shape the sizes decide, and, where the better form depends on how much
+// fires, the activity that the device last reported (no form changes a
+// result).  The lines, us per step of either side (a network's slices are
+// 64 neurons each; "busy": a fifth of the neurons fire):
+//   - networks of up to 16 slices, a workgroup each: 300 neurons 2.1 against
+//     6.9 (k_neuron and k_fanout launches), 1000 quiet neurons 3.3 against
+//     8.2, 1024 busy networks of 200-1000 neurons 108 against 181.  One
+//     compute unit per network bounds it: a busy network of 10 slices takes
+//     15.2 here and 21.2 in the wide form, one of 16 slices 23.6 and 21.7,
+//     64 of 3-16 slices 41 and 35, 256 of them 47 and 54.
+//   - up to 1024 slices, four waves a slice: 20 000 busy neurons 26.9 against
+//     49.8 of k_neuron, 60 000 quiet ones 11.5 against 12.4.
+//   - up to 4096 slices, two waves, if busy (2700 slices: 85 against 113);
+//     1563 quiet slices take 13.6 against 12.0 of k_neuron.
+//   - above, one wave, if busy (19 200 slices: 464 against 487); 10^6 quiet
+//     neurons take 91.7 against 87.4 of k_neuron.
+struct Form {
+  bool network = false;     // k_net_steps
+  uint32_t wide_waves = 0;  // k_neuron_wide with this many waves per slice (0: k_neuron)
+};
+
+Form step_form(const nc_sim* sim) {
+  Form f;
+  const nc_launch_cfg& c = sim->cfg;
+  if (c.waves_per_block != 4 || c.xcd_swizzle || c.graph_steps || c.stage_tables || c.fanout_waves || c.persistent)
+    return f;
+  if (sim->counting || sim->live_mw > NC_GW) return f;
+  const size_t slices = sim->active_host.size();
+  if (sim->live_nq <= 16 && !sim->kernel_timing && sim->T.t_pre.size() <= NC_GTAB &&
+      sim->T.t_post.size() <= NC_GTAB && !(sim->busy && sim->live_nq > 12 && slices <= 1024)) {
+    f.network = true;
+    return f;
+  }
+  if (slices <= 1024) f.wide_waves = 4;
+  else if (sim->busy) f.wide_waves = slices <= 4096 ? 2 : 1;
+  return f;
+}
+
+// Steps c0 .. c0 + len - 1 of a call in the workgroup-per-network form.
+template <int NSL, int W>
+nc_status launch_networks(nc_sim* sim, const nc_step_args& a, uint32_t c0, uint32_t len) {
+  const void* fn = (const void*)k_net_steps<NSL, W>;
+  const uint32_t lds = sizeof(nc_gsh<NSL, W, true>);
+  const nc_net_rec* nets = sim->net_recs;
+  const uint32_t* ev_step = sim->d_ev_step.p;
+  void* args[] = {const_cast<nc_step_args*>(&a), &nets, &ev_step, &c0, &len};
+  if (lds > 65536) NC_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  NC_HIP(hipLaunchKernel(fn, dim3((uint32_t)sim->net_recs_host.size()), dim3(64 * W), args, lds, sim->stream));
+  return NC_OK;
+}
+}  // namespace
+
 extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   if (!sim) return fail(NC_ERR_ARG, "null sim");
   if (n_steps == 0) return NC_OK;
@@ -1191,9 +1277,13 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   }
   NC_HIP(hipMemcpyAsync(sim->d_nets, nds.data(), nds.size() * sizeof(nc_netdesc), hipMemcpyHostToDevice, st));
 
+  const Form form = step_form(sim);
+
   // Host-scheduled events for steps [1, max_run] of this call, per step.
   std::vector<uint32_t>& ev_pos = sim->h_ev_pos;
   std::vector<uint8_t>& ev_kind = sim->h_ev_kind;
+  std::vector<uint32_t>& ev_step = sim->h_ev_step;
+  ev_step.clear();
   ev_pos.clear();
   ev_kind.clear();
   std::vector<uint32_t> ev_ptr(max_run + 1, 0);
@@ -1216,15 +1306,18 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       for (auto& e : per[k]) {
         ev_pos.push_back(e.first);
         ev_kind.push_back(e.second);
+        ev_step.push_back(k);
       }
     }
   }
   if (!ev_pos.empty()) {
     // nc_push_forced and nc_sim_restore reserve room for every queued event
-    if (sim->d_ev_pos.n < ev_pos.size() || sim->d_ev_kind.n < ev_kind.size())
+    if (sim->d_ev_pos.n < ev_pos.size() || sim->d_ev_kind.n < ev_kind.size() || sim->d_ev_step.n < ev_step.size())
       return fail(NC_ERR_STATE, "event buffer smaller than the queued events");
     NC_HIP(hipMemcpyAsync(sim->d_ev_pos.p, ev_pos.data(), ev_pos.size() * 4, hipMemcpyHostToDevice, st));
     NC_HIP(hipMemcpyAsync(sim->d_ev_kind.p, ev_kind.data(), ev_kind.size(), hipMemcpyHostToDevice, st));
+    if (form.network)
+      NC_HIP(hipMemcpyAsync(sim->d_ev_step.p, ev_step.data(), ev_step.size() * 4, hipMemcpyHostToDevice, st));
   }
   NC_HIP(hipEventRecord(sim->upload_done, st));
   sim->upload_pending = true;
@@ -1300,6 +1393,16 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, st, bar, 1u, 0u);
     NC_HIP(hipGetLastError());
   }
+  switch (form.wide_waves) {
+    case 1: fn_neuron = (const void*)k_neuron_wide<1>; break;
+    case 2: fn_neuron = (const void*)k_neuron_wide<2>; break;
+    case 4: fn_neuron = (const void*)k_neuron_wide<4>; break;
+    default: break;
+  }
+  const uint32_t n_grid = form.wide_waves ? a.n_active_slices : grid;
+  const uint32_t n_block = 64 * (form.wide_waves ? form.wide_waves : wpb);
+  a.activity = sim->d_chunk_off + 160;
+  const uint32_t call_tag = (uint32_t)(++sim->calls & 0x7FFFFFFFu) << 1;
   hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, st, sim->d_chunk_off, 1u, 0u);
   NC_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_zero_strided, dim3(1), dim3(2 * NC_FLISTS), 0, st, sim->fired_cnt, 2u * NC_FLISTS,
@@ -1328,7 +1431,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   };
   // Whole chunks as captured graphs when nothing per-step comes from the host.
   const uint32_t G =
-      (sim->cfg.graph_steps && ev_pos.empty() && sim->kernel_timing == 0 && max_run >= sim->cfg.graph_steps)
+      (!form.network && sim->cfg.graph_steps && ev_pos.empty() && sim->kernel_timing == 0 && max_run >= sim->cfg.graph_steps)
           ? sim->cfg.graph_steps
           : 0u;
   if (G) {
@@ -1377,6 +1480,17 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       hipLaunchKernelGGL(k_groups, dim3((a.gwords * 32 + 255) / 256, len), dim3(256), 0, st, a, c0);
       NC_HIP(hipGetLastError());
     }
+    if (form.network) {
+      if (c0 + len == max_run) a.call_tag = call_tag;
+      a.n_ev = (uint32_t)ev_pos.size();
+      a.ev_pos = sim->d_ev_pos.p;
+      a.ev_kind = sim->d_ev_kind.p;
+      const nc_status s1 = sim->live_nq <= 4   ? launch_networks<4, 8>(sim, a, c0, len)
+                           : sim->live_nq <= 8 ? launch_networks<8, 16>(sim, a, c0, len)
+                                               : launch_networks<16, 16>(sim, a, c0, len);
+      if (s1 != NC_OK) return s1;
+      continue;
+    }
     uint32_t j = 0;
     if (G)
       for (; len - j >= G; j += G) NC_HIP(hipGraphLaunch(sim->graph, st));
@@ -1395,7 +1509,8 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       if (fn_step) {
         if (s1 == NC_OK) s1 = launch(1, fn_step, pgrid, 64 * wpb, lds);
       } else {
-        if (s1 == NC_OK) s1 = launch(1, fn_neuron, grid, 64 * wpb, lds);
+        if (s1 == NC_OK) s1 = launch(1, fn_neuron, n_grid, n_block, lds);
+        if (i + 1 == max_run) a.call_tag = call_tag;
         if (s1 == NC_OK) s1 = launch(3, fn_fanout, fan_grid, 64 * wpb, 0);
       }
       if (s1 != NC_OK) return s1;
@@ -1491,9 +1606,10 @@ namespace {
 // After a synchronisation: did a grid barrier of the persistent form time out
 // (a grid whose workgroups were not all resident) since the last check?
 nc_status check_barrier(nc_sim* sim) {
-  uint32_t flag = 0;
-  NC_HIP(hipMemcpy(&flag, sim->d_chunk_off + 64, 4, hipMemcpyDeviceToHost));
-  if (!flag) return NC_OK;
+  uint32_t words[97];  // word 64 and the activity report
+  NC_HIP(hipMemcpy(words, sim->d_chunk_off + 64, sizeof words, hipMemcpyDeviceToHost));
+  sim->busy = (words[96] & 1u) != 0;
+  if (!words[0]) return NC_OK;
   NC_HIP(hipMemset(sim->d_chunk_off + 64, 0, 4));
   return fail(NC_ERR_STATE, "a grid barrier of the persistent launch timed out: the steps since the last check "
                             "are invalid");

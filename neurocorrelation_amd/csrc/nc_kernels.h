@@ -42,6 +42,8 @@
 #define NC_PEND_LOG_W 4
 // Spikes with delays up to NC_NB steps go to an arrival bucket instead: per
 // slice, one bucket per arrival step modulo NC_NB, of up to NC_BCAP entries
+// (two per neuron: at 50 synapses per neuron and a quarter of the neurons
+// firing, a slice has 107 arrivals in a step)
 // (slot - first slot of the slice | (delay - 1) << 24 | sign class << 31,
 // weight at the fire, whose product with 10.4 is the latched
 // depolarisation).  Fan-out takes
@@ -50,7 +52,7 @@
 // contribute -- and empties it.  A spike that finds its bucket full, or
 // whose delay exceeds NC_NB, goes to the pending list of its window.
 #define NC_NB 64u
-#define NC_BCAP 64u
+#define NC_BCAP 128u
 // Slices with fired lanes go to one of NC_FLISTS lists (by wave index), so
 // that the appends of a step spread over that many counters.
 #define NC_FLISTS 64
@@ -187,7 +189,16 @@ struct nc_step_args {
   const uint32_t* ev_pos;  // host events of this step
   const uint8_t* ev_kind;
   uint32_t n_ev;
+  uint32_t* activity;  // what nc_report leaves
+  uint32_t call_tag;   // call number << 1 on the launch that reports, else 0
 };
+
+// How busy the networks are, for the host's choice of the next call's form:
+// the newest call's word wins, and in it "busy" over "quiet".
+__device__ __forceinline__ void nc_report(const nc_step_args& a, bool busy) {
+  if (a.call_tag) atomicMax(a.activity, a.call_tag | (busy ? 1u : 0u));
+}
+#define NC_BUSY_LANES 6u  // fired lanes per slice and step from which a network is busy
 
 __device__ __forceinline__ float nc_lookup(const float* t, int32_t len, int32_t d) {
   return (d >= 0 && d < len) ? t[d] : 0.0f;
@@ -724,6 +735,15 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
   // the target lane give each lane the set of entries that are its own.
   const float tr_t = (!fire && tr_in) ? tr_tab : 0.0f;
   uint32_t arrw = 0;  // which of mask words 0-3 took arrivals
+  // A bucket's entries past the lanes' first 64 go through the pending list
+  // (its slots have room for every spike in flight to them).
+  if (b_take > 64u) {
+    if (64u + lane < b_take)
+      pl[pend_n + lane] = (a.bent[bi * NC_BCAP + 64u + lane].x << 8) | ((uint32_t)s & 255u);
+    pend_n += b_take - 64u;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  }
   // batch 0: the bucket's entries; batch b > 0: pending entries 64 (b - 1) ..
   const uint32_t n_batches = 1u + (pend_n + 63u) / 64u;
   uint32_t kept = 0;  // pending entries kept (compacted in place: write index <= read index)
@@ -874,7 +894,7 @@ __device__ __forceinline__ const float* nc_trace_tables(const nc_step_args& a) {
 // The neuron phase of one step for every active slice, one wave per slice,
 // WPB waves per workgroup.
 template <int WPB>
-__global__ __launch_bounds__(64 * WPB) void k_neuron(nc_step_args a) {
+__global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) void k_neuron(nc_step_args a) {
   const uint32_t blk = nc_block_id(a.xcd_swizzle);
   const uint32_t wave = __builtin_amdgcn_readfirstlane(blk * WPB + (threadIdx.x >> 6));
   const float* tpre = nc_trace_tables<WPB>(a);
@@ -937,6 +957,9 @@ __device__ __forceinline__ void nc_fanout_wave(const nc_step_args& a, uint32_t b
                                         a.fired_cnt[((((uint32_t)ci & 1u) * NC_FLISTS) + lst) * NC_FCNT_STRIDE])
                                   : 0u;
   const uint4* const flist = a.fired + lst * a.fcap;
+  // busy: two records per slice, or (unsplit: one per slice) most slices fired
+  if (a.call_tag && first == 0u && lane == 0)
+    nc_report(a, nf * (NC_FLISTS / 2u) >= a.n_active_slices * (a.fsplit_od ? 1.0f : 0.375f));
   for (uint32_t fb = first; fb < nf; fb += 64 * per) {
     const uint32_t fi = fb + lane * per;
     const uint4 fl = fi < nf ? flist[fi] : make_uint4(0u, 0u, 0u, 0u);
