@@ -243,7 +243,8 @@ nc_status nc_write_weights(nc_sim* sim, int32_t net_id, const float* w, uint64_t
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * weights are gathered in export order into a static per-GPU scratch array
  * of 16,777,216 floats (64 MiB, held by every GPU the library runs on until
- * the process ends) and copied into out.  A network with more synapses than
+ * the process ends; reads of up to 1 MiB into the simulation's pinned host
+ * buffer instead) and copied into out.  A network with more synapses than
  * that fails with NC_ERR_RANGE (nc_read_weights has no such limit).  Calls
  * that overlap on one GPU (from different threads) share the scratch and
  * race; calls on one nc_sim are serialised by its threading rule. */

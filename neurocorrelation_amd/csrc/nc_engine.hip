@@ -34,6 +34,7 @@
 #include "nc_internal.h"
 #include "nc_group.h"
 #include "nc_kernels.h"
+#include "nc_state.h"
 
 using nc::fail;
 
@@ -75,6 +76,10 @@ namespace {
   } while (0)
 
 constexpr uint32_t kSigma = 1024;
+
+// Results up to this size are written by the kernels into pinned host memory
+// (one launch and one wait); larger ones are staged on the device and copied.
+constexpr size_t kPinBytes = 1u << 20;
 
 // First-fit allocator over [0, cap) in units.
 struct RangeAlloc {
@@ -181,8 +186,7 @@ namespace nc {
 struct NetMaps {
   std::vector<uint32_t> pos_of_id;    // local position per neuron id
   std::vector<uint32_t> id_of_pos;    // neuron id per local position (nq*64, ~0u: padding)
-  std::vector<uint32_t> slot_of_syn;  // local slot per synapse, export order
-  std::vector<uint32_t> edge_of_syn;  // local out-edge per synapse, export order
+  std::vector<uint32_t> slice_off;    // first slot per slice
   std::vector<int64_t> in_ptr;        // incoming rows (export order)
   uint64_t digest = 0;                // identity of the wiring (checkpoints are checked against it)
 };
@@ -259,15 +263,15 @@ std::shared_ptr<const NetImage> build_image(const nc_net& net) {
   // Slot records, in layout order.
   I.slot_w.assign(L.nslots, 0.0f);
   I.slot_inh.assign((L.nslots + 31) / 32, 0u);
-  M.slot_of_syn.resize(S);
-  M.edge_of_syn.assign(S, 0u);
+  M.slice_off = I.slice_off;
+  std::vector<uint32_t> slot_of_syn(S);
   for (uint32_t id = 0; id < net.n; ++id) {
     const uint32_t pl = L.pos_of_id[id];
     const uint32_t q = pl / 64, l = pl % 64;
     const int64_t b = net.in_ptr[id], e = net.in_ptr[id + 1];
     for (int64_t k = 0; k < e - b; ++k) {
       const uint32_t j = nc_slot_of(I.slice_off[q], l, (uint32_t)k);
-      M.slot_of_syn[b + k] = j;
+      slot_of_syn[b + k] = j;
       I.slot_w[j] = net.w[b + k];
       if (net.inh[b + k]) I.slot_inh[j >> 5] |= 1u << (j & 31);
     }
@@ -289,8 +293,7 @@ std::shared_ptr<const NetImage> build_image(const nc_net& net) {
       const uint32_t tq = L.pos_of_id[tg] / 64;
       for (int64_t k = net.in_ptr[tg]; k < net.in_ptr[tg + 1]; ++k) {
         const uint32_t e = fillp[L.pos_of_id[net.in_src[k]]]++;
-        I.edge_jq[e] = make_uint2(M.slot_of_syn[k], (tq << 8) | net.delay[k]);
-        M.edge_of_syn[k] = e;
+        I.edge_jq[e] = make_uint2(slot_of_syn[k], (tq << 8) | net.delay[k]);
       }
     }
   }
@@ -461,8 +464,11 @@ struct nc_sim {
   bool busy = false;    // the last report read back (step_form)
   DevBuf<nc_group> d_groups;
   DevBuf<uint32_t> d_gfire;
-  DevBuf<float> d_wbuf;       // packed weights of one network, for host reads
-  DevBuf<uint32_t> d_stage;   // a network's compact upload, expanded in place by the placing kernels
+  // A network's compact upload, expanded in place by the placing kernels;
+  // later what crosses to or from the host, in the caller's order.  Grown by
+  // nc_sim_add alone, to hold either for the largest network added.
+  DevBuf<uint32_t> d_stage;
+  unsigned char* h_pin = nullptr;  // pinned host buffer of kPinBytes for what is small
   DevBuf<uint32_t> d_thr;
   DevBuf<uint32_t> d_ev_pos;
   DevBuf<uint8_t> d_ev_kind;
@@ -669,16 +675,43 @@ nc_status reserve_events(nc_sim* sim) {
 
 nc_status check_barrier(nc_sim* sim);
 
-// A network's weights in export order into dev (at least S floats), then the
-// first n of them to the caller's out.
-nc_status export_weights(nc_sim* sim, NetRec& r, float* dev, float* out, uint64_t n) {
-  const uint32_t pos0 = r.q0 * 64;
-  hipLaunchKernelGGL(k_export_w, dim3((r.n + 255) / 256), dim3(256), 0, sim->stream, sim->slots, sim->slice_off,
-                     sim->ndw, sim->id_pos, sim->id_row, pos0, r.q0, r.n, dev);
+nc_place place_of(const nc_sim* sim, const NetRec& r) {
+  return nc_place{sim->slots, sim->slice_off, sim->ndw, sim->id_pos, sim->id_row, r.q0 * 64u, r.q0, r.n};
+}
+
+dim3 row_blocks(const NetRec& r) { return dim3((uint32_t)(((uint64_t)r.n * NC_ROW_LANES + 255) / 256)); }
+
+// `bytes` of results for the caller: `fill` enqueues the kernel that writes
+// them to the address that it is given.  dev: device staging of that size.
+template <class F>
+nc_status deliver(nc_sim* sim, void* out, size_t bytes, void* dev, F fill) {
+  const bool pinned = bytes <= kPinBytes;
+  fill(pinned ? (void*)sim->h_pin : dev);
   NC_HIP(hipGetLastError());
-  NC_HIP(hipMemcpyAsync(out, dev, n * 4, hipMemcpyDeviceToHost, sim->stream));
+  if (!pinned) NC_HIP(hipMemcpyAsync(out, dev, bytes, hipMemcpyDeviceToHost, sim->stream));
   NC_HIP(hipStreamSynchronize(sim->stream));
+  if (pinned) memcpy(out, sim->h_pin, bytes);
   return check_barrier(sim);
+}
+
+// The caller's `bytes` at an address that kernels can read.
+nc_status fetch(nc_sim* sim, const void* in, size_t bytes, const void** at) {
+  if (bytes <= kPinBytes) {
+    memcpy(sim->h_pin, in, bytes);
+    *at = sim->h_pin;
+    return NC_OK;
+  }
+  NC_HIP(hipMemcpyAsync(sim->d_stage.p, in, bytes, hipMemcpyHostToDevice, sim->stream));
+  *at = sim->d_stage.p;
+  return NC_OK;
+}
+
+// A network's first n weights in export order; dev: device staging of n floats.
+nc_status export_weights(nc_sim* sim, NetRec& r, float* dev, float* out, uint64_t n) {
+  const nc_place N = place_of(sim, r);
+  return deliver(sim, out, 4 * n, dev, [&](void* to) {
+    hipLaunchKernelGGL(k_read_weights, row_blocks(r), dim3(256), 0, sim->stream, N, (float*)to, (uint32_t)n);
+  });
 }
 
 hipEvent_t get_event(nc_sim* sim, size_t i) {
@@ -803,6 +836,7 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
     H(hipMalloc(&sim->fired, (Q + NC_FLISTS * 8ull) * NC_FSPLIT * sizeof(uint4)), "hipMalloc fired");
     H(hipMalloc(&sim->fired_cnt, 2ull * NC_FLISTS * NC_FCNT_STRIDE * 4), "hipMalloc fired_cnt");
 
+    H(hipHostMalloc((void**)&sim->h_pin, kPinBytes, hipHostMallocDefault), "hipHostMalloc");
     H(hipMalloc(&sim->raster_cnt, 64), "hipMalloc raster_cnt");
     if (sim->raster_cap) H(hipMalloc(&sim->raster, 8ull * sim->raster_cap), "hipMalloc raster");
     sim->ctr_rows = Q + 2;
@@ -857,9 +891,10 @@ extern "C" void nc_sim_destroy(nc_sim* sim) {
                   sim->nid, sim->out_row, sim->edges, sim->pend0, sim->pend1, sim->pend_cnt, sim->bcnt, sim->bent, sim->acache, sim->slice_moff, sim->id_pos, sim->id_row, sim->slice_off, sim->slice_net, sim->active, sim->net_recs, sim->forced_in,
                   sim->forced_bg, sim->fired, sim->fired_cnt, sim->raster, sim->raster_cnt,
                   sim->ctr, sim->d_nets, sim->t_pre, sim->t_post, sim->w_ap, sim->d_groups.p,
-                  sim->d_thr.p, sim->d_ev_pos.p, sim->d_ev_kind.p, sim->d_ev_step.p, sim->d_gfire.p, sim->d_wbuf.p, sim->d_stage.p};
+                  sim->d_thr.p, sim->d_ev_pos.p, sim->d_ev_kind.p, sim->d_ev_step.p, sim->d_gfire.p, sim->d_stage.p};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
+  if (sim->h_pin) (void)hipHostFree(sim->h_pin);
   for (hipEvent_t e : sim->ev_pool) (void)hipEventDestroy(e);
   if (sim->upload_done) (void)hipEventDestroy(sim->upload_done);
   if (sim->stream) (void)hipStreamDestroy(sim->stream);
@@ -1077,7 +1112,7 @@ extern "C" nc_status nc_sim_add(nc_sim* sim, const nc_net* net, const nc_params*
   // to a staging buffer; the placing kernels expand it into the records.
   const uint64_t n_inh = I.slot_inh.size(), o_jq = (I.nslots + n_inh + 1) & ~1ull;
   {
-    nc_status sg = grow(&sim->d_stage, o_jq + 2 * S + 2, st);
+    nc_status sg = grow(&sim->d_stage, std::max<uint64_t>(o_jq + 2 * S + 2, 3ull * net->n + 4 * S + 4), st);
     if (sg != NC_OK) {
       if (r.has_drive) {
         const nc_group dead{0u, 1u, 0u, sim->max_nets};
@@ -1617,27 +1652,14 @@ nc_status check_barrier(nc_sim* sim) {
 
 template <class T>
 nc_status read_pos_array(nc_sim* sim, NetRec& r, const T* dev, T* out, uint32_t n) {
+  static_assert(sizeof(T) == 4, "4-byte values");
   if (!out) return fail(NC_ERR_ARG, "null argument");
   if (n > r.n) return fail(NC_ERR_RANGE, "more neurons requested than the network has");
-  std::vector<T> tmp((size_t)r.nq * 64);
-  NC_HIP(hipMemcpyAsync(tmp.data(), dev + (size_t)r.q0 * 64, tmp.size() * sizeof(T), hipMemcpyDeviceToHost,
-                        sim->stream));
-  NC_HIP(hipStreamSynchronize(sim->stream));
-  {
-    nc_status cb = check_barrier(sim);
-    if (cb != NC_OK) return cb;
-  }
-  for (uint32_t i = 0; i < n; ++i) out[i] = tmp[r.maps->pos_of_id[i]];
-  return NC_OK;
-}
-
-nc_status read_slots(nc_sim* sim, NetRec& r, std::vector<nc_slot>* hs) {
-  NC_HIP(hipSetDevice(sim->device));
-  hs->resize(r.nslots);
-  NC_HIP(hipMemcpyAsync(hs->data(), sim->slots + r.slot0, r.nslots * sizeof(nc_slot), hipMemcpyDeviceToHost,
-                        sim->stream));
-  NC_HIP(hipStreamSynchronize(sim->stream));
-  return check_barrier(sim);
+  const nc_place N = place_of(sim, r);
+  return deliver(sim, out, 4ull * n, sim->d_stage.p, [&](void* to) {
+    if (n) hipLaunchKernelGGL(k_read_neurons, dim3((n + 255) / 256), dim3(256), 0, sim->stream, N, (const uint32_t*)dev, n,
+                       (uint32_t*)to);
+  });
 }
 }  // namespace
 
@@ -1676,9 +1698,7 @@ extern "C" nc_status nc_read_weights(nc_sim* sim, int32_t net_id, float* out, ui
   if (n > r->S) return fail(NC_ERR_RANGE, "more synapses requested than the network has");
   NC_HIP(hipSetDevice(sim->device));
   if (r->S == 0 || n == 0) return NC_OK;
-  st = grow(&sim->d_wbuf, r->S, sim->stream);
-  if (st != NC_OK) return st;
-  return export_weights(sim, *r, sim->d_wbuf.p, out, n);
+  return export_weights(sim, *r, (float*)sim->d_stage.p, out, n);
 }
 NC_ABI_CATCH
 
@@ -1695,8 +1715,8 @@ extern "C" nc_status nc_read_weights_noalloc(nc_sim* sim, int32_t net_id, float*
   if (!scr) return fail(NC_ERR_STATE, "the static scratch of this device is not set up");
   NC_HIP(hipSetDevice(sim->device));
   if (r->S == 0 || n == 0) return NC_OK;
-  // the export kernel writes every one of the network's S entries before
-  // the copy reads them: nothing needs clearing first
+  // the export kernel writes every entry that the copy reads: nothing needs
+  // clearing first
   return export_weights(sim, *r, scr, out, n);
 }
 NC_ABI_CATCH
@@ -1707,18 +1727,18 @@ extern "C" nc_status nc_write_weights(nc_sim* sim, int32_t net_id, const float* 
   if (st != NC_OK) return st;
   if (!w) return fail(NC_ERR_ARG, "null argument");
   if (n > r->S) return fail(NC_ERR_RANGE, "more synapses given than the network has");
-  std::vector<nc_slot> hs;
-  st = read_slots(sim, *r, &hs);
+  NC_HIP(hipSetDevice(sim->device));
+  NC_HIP(hipStreamSynchronize(sim->stream));
+  st = check_barrier(sim);
   if (st != NC_OK) return st;
-  // Synapse::setWeight also re-derives the sign class (src/NeuCor.cpp:576-579).
-  for (uint64_t k = 0; k < n; ++k) {
-    nc_slot& x = hs[r->maps->slot_of_syn[k]];
-    x.w = w[k];
-    x.arr_inh = (x.arr_inh & ~1) | ((w[k] < 0.0f) ? 1 : 0);
-  }
   r->whost = r->steps_done + 1;
-  NC_HIP(hipMemcpyAsync(sim->slots + r->slot0, hs.data(), r->nslots * sizeof(nc_slot), hipMemcpyHostToDevice,
-                        sim->stream));
+  if (n == 0) return NC_OK;
+  const void* at = nullptr;
+  st = fetch(sim, w, 4 * n, &at);
+  if (st != NC_OK) return st;
+  hipLaunchKernelGGL(k_write_weights, row_blocks(*r), dim3(256), 0, sim->stream, place_of(sim, *r), (const float*)at,
+                     (uint32_t)n);
+  NC_HIP(hipGetLastError());
   NC_HIP(hipStreamSynchronize(sim->stream));
   return NC_OK;
 }
@@ -1731,17 +1751,37 @@ extern "C" nc_status nc_set_weights(nc_sim* sim, int32_t net_id, uint64_t n, con
   if (n && (!syn || !w)) return fail(NC_ERR_ARG, "null argument");
   for (uint64_t i = 0; i < n; ++i)
     if (syn[i] >= r->S) return fail(NC_ERR_RANGE, "synapse index out of range");
-  std::vector<nc_slot> hs;
-  st = read_slots(sim, *r, &hs);
-  if (st != NC_OK) return st;
+  // Of a synapse listed more than once the last weight holds: the entries in
+  // order of their synapse, then of the list, and of each the last.
+  std::vector<uint64_t> order(n);
+  std::iota(order.begin(), order.end(), 0ull);
+  std::stable_sort(order.begin(), order.end(), [&](uint64_t a, uint64_t b) { return syn[a] < syn[b]; });
+  std::vector<uint2> sw;
+  sw.reserve(n);
+  const nc::NetMaps& M = *r->maps;
+  uint32_t t = 0;  // target whose row holds the synapse
   for (uint64_t i = 0; i < n; ++i) {
-    nc_slot& x = hs[r->maps->slot_of_syn[syn[i]]];
-    x.w = w[i];
-    x.arr_inh = (x.arr_inh & ~1) | ((w[i] < 0.0f) ? 1 : 0);
+    const uint64_t k = syn[order[i]];
+    if (i + 1 < n && syn[order[i + 1]] == k) continue;
+    if ((uint64_t)M.in_ptr[t + 1] <= k)
+      t = (uint32_t)(std::upper_bound(M.in_ptr.begin() + t, M.in_ptr.end(), (int64_t)k) - M.in_ptr.begin() - 1);
+    const uint32_t p = M.pos_of_id[t];
+    uint32_t bits;
+    memcpy(&bits, &w[order[i]], 4);
+    sw.push_back(make_uint2((uint32_t)r->slot0 + nc_slot_of(M.slice_off[p / 64], p % 64, (uint32_t)(k - M.in_ptr[t])), bits));
   }
+  NC_HIP(hipSetDevice(sim->device));
+  NC_HIP(hipStreamSynchronize(sim->stream));
+  st = check_barrier(sim);
+  if (st != NC_OK) return st;
   r->whost = r->steps_done + 1;
-  NC_HIP(hipMemcpyAsync(sim->slots + r->slot0, hs.data(), r->nslots * sizeof(nc_slot), hipMemcpyHostToDevice,
-                        sim->stream));
+  if (sw.empty()) return NC_OK;
+  const void* at = nullptr;
+  st = fetch(sim, sw.data(), sw.size() * sizeof(uint2), &at);
+  if (st != NC_OK) return st;
+  hipLaunchKernelGGL(k_set_weights, dim3((uint32_t)((sw.size() + 255) / 256)), dim3(256), 0, sim->stream, sim->slots,
+                     (const uint2*)at, (uint32_t)sw.size());
+  NC_HIP(hipGetLastError());
   NC_HIP(hipStreamSynchronize(sim->stream));
   return NC_OK;
 }
@@ -1753,23 +1793,28 @@ extern "C" nc_status nc_read_synapse_state(nc_sim* sim, int32_t net_id, int32_t*
   nc_status st = check_net(sim, net_id, &r);
   if (st != NC_OK) return st;
   if (n > r->S) return fail(NC_ERR_RANGE, "more synapses requested than the network has");
-  std::vector<nc_slot> hs;
-  st = read_slots(sim, *r, &hs);
-  if (st != NC_OK) return st;
-  // Synapse::AP_fireTime: the latched spike's arrival until its latch
-  // releases (R steps after arrival), then 0.
-  const int32_t s = (int32_t)r->steps_done;
-  for (uint64_t k = 0; k < n; ++k) {
-    const uint64_t j = r->maps->slot_of_syn[k];
-    const int32_t a = hs[j].arr_inh >> 1;
-    if (arrival) arrival[k] = (a != NC_NEVER && s < a + sim->T.r_rel) ? a : 0;
-    // lastSpikeArrival: the latched spike's arrival once it has arrived, else
-    // last_arr (the one before it, which fan-out moved there, or a last
-    // arrival restored without a latched spike)
-    if (last_arrival) last_arrival[k] = (a != NC_NEVER && a <= s) ? a : hs[j].last_arr;
-    if (depol) depol[k] = hs[j].depol;
+  NC_HIP(hipSetDevice(sim->device));
+  void* const want[3] = {arrival, last_arrival, depol};
+  uint32_t m = 0, of[3] = {0, 0, 0};  // arrays wanted; the place of each
+  for (int i = 0; i < 3; ++i)
+    if (want[i]) of[i] = m++;
+  const bool pinned = 4 * n * m <= kPinBytes;
+  uint32_t* const to = pinned ? (uint32_t*)sim->h_pin : sim->d_stage.p;
+  auto at = [&](int i) { return want[i] ? to + of[i] * n : nullptr; };
+  if (n && m) {
+    hipLaunchKernelGGL(k_read_spikes, row_blocks(*r), dim3(256), 0, sim->stream, place_of(sim, *r),
+                       (int32_t)r->steps_done, sim->T.r_rel, (int32_t*)at(0), (int32_t*)at(1), (float*)at(2),
+                       (uint32_t)n);
+    NC_HIP(hipGetLastError());
+    if (!pinned)
+      for (int i = 0; i < 3; ++i)
+        if (want[i]) NC_HIP(hipMemcpyAsync(want[i], at(i), 4 * n, hipMemcpyDeviceToHost, sim->stream));
   }
-  return NC_OK;
+  NC_HIP(hipStreamSynchronize(sim->stream));
+  if (pinned && n)
+    for (int i = 0; i < 3; ++i)
+      if (want[i]) memcpy(want[i], at(i), 4 * n);
+  return check_barrier(sim);
 }
 NC_ABI_CATCH
 
@@ -1822,7 +1867,8 @@ NC_ABI_CATCH
 //   synapses: w f32, depol f32, lastArrival i32, arrival i32   (export order)
 //   events  : step offset u32, id u32, kind u32                (queued forced fires)
 // Active masks, their summaries, the pending lists and the fan-out latches
-// are functions of (arrival, steps_done) and are rebuilt on restore.
+// are functions of (arrival, steps_done) and are rebuilt on restore, on the
+// device (nc_state.h).
 namespace {
 struct nc_ckpt_header {
   uint32_t magic, version, n, pad0;
@@ -1845,9 +1891,6 @@ extern "C" nc_status nc_sim_save(nc_sim* sim, int32_t net_id, void* buf, uint64_
   *size = need;
   if (!buf) return NC_OK;
   if (cap < need) return fail(NC_ERR_RANGE, "checkpoint buffer too small");
-  std::vector<nc_slot> hs;
-  st = read_slots(sim, *r, &hs);
-  if (st != NC_OK) return st;
   unsigned char* p = (unsigned char*)buf;
   nc_ckpt_header h{};
   h.magic = 0x314b434eu;  // "NCK1"
@@ -1858,26 +1901,16 @@ extern "C" nc_status nc_sim_save(nc_sim* sim, int32_t net_id, void* buf, uint64_
   h.lr = r->lr, h.pre_f = r->pre_f, h.post_f = r->post_f, h.dt = sim->T.dt;
   h.n_events = (uint32_t)r->events.size();
   h.digest = r->maps->digest;
-  memcpy(p, &h, sizeof h);
-  p += sizeof h;
-  std::vector<float> V(r->n);
-  std::vector<int32_t> lf(r->n);
-  std::vector<uint32_t> fi(r->n);
-  st = read_pos_array(sim, *r, sim->V, V.data(), r->n);
-  if (st == NC_OK) st = read_pos_array(sim, *r, sim->last_fire, lf.data(), r->n);
-  if (st == NC_OK) st = read_pos_array(sim, *r, sim->firings, fi.data(), r->n);
+  NC_HIP(hipSetDevice(sim->device));
+  const uint64_t state = 12ull * r->n + 16ull * r->S;
+  st = deliver(sim, p + sizeof h, state, sim->d_stage.p, [&](void* to) {
+    if (r->n)
+      hipLaunchKernelGGL(k_pack, row_blocks(*r), dim3(256), 0, sim->stream, place_of(sim, *r), sim->V, sim->last_fire,
+                         sim->firings, (int32_t)r->steps_done, (uint32_t*)to);
+  });
   if (st != NC_OK) return st;
-  for (uint32_t i = 0; i < r->n; ++i) {
-    memcpy(p, &V[i], 4), memcpy(p + 4, &lf[i], 4), memcpy(p + 8, &fi[i], 4);
-    p += 12;
-  }
-  for (uint64_t k = 0; k < r->S; ++k) {
-    const nc_slot& x = hs[r->maps->slot_of_syn[k]];
-    const int32_t arr = x.arr_inh >> 1;
-    const int32_t last = (arr != NC_NEVER && arr <= (int32_t)r->steps_done) ? arr : x.last_arr;  // lastSpikeArrival
-    memcpy(p, &x.w, 4), memcpy(p + 4, &x.depol, 4), memcpy(p + 8, &last, 4), memcpy(p + 12, &arr, 4);
-    p += 16;
-  }
+  memcpy(p, &h, sizeof h);
+  p += sizeof h + state;
   for (auto& ev : r->events) {
     const uint32_t off = ev.first - r->steps_done, pos = ev.second.first - r->q0 * 64;
     const uint32_t id = r->maps->id_of_pos[pos], kind = ev.second.second;
@@ -1905,70 +1938,28 @@ extern "C" nc_status nc_sim_restore(nc_sim* sim, int32_t net_id, const void* buf
   if (h.steps_done >= (uint32_t)NC_MAX_STEPS) return fail(NC_ERR_RANGE, "checkpoint step count out of range");
   const unsigned char* p = (const unsigned char*)buf + sizeof h;
   NC_HIP(hipSetDevice(sim->device));
-  NC_HIP(hipStreamSynchronize(sim->stream));
+  hipStream_t sq = sim->stream;
+  NC_HIP(hipStreamSynchronize(sq));
   const int32_t s = (int32_t)h.steps_done;
-  const int32_t R = sim->T.r_rel;
-  const uint32_t npos = r->nq * 64, pos0 = r->q0 * 64;
-  // neurons
-  std::vector<float> V((size_t)npos, NC_BASELEVEL);
-  std::vector<int32_t> lf((size_t)npos, NC_NEVER);
-  std::vector<uint32_t> fi((size_t)npos, 0u), asum((size_t)npos, 0u);
-  NC_HIP(hipMemcpy(V.data(), sim->V + pos0, npos * 4, hipMemcpyDeviceToHost));
-  // Step values a checkpoint may hold: NC_NEVER, or a step of the run so far
-  // (arrivals: up to the longest delay ahead); anything else would index the
-  // step tables out of range.
-  auto past = [s](int32_t v) { return v == NC_NEVER || (v >= 1 && v <= s); };
-  for (uint32_t i = 0; i < h.n; ++i) {
-    const uint32_t pl = r->maps->pos_of_id[i];
-    memcpy(&V[pl], p, 4), memcpy(&lf[pl], p + 4, 4), memcpy(&fi[pl], p + 8, 4);
-    if (!past(lf[pl])) return fail(NC_ERR_ARG, "checkpoint last fire out of range");
-    p += 12;
+  const uint64_t state = 12ull * h.n + 16ull * h.n_syn;
+  // The neurons and synapses go to the staging buffer and are checked there
+  // before anything of the network is written.
+  uint32_t bad = 0;
+  if (h.n) {
+    uint32_t* const flag = sim->d_chunk_off + 192;
+    NC_HIP(hipMemcpyAsync(sim->d_stage.p, p, state, hipMemcpyHostToDevice, sq));
+    hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, sq, flag, 1u, 0u);
+    NC_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_check_checkpoint, dim3((uint32_t)std::min<uint64_t>((h.n + h.n_syn + 255) / 256, 2048)),
+                       dim3(256), 0, sq, sim->d_stage.p, h.n, h.n_syn, s, flag);
+    NC_HIP(hipGetLastError());
+    NC_HIP(hipMemcpyAsync(&bad, flag, 4, hipMemcpyDeviceToHost, sq));
+    NC_HIP(hipStreamSynchronize(sq));
   }
-  // synapses, and from their arrivals the active masks, summaries, pending
-  // lists and fan-out latches
-  std::vector<nc_slot> hs(r->nslots);
-  NC_HIP(hipMemcpy(hs.data(), sim->slots + r->slot0, r->nslots * sizeof(nc_slot), hipMemcpyDeviceToHost));
-  std::vector<uint32_t> masks(r->nmwords, 0u);
-  // the active-slot cache: each position's first NC_ACACHE active slots,
-  // {depol 0, depol 1, depol 2, low bytes of their arrivals}
-  static_assert(NC_ACACHE == 3, "three depolarisations and their arrivals' low bytes per 16-byte record");
-  std::vector<uint4> cache((size_t)npos, make_uint4(0u, 0u, 0u, 0u));
-  std::vector<uint8_t> ncache((size_t)npos, 0u);
-  std::vector<std::vector<uint2>> pend(r->nq);
-  std::vector<int32_t> edge_arr(r->S);
-  for (uint32_t t = 0; t < h.n; ++t) {
-    const uint32_t pl = r->maps->pos_of_id[t], q = pl / 64, lane = pl % 64;
-    const uint32_t deg = (uint32_t)(r->maps->in_ptr[t + 1] - r->maps->in_ptr[t]);
-    const uint32_t nmw = (deg + 31) / 32, G = nmw <= 32 ? 1u : (nmw + 31) / 32;
-    for (uint32_t k = 0; k < deg; ++k) {
-      const uint64_t syn = (uint64_t)r->maps->in_ptr[t] + k;
-      const unsigned char* e = p + 16ull * syn;
-      nc_slot& x = hs[r->maps->slot_of_syn[syn]];
-      int32_t arr;
-      memcpy(&x.w, e, 4), memcpy(&x.depol, e + 4, 4), memcpy(&x.last_arr, e + 8, 4), memcpy(&arr, e + 12, 4);
-      if (!past(x.last_arr)) return fail(NC_ERR_ARG, "checkpoint last arrival out of range");
-      if (arr != NC_NEVER && (arr < 1 || arr > s + 255)) return fail(NC_ERR_ARG, "checkpoint arrival out of range");
-      x.arr_inh = arr * 2 + (x.arr_inh & 1);
-      edge_arr[syn] = arr;
-      if (arr == NC_NEVER) continue;
-      if (arr <= s && s < arr + R) {
-        const uint64_t word = sim->slice_moff_host[r->q0 + q] + (k >> 5) * 64 + lane - r->mask0;
-        masks[word] |= 1u << (k & 31);
-        asum[pl] |= 1u << ((k >> 5) / G);
-        uint32_t dbits;
-        memcpy(&dbits, &x.depol, 4);
-        if (ncache[pl] < NC_ACACHE) {
-          uint4& c = cache[pl];
-          const uint32_t e = ncache[pl]++;
-          (e == 0 ? c.x : e == 1 ? c.y : c.z) = dbits;
-          c.w |= ((uint32_t)arr & 255u) << (8 * e);
-        }
-      } else if (arr > s) {
-        pend[q].push_back(make_uint2((uint32_t)r->slot0 + r->maps->slot_of_syn[syn], (uint32_t)arr));
-      }
-    }
-  }
-  p += 16ull * h.n_syn;
+  if (bad & 1u) return fail(NC_ERR_ARG, "checkpoint last fire out of range");
+  if (bad & 2u) return fail(NC_ERR_ARG, "checkpoint last arrival out of range");
+  if (bad & 4u) return fail(NC_ERR_ARG, "checkpoint arrival out of range");
+  p += state;
   std::vector<std::pair<uint32_t, std::pair<uint32_t, uint8_t>>> events;
   for (uint32_t i = 0; i < h.n_events; ++i) {
     uint32_t off, id, kind;
@@ -1984,37 +1975,18 @@ extern "C" nc_status nc_sim_restore(nc_sim* sim, int32_t net_id, const void* buf
     r->events.clear();
     return st;
   }
-  // upload
-  hipStream_t sq = sim->stream;
-  NC_HIP(hipMemcpyAsync(sim->V + pos0, V.data(), npos * 4, hipMemcpyHostToDevice, sq));
-  NC_HIP(hipMemcpyAsync(sim->last_fire + pos0, lf.data(), npos * 4, hipMemcpyHostToDevice, sq));
-  NC_HIP(hipMemcpyAsync(sim->firings + pos0, fi.data(), npos * 4, hipMemcpyHostToDevice, sq));
-  NC_HIP(hipMemcpyAsync(sim->asum + pos0, asum.data(), npos * 4, hipMemcpyHostToDevice, sq));
-  NC_HIP(hipMemcpyAsync(sim->slots + r->slot0, hs.data(), r->nslots * sizeof(nc_slot), hipMemcpyHostToDevice, sq));
-  NC_HIP(hipMemcpyAsync(sim->amask + r->mask0, masks.data(), r->nmwords * 4, hipMemcpyHostToDevice, sq));
-  NC_HIP(hipMemcpyAsync(sim->acache + pos0, cache.data(), npos * sizeof(uint4), hipMemcpyHostToDevice, sq));
-  // each slice's spikes in flight into the pending list of their arrival
-  // window, entries relative to the slice's first slot
-  std::vector<uint2> cnt2(r->nq);
-  std::vector<std::vector<uint32_t>> lists(2 * (size_t)r->nq);
-  for (uint32_t q = 0; q < r->nq; ++q) {
-    const uint32_t first = sim->slice_off_host[r->q0 + q];
-    for (const uint2& e : pend[q])
-      lists[2 * q + ((e.y >> NC_PEND_LOG_W) & 1u)].push_back(((e.x - first) << 8) | (e.y & 255u));
-    cnt2[q] = make_uint2((uint32_t)lists[2 * q].size(), (uint32_t)lists[2 * q + 1].size());
-    for (uint32_t k = 0; k < 2; ++k) {
-      const std::vector<uint32_t>& l = lists[2 * q + k];
-      if (!l.empty())
-        NC_HIP(hipMemcpyAsync((k ? sim->pend1 : sim->pend0) + first, l.data(), l.size() * 4, hipMemcpyHostToDevice,
-                              sq));
+  if (h.n) {
+    hipLaunchKernelGGL(k_unpack, dim3(r->nq), dim3(64), 0, sq, place_of(sim, *r), sim->nid, sim->slice_moff,
+                       sim->d_stage.p, s, sim->T.r_rel, sim->V, sim->last_fire, sim->firings, sim->amask, sim->asum,
+                       sim->acache, sim->pend0, sim->pend1, sim->pend_cnt);
+    NC_HIP(hipGetLastError());
+    if (r->S) {
+      hipLaunchKernelGGL(k_restore_latches, dim3((uint32_t)std::min<uint64_t>((r->S + 255) / 256, 4096)), dim3(256), 0,
+                         sq, sim->edges + r->out0, sim->slots, r->S);
+      NC_HIP(hipGetLastError());
     }
+    NC_HIP(hipStreamSynchronize(sq));
   }
-  NC_HIP(hipMemcpyAsync(sim->pend_cnt + r->q0, cnt2.data(), r->nq * sizeof(uint2), hipMemcpyHostToDevice, sq));
-  std::vector<nc_edge> ed(r->S);
-  if (r->S) NC_HIP(hipMemcpy(ed.data(), sim->edges + r->out0, r->S * sizeof(nc_edge), hipMemcpyDeviceToHost));
-  for (uint64_t k = 0; k < r->S; ++k) ed[r->maps->edge_of_syn[k]].arr = edge_arr[k];
-  if (r->S) NC_HIP(hipMemcpyAsync(sim->edges + r->out0, ed.data(), r->S * sizeof(nc_edge), hipMemcpyHostToDevice, sq));
-  NC_HIP(hipStreamSynchronize(sq));
   r->steps_done = h.steps_done;
   r->lr = h.lr, r->pre_f = h.pre_f, r->post_f = h.post_f;
   return NC_OK;
