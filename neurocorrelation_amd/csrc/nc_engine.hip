@@ -80,6 +80,8 @@ constexpr uint32_t kSigma = 1024;
 // Results up to this size are written by the kernels into pinned host memory
 // (one launch and one wait); larger ones are staged on the device and copied.
 constexpr size_t kPinBytes = 1u << 20;
+// Host events a call passes through pinned memory (more: copied).
+constexpr size_t kPinEvents = 4096;
 
 // First-fit allocator over [0, cap) in units.
 struct RangeAlloc {
@@ -460,7 +462,7 @@ struct nc_sim {
   uint32_t graph_key[5] = {0, 0, 0, 0, 0};
   nc_netdesc* d_nets = nullptr;
   float *t_pre = nullptr, *t_post = nullptr, *w_ap = nullptr;
-  uint64_t calls = 0;   // nc_sim_step calls, numbering the activity reports
+  uint32_t calls = 0;   // nc_sim_step calls, numbering the activity reports (never 0 in a report)
   bool busy = false;    // the last report read back (step_form)
   DevBuf<nc_group> d_groups;
   DevBuf<uint32_t> d_gfire;
@@ -468,7 +470,13 @@ struct nc_sim {
   // later what crosses to or from the host, in the caller's order.  Grown by
   // nc_sim_add alone, to hold either for the largest network added.
   DevBuf<uint32_t> d_stage;
-  unsigned char* h_pin = nullptr;  // pinned host buffer of kPinBytes for what is small
+  // Pinned host memory: kPinBytes for small results and inputs; the network
+  // windows and host events of a call, reused only after upload_done; two
+  // words that kernels write (nc_step_args::host_words).
+  unsigned char* h_pin = nullptr;
+  nc_netdesc* h_nds = nullptr;
+  uint32_t* h_ev = nullptr;
+  uint32_t* h_words = nullptr;
   DevBuf<uint32_t> d_thr;
   DevBuf<uint32_t> d_ev_pos;
   DevBuf<uint8_t> d_ev_kind;
@@ -489,8 +497,7 @@ struct nc_sim {
   bool act_identity = false;  // active record i is slice act_q0 + i
   uint32_t act_q0 = 0;
   uint64_t host_neuron_steps = 0, host_synapse_steps = 0, host_mword_steps = 0;
-  // Host staging of the per-call uploads; reused only after upload_done.
-  std::vector<nc_netdesc> h_nds;
+  // Host staging of a call's events; reused only after upload_done.
   std::vector<uint32_t> h_ev_pos;
   std::vector<uint8_t> h_ev_kind;
   std::vector<uint32_t> h_ev_step;
@@ -575,6 +582,7 @@ nc_step_args base_args(nc_sim* sim) {
   a.acache = sim->acache;
   a.fired = sim->fired;
   a.fired_cnt = sim->fired_cnt;
+  a.host_words = sim->h_words;
   return a;
 }
 
@@ -668,7 +676,7 @@ nc_status reserve_events(nc_sim* sim) {
     sim->upload_pending = false;
   }
   nc_status st = grow(&sim->d_ev_pos, total, sim->stream);
-  if (st == NC_OK) st = grow(&sim->d_ev_kind, total, sim->stream);
+  if (st == NC_OK) st = grow(&sim->d_ev_kind, (total + 3) / 4 * 4, sim->stream);  // whole words
   if (st == NC_OK) st = grow(&sim->d_ev_step, total, sim->stream);
   return st;
 }
@@ -836,14 +844,20 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
     H(hipMalloc(&sim->fired, (Q + NC_FLISTS * 8ull) * NC_FSPLIT * sizeof(uint4)), "hipMalloc fired");
     H(hipMalloc(&sim->fired_cnt, 2ull * NC_FLISTS * NC_FCNT_STRIDE * 4), "hipMalloc fired_cnt");
 
-    H(hipHostMalloc((void**)&sim->h_pin, kPinBytes, hipHostMallocDefault), "hipHostMalloc");
+    H(hipHostMalloc((void**)&sim->h_pin, kPinBytes + 64 + sim->max_nets * sizeof(nc_netdesc) + kPinEvents * 12,
+                    hipHostMallocDefault), "hipHostMalloc");
+    if (sim->h_pin) {
+      sim->h_words = (uint32_t*)(sim->h_pin + kPinBytes);
+      sim->h_nds = (nc_netdesc*)(sim->h_pin + kPinBytes + 64);
+      sim->h_ev = (uint32_t*)(sim->h_nds + sim->max_nets);
+      sim->h_words[0] = sim->h_words[1] = 0u;
+    }
     H(hipMalloc(&sim->raster_cnt, 64), "hipMalloc raster_cnt");
     if (sim->raster_cap) H(hipMalloc(&sim->raster, 8ull * sim->raster_cap), "hipMalloc raster");
     sim->ctr_rows = Q + 2;
     // word 0: chunk offset; word 32: grid-barrier arrivals of the call;
-    // word 64: a grid barrier timed out (sticky until reported); word 128:
-    // zero, the group-spike-train word read when there are no groups; word
-    // 160: the activity report of the newest call
+    // word 128: zero, the group-spike-train word read when there are no
+    // groups; word 192: a checkpoint's faults (nc_sim_restore)
     H(hipMalloc(&sim->d_chunk_off, 1024), "hipMalloc chunk_off");
     H(hipMalloc(&sim->ctr, sim->ctr_rows * NC_NCTR * 8), "hipMalloc ctr");
     // one more, never written: the (never live) network of hole records
@@ -1272,8 +1286,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     NC_HIP(hipEventSynchronize(sim->upload_done));
     sim->upload_pending = false;
   }
-  std::vector<nc_netdesc>& nds = sim->h_nds;
-  nds.assign(sim->nets.size(), nc_netdesc{});
+  nc_netdesc* const nds = sim->h_nds;
   bool any_active = false;
   uint32_t max_run = 0;
   for (size_t i = 0; i < sim->nets.size(); ++i) {
@@ -1310,8 +1323,6 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     nc_status s0 = rebuild_active(sim);
     if (s0 != NC_OK) return s0;
   }
-  NC_HIP(hipMemcpyAsync(sim->d_nets, nds.data(), nds.size() * sizeof(nc_netdesc), hipMemcpyHostToDevice, st));
-
   const Form form = step_form(sim);
 
   // Host-scheduled events for steps [1, max_run] of this call, per step.
@@ -1323,7 +1334,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   ev_kind.clear();
   std::vector<uint32_t> ev_ptr(max_run + 1, 0);
   {
-    std::vector<std::vector<std::pair<uint32_t, uint8_t>>> per(max_run);
+    std::vector<std::pair<uint32_t, std::pair<uint32_t, uint8_t>>> due;  // by step of the call, in queue order
     for (size_t i = 0; i < sim->nets.size(); ++i) {
       NetRec& r = sim->nets[i];
       if (!r.live || r.events.empty()) continue;
@@ -1331,29 +1342,54 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       const uint32_t run = (uint32_t)nds[i].remaining;
       for (auto& ev : r.events) {
         uint32_t k = ev.first - r.steps_done;  // 1-based offset in this call
-        if (k >= 1 && k <= run) per[k - 1].push_back(ev.second);
+        if (k >= 1 && k <= run) due.push_back({k - 1, ev.second});
         else if (k > run) keep.push_back(ev);
       }
       r.events.swap(keep);
     }
-    for (uint32_t k = 0; k < max_run; ++k) {
-      ev_ptr[k + 1] = ev_ptr[k] + (uint32_t)per[k].size();
-      for (auto& e : per[k]) {
-        ev_pos.push_back(e.first);
-        ev_kind.push_back(e.second);
-        ev_step.push_back(k);
-      }
+    std::stable_sort(due.begin(), due.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
+    for (auto& e : due) {
+      ++ev_ptr[e.first + 1];
+      ev_pos.push_back(e.second.first);
+      ev_kind.push_back(e.second.second);
+      ev_step.push_back(e.first);
+    }
+    for (uint32_t k = 0; k < max_run; ++k) ev_ptr[k + 1] += ev_ptr[k];
+  }
+  nc_begin b;
+  memset(&b, 0, sizeof b);
+  b.chunk_off = sim->d_chunk_off;
+  b.bar = sim->d_chunk_off + 32;
+  b.fired_cnt = sim->fired_cnt;
+  auto part = [&](int p, void* dst, const void* src, uint64_t words) {
+    b.dst[p] = (uint32_t*)dst;
+    b.src[p] = (const uint32_t*)src;
+    b.n[p] = (uint32_t)words;
+  };
+  part(0, sim->d_nets, nds, sim->nets.size() * (sizeof(nc_netdesc) / 4));
+  const size_t n_ev = ev_pos.size();
+  if (n_ev) {
+    // nc_push_forced and nc_sim_restore reserve room for every queued event
+    if (sim->d_ev_pos.n < n_ev || sim->d_ev_kind.n < n_ev || sim->d_ev_step.n < n_ev)
+      return fail(NC_ERR_STATE, "event buffer smaller than the queued events");
+    if (n_ev <= kPinEvents) {
+      // (the kinds are bytes, copied as whole words)
+      uint32_t* const h = sim->h_ev;
+      memcpy(h, ev_pos.data(), n_ev * 4);
+      memcpy(h + kPinEvents, ev_step.data(), n_ev * 4);
+      memcpy(h + 2 * kPinEvents, ev_kind.data(), n_ev);
+      part(1, sim->d_ev_pos.p, h, n_ev);
+      part(2, sim->d_ev_step.p, h + kPinEvents, n_ev);
+      part(3, sim->d_ev_kind.p, h + 2 * kPinEvents, (n_ev + 3) / 4);
+    } else {
+      NC_HIP(hipMemcpyAsync(sim->d_ev_pos.p, ev_pos.data(), n_ev * 4, hipMemcpyHostToDevice, st));
+      NC_HIP(hipMemcpyAsync(sim->d_ev_kind.p, ev_kind.data(), n_ev, hipMemcpyHostToDevice, st));
+      NC_HIP(hipMemcpyAsync(sim->d_ev_step.p, ev_step.data(), n_ev * 4, hipMemcpyHostToDevice, st));
     }
   }
-  if (!ev_pos.empty()) {
-    // nc_push_forced and nc_sim_restore reserve room for every queued event
-    if (sim->d_ev_pos.n < ev_pos.size() || sim->d_ev_kind.n < ev_kind.size() || sim->d_ev_step.n < ev_step.size())
-      return fail(NC_ERR_STATE, "event buffer smaller than the queued events");
-    NC_HIP(hipMemcpyAsync(sim->d_ev_pos.p, ev_pos.data(), ev_pos.size() * 4, hipMemcpyHostToDevice, st));
-    NC_HIP(hipMemcpyAsync(sim->d_ev_kind.p, ev_kind.data(), ev_kind.size(), hipMemcpyHostToDevice, st));
-    if (form.network)
-      NC_HIP(hipMemcpyAsync(sim->d_ev_step.p, ev_step.data(), ev_step.size() * 4, hipMemcpyHostToDevice, st));
-  }
+  const uint64_t words = std::max<uint64_t>({b.n[0], b.n[1], 2 * NC_FLISTS});
+  hipLaunchKernelGGL(k_begin, dim3((uint32_t)std::min<uint64_t>((words + 255) / 256, 256)), dim3(256), 0, st, b);
+  NC_HIP(hipGetLastError());
   NC_HIP(hipEventRecord(sim->upload_done, st));
   sim->upload_pending = true;
 
@@ -1425,8 +1461,6 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     NC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, sim->device));
     pgrid = std::min<uint32_t>((uint32_t)std::max(per_cu, 0) * (uint32_t)std::max(cus, 0), std::max(grid, fan_grid));
     if (pgrid * wpb < NC_FLISTS) return fail(NC_ERR_STATE, "the device holds too few workgroups for the persistent form");
-    hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, st, bar, 1u, 0u);
-    NC_HIP(hipGetLastError());
   }
   switch (form.wide_waves) {
     case 1: fn_neuron = (const void*)k_neuron_wide<1>; break;
@@ -1436,13 +1470,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   }
   const uint32_t n_grid = form.wide_waves ? a.n_active_slices : grid;
   const uint32_t n_block = 64 * (form.wide_waves ? form.wide_waves : wpb);
-  a.activity = sim->d_chunk_off + 160;
-  const uint32_t call_tag = (uint32_t)(++sim->calls & 0x7FFFFFFFu) << 1;
-  hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, st, sim->d_chunk_off, 1u, 0u);
-  NC_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_zero_strided, dim3(1), dim3(2 * NC_FLISTS), 0, st, sim->fired_cnt, 2u * NC_FLISTS,
-                     (uint32_t)NC_FCNT_STRIDE);
-  NC_HIP(hipGetLastError());
+  sim->calls = sim->calls % 0xFFFFFFFFu + 1u;
   size_t nev_used = 0;
   std::vector<int> timed_kinds;
   auto launch = [&](int kind, const void* fn, uint32_t g, uint32_t block, uint32_t shmem) -> nc_status {
@@ -1516,7 +1544,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       NC_HIP(hipGetLastError());
     }
     if (form.network) {
-      if (c0 + len == max_run) a.call_tag = call_tag;
+      if (c0 + len == max_run) a.call_tag = sim->calls;
       a.n_ev = (uint32_t)ev_pos.size();
       a.ev_pos = sim->d_ev_pos.p;
       a.ev_kind = sim->d_ev_kind.p;
@@ -1545,7 +1573,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
         if (s1 == NC_OK) s1 = launch(1, fn_step, pgrid, 64 * wpb, lds);
       } else {
         if (s1 == NC_OK) s1 = launch(1, fn_neuron, n_grid, n_block, lds);
-        if (i + 1 == max_run) a.call_tag = call_tag;
+        if (i + 1 == max_run) a.call_tag = sim->calls;
         if (s1 == NC_OK) s1 = launch(3, fn_fanout, fan_grid, 64 * wpb, 0);
       }
       if (s1 != NC_OK) return s1;
@@ -1641,11 +1669,10 @@ namespace {
 // After a synchronisation: did a grid barrier of the persistent form time out
 // (a grid whose workgroups were not all resident) since the last check?
 nc_status check_barrier(nc_sim* sim) {
-  uint32_t words[97];  // word 64 and the activity report
-  NC_HIP(hipMemcpy(words, sim->d_chunk_off + 64, sizeof words, hipMemcpyDeviceToHost));
-  sim->busy = (words[96] & 1u) != 0;
-  if (!words[0]) return NC_OK;
-  NC_HIP(hipMemset(sim->d_chunk_off + 64, 0, 4));
+  volatile uint32_t* const w = sim->h_words;
+  sim->busy = sim->calls && w[0] == sim->calls;
+  if (!w[1]) return NC_OK;
+  w[1] = 0u;
   return fail(NC_ERR_STATE, "a grid barrier of the persistent launch timed out: the steps since the last check "
                             "are invalid");
 }

@@ -189,14 +189,15 @@ struct nc_step_args {
   const uint32_t* ev_pos;  // host events of this step
   const uint8_t* ev_kind;
   uint32_t n_ev;
-  uint32_t* activity;  // what nc_report leaves
-  uint32_t call_tag;   // call number << 1 on the launch that reports, else 0
+  uint32_t* host_words;  // pinned host memory: [0] the last call found busy, [1] a grid barrier timed out
+  uint32_t call_tag;     // call number on the launch that reports, else 0
 };
 
 // How busy the networks are, for the host's choice of the next call's form:
-// the newest call's word wins, and in it "busy" over "quiet".
+// the call's number where it found them busy (every writer writes the same).
 __device__ __forceinline__ void nc_report(const nc_step_args& a, bool busy) {
-  if (a.call_tag) atomicMax(a.activity, a.call_tag | (busy ? 1u : 0u));
+  if (a.call_tag && busy)
+    __hip_atomic_store(a.host_words, a.call_tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 #define NC_BUSY_LANES 6u  // fired lanes per slice and step from which a network is busy
 
@@ -297,8 +298,25 @@ __global__ void k_advance(uint32_t* chunk_off, uint32_t steps) {
 __global__ void k_set_u32(uint32_t* p, uint32_t n, uint32_t v) {
   if (threadIdx.x < n) p[threadIdx.x] = v;
 }
-__global__ void k_zero_strided(uint32_t* p, uint32_t n, uint32_t stride) {
-  if (threadIdx.x < n) p[threadIdx.x * stride] = 0u;
+
+// What a call of nc_sim_step starts with, in one launch: its network windows
+// and host events from pinned host memory to their device arrays, the chunk
+// offset, the barrier count and both parities' fired-list lengths cleared.
+// (As three copies and three launches these were half of a one-step call of a
+// small network: 43 us with its wait, 27 so.)
+struct nc_begin {
+  uint32_t* dst[4];
+  const uint32_t* src[4];
+  uint32_t n[4];  // words
+  uint32_t *chunk_off, *bar, *fired_cnt;
+};
+__global__ __launch_bounds__(256) void k_begin(nc_begin b) {
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x, stride = gridDim.x * 256u;
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+    for (uint32_t i = t; i < b.n[p]; i += stride) b.dst[p][i] = b.src[p][i];
+  if (t < 2u * NC_FLISTS) b.fired_cnt[t * NC_FCNT_STRIDE] = 0u;
+  if (t == 0) *b.chunk_off = 0u, *b.bar = 0u;
 }
 
 // Slot index of in-slot k of lane l in a slice whose slots start at slot_off
@@ -1044,7 +1062,7 @@ __device__ __forceinline__ void nc_grid_barrier(uint32_t* bar, uint32_t target, 
       __builtin_amdgcn_s_sleep(2);
       // bounded by time and, should the clock not advance, by count
       if (__builtin_amdgcn_s_memrealtime() - t0 > NC_BARRIER_TICKS || ++spins > NC_BARRIER_SPINS) {
-        __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         break;
       }
     }
@@ -1057,8 +1075,7 @@ __device__ __forceinline__ void nc_grid_barrier(uint32_t* bar, uint32_t target, 
 // every wave takes active slices w, w + waves, ... through the neuron phase,
 // the grid meets at a barrier, then all waves share the fan-out.  The
 // launch's end orders it before the next step.  bar[0] counts barrier
-// arrivals in this call (zeroed at its start), bar[32] flags a timed-out
-// wait.
+// arrivals in this call (zeroed at its start).
 template <int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_step(nc_step_args a, uint32_t* bar) {
   const uint32_t blk = blockIdx.x % a.ctr_rows;
@@ -1068,6 +1085,6 @@ __global__ __launch_bounds__(64 * WPB) void k_step(nc_step_args a, uint32_t* bar
   const float* tpre = nc_trace_tables<WPB>(a);
   // every wave of the grid runs the same number of slice passes
   for (uint32_t b = 0; b < a.n_active_slices; b += nwaves) nc_neuron_slice<WPB>(a, blk, b + w0, ci, tpre);
-  nc_grid_barrier(bar, ((uint32_t)ci + 1u) * gridDim.x, bar + 32);
+  nc_grid_barrier(bar, ((uint32_t)ci + 1u) * gridDim.x, a.host_words + 1);
   nc_fanout_wave(a, blk, w0 % NC_FLISTS, w0 / NC_FLISTS, nwaves / NC_FLISTS, ci);
 }
