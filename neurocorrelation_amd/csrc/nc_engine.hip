@@ -261,7 +261,7 @@ std::shared_ptr<const NetImage> build_image(const nc_net& net) {
   fnv_mix(&h, net.delay.data(), net.delay.size());
   fnv_mix(&h, net.inh.data(), net.inh.size());
   M.digest = h;
-  M.in_ptr = net.in_ptr;
+  M.in_ptr.assign(net.in_ptr.begin(), net.in_ptr.end());
   // Slot records, in layout order.
   I.slot_w.assign(L.nslots, 0.0f);
   I.slot_inh.assign((L.nslots + 31) / 32, 0u);
@@ -409,6 +409,7 @@ struct DevBuf {
 
 struct nc_sim {
   int device = 0;
+  bool counted = false;  // among nc::xfer_user's
   hipStream_t stream = nullptr;
   uint64_t max_pos = 0, max_slots = 0, max_out = 0;
   uint32_t max_nets = 0, raster_cap = 0;
@@ -696,7 +697,10 @@ nc_status deliver(nc_sim* sim, void* out, size_t bytes, void* dev, F fill) {
   const bool pinned = bytes <= kPinBytes;
   fill(pinned ? (void*)sim->h_pin : dev);
   NC_HIP(hipGetLastError());
-  if (!pinned) NC_HIP(hipMemcpyAsync(out, dev, bytes, hipMemcpyDeviceToHost, sim->stream));
+  if (!pinned) {
+    const nc::Segment g{out, dev, bytes};
+    NC_HIP(nc::download(sim->device, sim->stream, &g, 1));
+  }
   NC_HIP(hipStreamSynchronize(sim->stream));
   if (pinned) memcpy(out, sim->h_pin, bytes);
   return check_barrier(sim);
@@ -709,7 +713,8 @@ nc_status fetch(nc_sim* sim, const void* in, size_t bytes, const void** at) {
     *at = sim->h_pin;
     return NC_OK;
   }
-  NC_HIP(hipMemcpyAsync(sim->d_stage.p, in, bytes, hipMemcpyHostToDevice, sim->stream));
+  const nc::Segment g{const_cast<void*>(in), sim->d_stage.p, bytes};
+  NC_HIP(nc::upload(sim->device, sim->stream, &g, 1));
   *at = sim->d_stage.p;
   return NC_OK;
 }
@@ -892,6 +897,8 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
   sim->a_masks.init(sim->max_mwords / 64);
   if (st != NC_OK) return st;
   *out = guard.release();
+  nc::xfer_user(1);
+  sim->counted = true;
   return NC_OK;
 }
 NC_ABI_CATCH
@@ -912,6 +919,7 @@ extern "C" void nc_sim_destroy(nc_sim* sim) {
   for (hipEvent_t e : sim->ev_pool) (void)hipEventDestroy(e);
   if (sim->upload_done) (void)hipEventDestroy(sim->upload_done);
   if (sim->stream) (void)hipStreamDestroy(sim->stream);
+  if (sim->counted) nc::xfer_user(-1);
   delete sim;
 }
 
@@ -1833,9 +1841,11 @@ extern "C" nc_status nc_read_synapse_state(nc_sim* sim, int32_t net_id, int32_t*
                        (int32_t)r->steps_done, sim->T.r_rel, (int32_t*)at(0), (int32_t*)at(1), (float*)at(2),
                        (uint32_t)n);
     NC_HIP(hipGetLastError());
+    std::vector<nc::Segment> seg;
     if (!pinned)
       for (int i = 0; i < 3; ++i)
-        if (want[i]) NC_HIP(hipMemcpyAsync(want[i], at(i), 4 * n, hipMemcpyDeviceToHost, sim->stream));
+        if (want[i]) seg.push_back(nc::Segment{want[i], at(i), 4 * n});
+    NC_HIP(nc::download(sim->device, sim->stream, seg.data(), seg.size()));
   }
   NC_HIP(hipStreamSynchronize(sim->stream));
   if (pinned && n)
@@ -1974,7 +1984,8 @@ extern "C" nc_status nc_sim_restore(nc_sim* sim, int32_t net_id, const void* buf
   uint32_t bad = 0;
   if (h.n) {
     uint32_t* const flag = sim->d_chunk_off + 192;
-    NC_HIP(hipMemcpyAsync(sim->d_stage.p, p, state, hipMemcpyHostToDevice, sq));
+    const nc::Segment g{const_cast<unsigned char*>(p), sim->d_stage.p, state};
+    NC_HIP(nc::upload(sim->device, sq, &g, 1));
     hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, sq, flag, 1u, 0u);
     NC_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_check_checkpoint, dim3((uint32_t)std::min<uint64_t>((h.n + h.n_syn + 255) / 256, 2048)),

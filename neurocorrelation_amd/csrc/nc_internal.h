@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/neucor_amd.h"
+#include "nc_hostmem.h"
 
 // A network on the host.  Incoming synapses of neuron i are
 // [in_ptr[i], in_ptr[i+1]) with strictly ascending source id: the iteration
@@ -20,12 +21,13 @@ struct NetImage;  // the engine's device image of a network (nc_net_prepare)
 
 struct nc_net {
   uint32_t n = 0;
-  std::vector<float> xyz;          // 3 per neuron
-  std::vector<int64_t> in_ptr;     // n + 1
-  std::vector<uint32_t> in_src;    // S
-  std::vector<float> w;            // S
-  std::vector<uint8_t> delay;      // S, steps >= 1
-  std::vector<uint8_t> inh;        // S, 1 = inhibitory sign class
+  // (resize() leaves new elements unset)
+  nc::RawVec<float> xyz;           // 3 per neuron
+  nc::RawVec<int64_t> in_ptr;      // n + 1
+  nc::RawVec<uint32_t> in_src;     // S
+  nc::RawVec<float> w;             // S
+  nc::RawVec<uint8_t> delay;       // S, steps >= 1
+  nc::RawVec<uint8_t> inh;         // S, 1 = inhibitory sign class
   uint32_t max_in_degree = 0;
   uint32_t max_delay = 0;
   // Cached device image, built by nc_net_prepare; a network never changes
@@ -49,6 +51,20 @@ nc_status fail(nc_status code, const std::string& msg);
   }
 void finish_net_stats(nc_net* net);
 nc_status check_wiring_spec(const nc_wiring_spec& s);
+
+#if defined(__HIP__)
+// Copies between device and pageable host memory (nc_xfer.hip), in the order
+// of the stream; done when they return.
+struct Segment {
+  void *host, *dev;
+  size_t bytes;
+};
+hipError_t download(int device, hipStream_t st, const Segment* seg, size_t n_seg);
+hipError_t upload(int device, hipStream_t st, const Segment* seg, size_t n_seg);
+// A simulation came (+1) or went (-1): the last one's end frees the pinned
+// memory kept between copies.
+void xfer_user(int change);
+#endif
 
 // Input selection shared by the engine and nc_net_select_inputs.
 struct InputSel {

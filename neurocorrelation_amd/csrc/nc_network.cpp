@@ -304,12 +304,12 @@ extern "C" nc_status nc_net_export(const nc_net* net, float* xyz, int64_t* in_pt
                                    float* w, uint8_t* delay_steps, uint8_t* inhibitory) try {
   if (!net) return fail(NC_ERR_ARG, "null network");
   const uint64_t S = net->n_syn();
-  if (xyz) memcpy(xyz, net->xyz.data(), 12ull * net->n);
-  if (in_ptr) memcpy(in_ptr, net->in_ptr.data(), 8ull * (net->n + 1));
-  if (in_src) memcpy(in_src, net->in_src.data(), 4 * S);
-  if (w) memcpy(w, net->w.data(), 4 * S);
-  if (delay_steps) memcpy(delay_steps, net->delay.data(), S);
-  if (inhibitory) memcpy(inhibitory, net->inh.data(), S);
+  if (xyz) nc::copy_bytes(xyz, net->xyz.data(), 12ull * net->n);
+  if (in_ptr) nc::copy_bytes(in_ptr, net->in_ptr.data(), 8ull * (net->n + 1));
+  if (in_src) nc::copy_bytes(in_src, net->in_src.data(), 4 * S);
+  if (w) nc::copy_bytes(w, net->w.data(), 4 * S);
+  if (delay_steps) nc::copy_bytes(delay_steps, net->delay.data(), S);
+  if (inhibitory) nc::copy_bytes(inhibitory, net->inh.data(), S);
   return NC_OK;
 }
 NC_ABI_CATCH

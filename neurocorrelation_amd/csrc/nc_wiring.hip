@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <new>
 #include <vector>
 
@@ -411,7 +412,7 @@ uint32_t bits_for(uint64_t v) {
 
 }  // namespace
 
-extern "C" nc_status nc_net_generate_device(const nc_wiring_spec* spec, int32_t device, nc_net** out) {
+extern "C" nc_status nc_net_generate_device(const nc_wiring_spec* spec, int32_t device, nc_net** out) try {
   if (!spec || !out) return fail(NC_ERR_ARG, "null argument");
   *out = nullptr;
   const nc_wiring_spec s = *spec;
@@ -541,7 +542,7 @@ extern "C" nc_status nc_net_generate_device(const nc_wiring_spec* spec, int32_t 
                        in_src, w, delay, inh, max_dly);
     NW_HIP(hipGetLastError());
   }
-  nc_net* net = new (std::nothrow) nc_net();
+  std::unique_ptr<nc_net> net(new (std::nothrow) nc_net());
   if (!net) return fail(NC_ERR_OOM, "host allocation failed");
   try {
     net->n = n;
@@ -552,24 +553,18 @@ extern "C" nc_status nc_net_generate_device(const nc_wiring_spec* spec, int32_t 
     net->delay.resize(S);
     net->inh.resize(S);
   } catch (const std::bad_alloc&) {
-    delete net;
     return fail(NC_ERR_OOM, "host allocation failed");
   }
-  hipError_t e = hipMemcpyAsync(net->xyz.data(), xyz, 12ull * n, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(seen, meta, sizeof seen, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(net->in_ptr.data(), in_ptr, 8ull * (n + 1ull), hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess && S) e = hipMemcpyAsync(net->in_src.data(), in_src, 4ull * S, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess && S) e = hipMemcpyAsync(net->w.data(), w, 4ull * S, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess && S) e = hipMemcpyAsync(net->delay.data(), delay, S, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess && S) e = hipMemcpyAsync(net->inh.data(), inh, S, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (e != hipSuccess) {
-    delete net;
-    return fail(NC_ERR_HIP, hipGetErrorString(e));
-  }
+  const nc::Segment seg[] = {
+      {net->in_src.data(), in_src, 4ull * S}, {net->w.data(), w, 4ull * S},
+      {net->delay.data(), delay, S},          {net->inh.data(), inh, S},
+      {net->xyz.data(), xyz, 12ull * n},      {net->in_ptr.data(), in_ptr, 8ull * (n + 1ull)},
+      {seen, meta, sizeof seen}};
+  hipError_t e = nc::download(device, st, seg, sizeof seg / sizeof seg[0]);
+  if (e != hipSuccess) return fail(NC_ERR_HIP, hipGetErrorString(e));
   net->max_in_degree = seen[1];
   net->max_delay = seen[3];
-  *out = net;
+  *out = net.release();
   return NC_OK;
 }
+NC_ABI_CATCH

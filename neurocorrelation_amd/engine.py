@@ -261,14 +261,17 @@ class Simulation:
         """The network's dynamic state as bytes (a checkpoint)."""
         size = C.c_uint64()
         check(lib().nc_sim_save(self._h, net_id, None, 0, C.byref(size)))
-        buf = C.create_string_buffer(size.value)
-        check(lib().nc_sim_save(self._h, net_id, buf, size.value, C.byref(size)))
-        return buf.raw[:size.value]
+        # the call fills a new bytes object in place, before anything else holds it
+        new_bytes = C.pythonapi.PyBytes_FromStringAndSize
+        new_bytes.restype, new_bytes.argtypes = C.py_object, [C.c_char_p, C.c_ssize_t]
+        data = new_bytes(None, size.value)
+        check(lib().nc_sim_save(self._h, net_id, C.cast(C.c_char_p(data), C.c_void_p), size.value, C.byref(size)))
+        return data
 
     def restore(self, net_id, data):
         """Loads a checkpoint into a network just added from the same wiring."""
-        buf = C.create_string_buffer(bytes(data), len(data))
-        check(lib().nc_sim_restore(self._h, net_id, buf, len(data)))
+        data = bytes(data)
+        check(lib().nc_sim_restore(self._h, net_id, data, len(data)))
 
     def set_counting(self, enable):
         check(lib().nc_set_counting(self._h, 1 if enable else 0))
