@@ -142,3 +142,15 @@ def test_busy_many_slices(n, nets):
         got.append(out)
         sim.close()
     _same(*got)
+
+
+def test_own_graphs_from_the_second_equal_call():
+    # 3000 quiet neurons: the second and later calls of more than 16 steps run
+    # as captured chunks; a call with events, a shorter one, a host write and a
+    # longer one than the drive ring come between
+    net = _net(3000, 60, delay_max=40, seed=6, inhib=0.2, w=(0.05, 0.3))
+
+    def events(i, steps):
+        m = 20 if i == 3 else 0
+        return np.arange(m) % 30 + 1, np.arange(m), np.zeros(m)
+    _both(net, _drive(3000, seed=6, bg=0.003), 1.0, [40, 40, 33, 40, 17, 40, 1100, 5, 40], events=events)
