@@ -1252,9 +1252,14 @@ namespace {
 //     1563 quiet slices take 13.6 against 12.0 of k_neuron.
 //   - above, one wave, if busy (19 200 slices: 464 against 487); 10^6 quiet
 //     neurons take 91.7 against 87.4 of k_neuron.
+//   - above 8192 slices, quiet: k_neuron and k_fanout of one wave per
+//     workgroup in XCD order: 84.2 against 87.5 at 10^6 neurons (an XCD's L2
+//     then holds a run of slices and most of its fan-out targets), 56.0
+//     against 56.2 at 600 000; at 300 000 nothing, below it costs.
 struct Form {
   bool network = false;     // k_net_steps
   uint32_t wide_waves = 0;  // k_neuron_wide with this many waves per slice (0: k_neuron)
+  bool xcd = false;         // k_neuron and k_fanout of one wave per workgroup, in XCD order
 };
 
 Form step_form(const nc_sim* sim) {
@@ -1271,6 +1276,7 @@ Form step_form(const nc_sim* sim) {
   }
   if (slices <= 1024) f.wide_waves = 4;
   else if (sim->busy) f.wide_waves = slices <= 4096 ? 2 : 1;
+  else f.xcd = slices > 8192;
   return f;
 }
 
@@ -1416,7 +1422,8 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   // nc_sim_add sizes the drive tables and the group-train ring; nothing here allocates
   if (a.n_groups && (sim->d_groups.n < a.n_groups || sim->d_gfire.n < (size_t)NC_GRING * a.gwords))
     return fail(NC_ERR_STATE, "drive tables were not placed");
-  const uint32_t wpb = sim->cfg.waves_per_block;
+  const uint32_t wpb = form.xcd ? 1u : sim->cfg.waves_per_block;
+  if (form.xcd) a.xcd_swizzle = 1u;
   const uint32_t grid = (a.n_active_slices + wpb - 1) / wpb;
   // A fired list holds at most fcap records (up to NC_FSPLIT per k_neuron
   // wave of its residue).  k_fanout gives the lists about one reader per
@@ -1428,7 +1435,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   // With XCD lists (the XCD-ordered remap, ordinary launches), list (x, j)
   // takes the k_neuron waves of workgroups b = x mod 8 whose rank on the XCD
   // is j mod 8.
-  a.xcd_lists = (sim->cfg.xcd_swizzle && !sim->cfg.persistent) ? 1u : 0u;
+  a.xcd_lists = (a.xcd_swizzle && !sim->cfg.persistent) ? 1u : 0u;
   a.fcap = (a.xcd_lists ? ((grid + 7) / 8 * wpb + 7) / 8 : (grid * wpb + NC_FLISTS - 1) / NC_FLISTS) * NC_FSPLIT;
   uint64_t syn_active = 0, n_active = 0;
   for (size_t i = 0; i < sim->nets.size(); ++i)

@@ -122,6 +122,13 @@ def test_uneven_budgets():
     _same(*got)
 
 
+def test_quiet_many_slices():
+    # more than 8192 slices, which the default shape takes in XCD order
+    net = nc.Network.generate(530_000, W.side_for(530_000), W.radius_for_degree(8), 1, 20, 0.05, 0.3, 0.2, seed=2,
+                              device=0)
+    _both(net, _drive(530_000, seed=2, bg=0.01), 1.0, [30, 30], cap=1 << 21)
+
+
 # busy simulations of more than 1024 and more than 4096 slices, in networks of
 # more than 16: two waves and one wave per slice, from the second call on (the
 # first one's activity is read back with its state)
