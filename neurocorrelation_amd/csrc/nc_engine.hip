@@ -77,6 +77,14 @@ namespace {
 
 constexpr uint32_t kSigma = 1024;
 
+// Staging words of a result's digest: its words, a byte per low byte and piece
+// for the maps, and the groups' maps and starts.
+inline uint64_t digest_words(uint64_t n, uint64_t S) {
+  const uint64_t m = 2 * n + S, pieces = (m + NC_FNV_PIECE - 1) / NC_FNV_PIECE;
+  const uint64_t groups = m / (NC_FNV_SEG * NC_FNV_GROUP) + 1;
+  return m + 64 * pieces + 65 * groups + 64;
+}
+
 // Results up to this size are written by the kernels into pinned host memory
 // (one launch and one wait); larger ones are staged on the device and copied.
 constexpr size_t kPinBytes = 1u << 20;
@@ -1138,7 +1146,7 @@ extern "C" nc_status nc_sim_add(nc_sim* sim, const nc_net* net, const nc_params*
   // to a staging buffer; the placing kernels expand it into the records.
   const uint64_t n_inh = I.slot_inh.size(), o_jq = (I.nslots + n_inh + 1) & ~1ull;
   {
-    nc_status sg = grow(&sim->d_stage, std::max<uint64_t>(o_jq + 2 * S + 2, 3ull * net->n + 4 * S + 4), st);
+    nc_status sg = grow(&sim->d_stage, std::max<uint64_t>({o_jq + 2 * S + 2, 3ull * net->n + 4 * S + 4, digest_words(net->n, S)}), st);
     if (sg != NC_OK) {
       if (r.has_drive) {
         const nc_group dead{0u, 1u, 0u, sim->max_nets};
@@ -1780,6 +1788,56 @@ extern "C" nc_status nc_read_weights_noalloc(nc_sim* sim, int32_t net_id, float*
   return export_weights(sim, *r, scr, out, n);
 }
 NC_ABI_CATCH
+
+nc_status nc::sim_result(nc_sim* sim, int32_t net_id, uint64_t* digest, uint64_t* spikes) {
+  NetRec* r;
+  nc_status st = check_net(sim, net_id, &r);
+  if (st != NC_OK) return st;
+  NC_HIP(hipSetDevice(sim->device));
+  const uint64_t h0 = 14695981039346656037ull;
+  const uint64_t m64 = 2ull * r->n + r->S;
+  if (m64 < 16384 || m64 >= (1ull << 32) - NC_FNV_SEG * NC_FNV_GROUP) {
+    // a few words are hashed sooner than six kernels run
+    std::vector<float> V(r->n), w(r->S);
+    std::vector<uint32_t> f(r->n);
+    st = nc_read_potential(sim, net_id, V.data(), r->n);
+    if (st == NC_OK) st = nc_read_weights(sim, net_id, w.data(), r->S);
+    if (st == NC_OK) st = nc_read_firings(sim, net_id, f.data(), r->n);
+    if (st != NC_OK) return st;
+    *digest = nc_digest(f.data(), 4ull * r->n, nc_digest(w.data(), 4ull * r->S, nc_digest(V.data(), 4ull * r->n, h0)));
+    *spikes = std::accumulate(f.begin(), f.end(), (uint64_t)0);
+    return NC_OK;
+  }
+  const uint32_t m = (uint32_t)m64, pieces = (m + NC_FNV_PIECE - 1) / NC_FNV_PIECE;
+  const uint32_t segs = (m + NC_FNV_SEG - 1) / NC_FNV_SEG, groups = (segs + NC_FNV_GROUP - 1) / NC_FNV_GROUP;
+  uint32_t* const words = sim->d_stage.p;
+  uint8_t* const maps = (uint8_t*)(words + (m + 63) / 64 * 64);
+  uint8_t* const gmaps = maps + 256ull * pieces;
+  uint8_t* const starts = gmaps + 256ull * groups;
+  unsigned long long* const sums = (unsigned long long*)(sim->d_chunk_off + 200);
+  hipStream_t q = sim->stream;
+  hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, q, (uint32_t*)sums, 4u, 0u);
+  NC_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_result_words, row_blocks(*r), dim3(256), 0, q, place_of(sim, *r), sim->V, sim->firings,
+                     (uint32_t)r->S, words, sums + 1);
+  NC_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_fnv_maps, dim3(segs), dim3(256), 0, q, words, m, maps);
+  NC_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_fnv_groups, dim3(groups), dim3(256), 0, q, maps, pieces, gmaps);
+  NC_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_fnv_starts, dim3(1), dim3(256), 0, q, gmaps, groups, (uint32_t)(h0 & 255u), starts);
+  NC_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_fnv_sum, dim3(groups * (NC_FNV_SEG / NC_FNV_PIECE)), dim3(64), 0, q, words, m, maps, starts, h0,
+                     sums);
+  NC_HIP(hipGetLastError());
+  NC_HIP(hipMemcpyAsync(sim->h_pin, sums, 16, hipMemcpyDeviceToHost, q));
+  NC_HIP(hipStreamSynchronize(q));
+  uint64_t got[2];
+  memcpy(got, sim->h_pin, 16);
+  *digest = got[0];
+  *spikes = got[1];
+  return check_barrier(sim);
+}
 
 extern "C" nc_status nc_write_weights(nc_sim* sim, int32_t net_id, const float* w, uint64_t n) try {
   NetRec* r;

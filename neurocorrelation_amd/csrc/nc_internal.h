@@ -52,6 +52,11 @@ nc_status fail(nc_status code, const std::string& msg);
 void finish_net_stats(nc_net* net);
 nc_status check_wiring_spec(const nc_wiring_spec& s);
 
+// A network's potentials, weights (export order) and firings digested as
+// nc_digest does in that order from the offset basis, and the sum of its
+// firings.
+nc_status sim_result(nc_sim* sim, int32_t net_id, uint64_t* digest, uint64_t* spikes);
+
 #if defined(__HIP__)
 // Copies between device and pageable host memory (nc_xfer.hip), in the order
 // of the stream; done when they return.

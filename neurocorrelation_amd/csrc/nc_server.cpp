@@ -154,23 +154,13 @@ void builder_main(nc_server* s) {
   }
 }
 
-// The finished job's result: potentials, weights (export order) and firing
-// counts hashed in that order.
+// The finished job's result: its firings, and the digest of potentials,
+// weights (export order) and firing counts.
 nc_status finish_job(nc_server* s, Lane& L, JobRec* j) {
-  std::vector<float> V(j->n);
-  std::vector<float> w(j->S);
-  std::vector<uint32_t> f(j->n);
-  nc_status r = nc_read_potential(L.sim, j->nid, V.data(), j->n);
-  if (r == NC_OK) r = nc_read_weights(L.sim, j->nid, w.data(), j->S);
-  if (r == NC_OK) r = nc_read_firings(L.sim, j->nid, f.data(), j->n);
+  uint64_t h = 0, spikes = 0;
+  nc_status r = nc::sim_result(L.sim, j->nid, &h, &spikes);
   if (r == NC_OK) r = nc_sim_remove(L.sim, j->nid);
   if (r != NC_OK) return r;
-  uint64_t h = 14695981039346656037ull;
-  h = nc_digest(V.data(), 4ull * j->n, h);
-  h = nc_digest(w.data(), 4ull * j->S, h);
-  h = nc_digest(f.data(), 4ull * j->n, h);
-  uint64_t spikes = 0;
-  for (uint32_t x : f) spikes += x;
   std::lock_guard<std::mutex> g(s->mu);
   j->res.status = NC_OK;
   j->res.spikes = spikes;
