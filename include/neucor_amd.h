@@ -412,7 +412,7 @@ typedef struct nc_server nc_server;
 
 typedef struct nc_server_spec {
   int32_t device;
-  uint32_t lanes;          /* simulations stepped in turn (0 = 2) */
+  uint32_t lanes;          /* simulations, each stepped on its own stream (0 = 2) */
   uint32_t chunk;          /* steps per lane turn (0 = 200) */
   uint32_t builders;       /* host threads building job networks (0 = 4) */
   uint32_t device_wiring;  /* 1: build job networks with nc_net_generate_device */
