@@ -409,6 +409,23 @@ struct NetRec {
   std::vector<std::pair<uint32_t, std::pair<uint32_t, uint8_t>>> events;  // abs step, (pos, kind)
 };
 
+// Arrays cut from one allocation: at multiples of 2 MiB if that large, else of
+// 256 bytes.
+struct Arena {
+  std::vector<std::pair<void**, uint64_t>> a;  // where the pointer goes, its offset
+  uint64_t bytes = 0;
+  template <class T>
+  void want(T** p, uint64_t n) {
+    const uint64_t need = n * sizeof(T), to = need >= (2ull << 20) ? 2ull << 20 : 256;
+    bytes = (bytes + to - 1) / to * to;
+    if (n) a.push_back({(void**)p, bytes});
+    bytes += need;
+  }
+  void place(void* base) {
+    for (auto& x : a) *x.first = (unsigned char*)base + x.second;
+  }
+};
+
 template <class T>
 struct DevBuf {
   T* p = nullptr;
@@ -436,7 +453,8 @@ struct nc_sim {
   double k_ms[4] = {0, 0, 0, 0};
   std::vector<hipEvent_t> ev_pool;
 
-  // device buffers
+  // device buffers: one allocation, cut into the arrays that follow
+  void* arena = nullptr;
   nc_slot* slots = nullptr;
   uint32_t* amask = nullptr;
   uint32_t* asum = nullptr;
@@ -453,7 +471,7 @@ struct nc_sim {
   uint4* acache = nullptr;         // active-slot cache: one 16-byte entry per position
   uint32_t *id_pos = nullptr, *id_row = nullptr;  // per network, at its positions: neuron id -> local position, first synapse
   uint32_t* slice_moff = nullptr;  // per slice: first active-mask word
-  uint32_t *slice_off = nullptr, *slice_net = nullptr;
+  uint32_t* slice_off = nullptr;
   nc_slice_rec* active = nullptr;
   nc_net_rec* net_recs = nullptr;  // live networks with neurons, for the workgroup-per-network form
   uint32_t *forced_in = nullptr, *forced_bg = nullptr;
@@ -760,7 +778,7 @@ extern "C" nc_status nc_sim_footprint(uint64_t n_neurons, uint64_t n_syn, uint64
   const uint64_t mwords = slots / 32 + 64 * Q;
   *bytes = P * (4 + 12 + 8 + 4 + 8) + P / 4                // asum, V/lastFire/firings, ndw, nid, out_row, forced
            + P * sizeof(uint4)                             // active-slot cache
-           + Q * (8 + 4 + 4 + sizeof(nc_slice_rec))       // pend_cnt, slice_off, slice_net, active
+           + Q * (8 + 4 + 4 + sizeof(nc_slice_rec))       // pend_cnt, slice_off, slice_moff, active
            + (Q + NC_FLISTS * 8) * NC_FSPLIT * 16          // fired lists
            + Q * NC_NB * (4ull + 8ull * NC_BCAP) + Q * 4     // arrival buckets, slice mask offsets
            + slots * (sizeof(nc_slot) + 8) + mwords * 4    // slot records, pending lists, active masks
@@ -833,34 +851,33 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
   const uint64_t P = sim->max_pos, Q = P / 64;
   sim->max_mwords = sim->max_slots / 32 + 64 * Q;
   if (st == NC_OK) {
-    H(hipMalloc(&sim->amask, sim->max_mwords * 4), "hipMalloc amask");
-    H(hipMalloc(&sim->asum, P * 4), "hipMalloc asum");
-    H(hipMalloc(&sim->slots, sim->max_slots * sizeof(nc_slot)), "hipMalloc slots");
-    H(hipMalloc(&sim->V, P * 4), "hipMalloc V");
-    H(hipMalloc(&sim->last_fire, P * 4), "hipMalloc lastFire");
-    H(hipMalloc(&sim->firings, P * 4), "hipMalloc firings");
-    H(hipMalloc(&sim->ndw, P * sizeof(uint2)), "hipMalloc ndw");
-    H(hipMalloc(&sim->nid, P * 4), "hipMalloc nid");
-    H(hipMalloc(&sim->out_row, P * sizeof(uint2)), "hipMalloc out_row");
-    H(hipMalloc(&sim->edges, sim->max_out * sizeof(nc_edge)), "hipMalloc edges");
-    H(hipMalloc(&sim->pend0, sim->max_slots * 4), "hipMalloc pend0");
-    H(hipMalloc(&sim->pend1, sim->max_slots * 4), "hipMalloc pend1");
-    H(hipMalloc(&sim->pend_cnt, Q * sizeof(uint2)), "hipMalloc pend_cnt");
-    H(hipMalloc(&sim->bcnt, Q * NC_NB * 4ull), "hipMalloc bcnt");
-    H(hipMalloc(&sim->bent, Q * NC_NB * NC_BCAP * sizeof(uint2)), "hipMalloc bent");
-    H(hipMalloc(&sim->acache, P * sizeof(uint4)), "hipMalloc acache");
-    H(hipMalloc(&sim->slice_moff, Q * 4), "hipMalloc slice_moff");
-    H(hipMalloc(&sim->id_pos, P * 4), "hipMalloc id_pos");
-    H(hipMalloc(&sim->id_row, P * 4), "hipMalloc id_row");
-    H(hipMalloc(&sim->slice_off, Q * 4), "hipMalloc slice_off");
-    H(hipMalloc(&sim->slice_net, Q * 4), "hipMalloc slice_net");
-    H(hipMalloc(&sim->active, Q * sizeof(nc_slice_rec)), "hipMalloc active");
-    H(hipMalloc(&sim->net_recs, sim->max_nets * sizeof(nc_net_rec)), "hipMalloc network records");
-    H(hipMalloc(&sim->forced_in, (P / 32) * 4), "hipMalloc forced_in");
-    H(hipMalloc(&sim->forced_bg, (P / 32) * 4), "hipMalloc forced_bg");
-    H(hipMalloc(&sim->fired, (Q + NC_FLISTS * 8ull) * NC_FSPLIT * sizeof(uint4)), "hipMalloc fired");
-    H(hipMalloc(&sim->fired_cnt, 2ull * NC_FLISTS * NC_FCNT_STRIDE * 4), "hipMalloc fired_cnt");
-
+    // One allocation, cut into the arrays: first those that start cleared.
+    Arena R;
+    sim->ctr_rows = Q + 2;
+    R.want(&sim->amask, sim->max_mwords), R.want(&sim->asum, P), R.want(&sim->ndw, P);
+    R.want(&sim->forced_in, P / 32), R.want(&sim->forced_bg, P / 32);
+    R.want(&sim->fired, (Q + NC_FLISTS * 8ull) * NC_FSPLIT), R.want(&sim->fired_cnt, 2ull * NC_FLISTS * NC_FCNT_STRIDE);
+    R.want(&sim->pend_cnt, Q), R.want(&sim->bcnt, Q * NC_NB), R.want(&sim->acache, P);
+    R.want(&sim->raster_cnt, 16), R.want(&sim->ctr, sim->ctr_rows * NC_NCTR);
+    // word 0: chunk offset; word 32: grid-barrier arrivals of the call;
+    // word 128: zero, the group-spike-train word read when there are no
+    // groups; word 192: a checkpoint's faults (nc_sim_restore); words
+    // 200-203: a result's digest and firings (sim_result)
+    R.want(&sim->d_chunk_off, 256);
+    // one more, never written: the (never live) network of hole records
+    R.want(&sim->d_nets, sim->max_nets + 1ull);
+    const uint64_t cleared = R.bytes;
+    R.want(&sim->slots, sim->max_slots), R.want(&sim->edges, sim->max_out);
+    R.want(&sim->pend0, sim->max_slots), R.want(&sim->pend1, sim->max_slots), R.want(&sim->bent, Q * NC_NB * NC_BCAP);
+    R.want(&sim->V, P), R.want(&sim->last_fire, P), R.want(&sim->firings, P), R.want(&sim->nid, P);
+    R.want(&sim->out_row, P), R.want(&sim->id_pos, P), R.want(&sim->id_row, P);
+    R.want(&sim->slice_off, Q), R.want(&sim->slice_moff, Q), R.want(&sim->active, Q);
+    R.want(&sim->net_recs, sim->max_nets), R.want(&sim->raster, 2ull * sim->raster_cap);
+    H(hipMalloc(&sim->arena, R.bytes), "hipMalloc");
+    if (st == NC_OK) {
+      R.place(sim->arena);
+      H(hipMemsetAsync(sim->arena, 0, cleared, sim->stream), "memset");
+    }
     H(hipHostMalloc((void**)&sim->h_pin, kPinBytes + 64 + sim->max_nets * sizeof(nc_netdesc) + kPinEvents * 12,
                     hipHostMallocDefault), "hipHostMalloc");
     if (sim->h_pin) {
@@ -869,38 +886,11 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
       sim->h_ev = (uint32_t*)(sim->h_nds + sim->max_nets);
       sim->h_words[0] = sim->h_words[1] = 0u;
     }
-    H(hipMalloc(&sim->raster_cnt, 64), "hipMalloc raster_cnt");
-    if (sim->raster_cap) H(hipMalloc(&sim->raster, 8ull * sim->raster_cap), "hipMalloc raster");
-    sim->ctr_rows = Q + 2;
-    // word 0: chunk offset; word 32: grid-barrier arrivals of the call;
-    // word 128: zero, the group-spike-train word read when there are no
-    // groups; word 192: a checkpoint's faults (nc_sim_restore)
-    H(hipMalloc(&sim->d_chunk_off, 1024), "hipMalloc chunk_off");
-    H(hipMalloc(&sim->ctr, sim->ctr_rows * NC_NCTR * 8), "hipMalloc ctr");
-    // one more, never written: the (never live) network of hole records
-    H(hipMalloc(&sim->d_nets, (sim->max_nets + 1ull) * sizeof(nc_netdesc)), "hipMalloc nets");
   }
   if (st == NC_OK) {
-    H(hipMemsetAsync(sim->amask, 0, sim->max_mwords * 4, sim->stream), "memset");
-    H(hipMemsetAsync(sim->asum, 0, P * 4, sim->stream), "memset");
-    H(hipMemsetAsync(sim->ndw, 0, P * sizeof(uint2), sim->stream), "memset");
-    H(hipMemsetAsync(sim->forced_in, 0, (P / 32) * 4, sim->stream), "memset");
-    H(hipMemsetAsync(sim->forced_bg, 0, (P / 32) * 4, sim->stream), "memset");
-    H(hipMemsetAsync(sim->fired, 0, (Q + NC_FLISTS * 8ull) * NC_FSPLIT * sizeof(uint4), sim->stream), "memset");
-    H(hipMemsetAsync(sim->fired_cnt, 0, 2ull * NC_FLISTS * NC_FCNT_STRIDE * 4, sim->stream), "memset");
-    H(hipMemsetAsync(sim->pend_cnt, 0, Q * sizeof(uint2), sim->stream), "memset");
-    H(hipMemsetAsync(sim->bcnt, 0, Q * NC_NB * 4ull, sim->stream), "memset");
-    H(hipMemsetAsync(sim->acache, 0, P * sizeof(uint4), sim->stream), "memset");
-
-    H(hipMemsetAsync(sim->raster_cnt, 0, 64, sim->stream), "memset");
-    H(hipMemsetAsync(sim->d_chunk_off, 0, 1024, sim->stream), "memset");
-    H(hipMemsetAsync(sim->ctr, 0, sim->ctr_rows * NC_NCTR * 8, sim->stream), "memset");
-    H(hipMemsetAsync(sim->d_nets, 0, (sim->max_nets + 1ull) * sizeof(nc_netdesc), sim->stream), "memset");
-    std::vector<uint32_t> none(Q, NC_SLICE_NONE);
-    sim->slice_net_host = none;
+    sim->slice_net_host.assign(Q, NC_SLICE_NONE);
     sim->slice_off_host.assign(Q, 0u);
     sim->slice_moff_host.assign(Q, 0u);
-    H(hipMemcpyAsync(sim->slice_net, none.data(), Q * 4, hipMemcpyHostToDevice, sim->stream), "memcpy");
     H(hipStreamSynchronize(sim->stream), "sync");
   }
   sim->a_slices.init(Q);
@@ -920,11 +910,8 @@ extern "C" void nc_sim_destroy(nc_sim* sim) {
   (void)hipSetDevice(sim->device);
   if (sim->stream) (void)hipStreamSynchronize(sim->stream);
   if (sim->graph) (void)hipGraphExecDestroy(sim->graph);
-  void* ptrs[] = {sim->d_chunk_off, sim->amask, sim->asum, sim->slots, sim->V, sim->last_fire, sim->firings, sim->ndw,
-                  sim->nid, sim->out_row, sim->edges, sim->pend0, sim->pend1, sim->pend_cnt, sim->bcnt, sim->bent, sim->acache, sim->slice_moff, sim->id_pos, sim->id_row, sim->slice_off, sim->slice_net, sim->active, sim->net_recs, sim->forced_in,
-                  sim->forced_bg, sim->fired, sim->fired_cnt, sim->raster, sim->raster_cnt,
-                  sim->ctr, sim->d_nets, sim->t_pre, sim->t_post, sim->w_ap, sim->d_groups.p,
-                  sim->d_thr.p, sim->d_ev_pos.p, sim->d_ev_kind.p, sim->d_ev_step.p, sim->d_gfire.p, sim->d_stage.p};
+  void* ptrs[] = {sim->arena, sim->t_pre, sim->t_post, sim->w_ap, sim->d_groups.p, sim->d_thr.p, sim->d_ev_pos.p,
+                  sim->d_ev_kind.p, sim->d_ev_step.p, sim->d_gfire.p, sim->d_stage.p};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (sim->h_pin) (void)hipHostFree(sim->h_pin);
@@ -1042,20 +1029,9 @@ extern "C" nc_status nc_sim_add(nc_sim* sim, const nc_net* net, const nc_params*
 
   const uint32_t npos = I.nq * 64;
   const uint32_t pos0 = (uint32_t)(q0 * 64);
-  std::vector<uint32_t> slice_off(I.nq), slice_moff(I.nq);
-  for (uint32_t q = 0; q < I.nq; ++q) {
-    slice_off[q] = (uint32_t)sl0 + I.slice_off[q];
-    slice_moff[q] = (uint32_t)mk0 + I.slice_moff[q];
-  }
-  std::vector<uint2> orow(npos);
-  for (uint32_t pl = 0; pl < npos; ++pl) orow[pl] = make_uint2((uint32_t)o0 + I.out_row[pl].x, I.out_row[pl].y);
   // Drive.
-  std::vector<uint2> ndwv(npos);
-  for (uint32_t pl = 0; pl < npos; ++pl) ndwv[pl] = make_uint2(I.degw[pl], 0u);
-  nc_netdesc nd{};
-  nd.lr = r.lr;
-  nd.pre_f = r.pre_f;
-  nd.post_f = r.post_f;
+  std::vector<uint2> inputs;  // (local position, group)
+  bool tables_placed = false;
   if (drive) {
     nc::InputSel sel;
     nc_status stt = nc::select_inputs(*net, *drive, &sel);
@@ -1118,35 +1094,34 @@ extern "C" nc_status nc_sim_add(nc_sim* sim, const nc_net* net, const nc_params*
                             hipMemcpyHostToDevice, sim->stream));
       NC_HIP(hipMemcpyAsync(sim->d_thr.p, sim->thr.data(), sim->thr.size() * 4, hipMemcpyHostToDevice,
                             sim->stream));
-    } else if (r.ngrp) {
-      NC_HIP(hipMemcpyAsync(sim->d_groups.p + g0, sim->groups.data() + g0, r.ngrp * sizeof(nc_group),
-                            hipMemcpyHostToDevice, sim->stream));
-      NC_HIP(hipMemcpyAsync(sim->d_thr.p + t0, sim->thr.data() + t0, r.nthr * 4ull, hipMemcpyHostToDevice,
-                            sim->stream));
+      tables_placed = true;
     }
-    for (size_t k = 0; k < sel.ids.size(); ++k) {
-      uint32_t pl = M.pos_of_id[sel.ids[k]];
-      ndwv[pl].x |= NC_DEG_INPUT;
-      ndwv[pl].y = r.grp0 + sel.group[k];
-    }
-    nd.drive_lo = (uint32_t)drive->seed;
-    nd.drive_hi = (uint32_t)(drive->seed >> 32);
-    if (drive->bg_prob > 0.0f) {
-      double th = floor((double)drive->bg_prob * 4294967296.0);
-      nd.bg_thr = th >= 4294967295.0 ? 0xFFFFFFFFu : (uint32_t)th;
-      if (nd.bg_thr == 0) nd.bg_thr = 1;
-      uint64_t bs = drive->seed ^ 0x9E3779B97F4A7C15ull;
-      nd.bg_lo = (uint32_t)bs;
-      nd.bg_hi = (uint32_t)(bs >> 32);
-    }
+    for (size_t k = 0; k < sel.ids.size(); ++k)
+      inputs.push_back(make_uint2(M.pos_of_id[sel.ids[k]], r.grp0 + sel.group[k]));
   }
-  std::vector<uint32_t> snet(I.nq, (uint32_t)id);
   hipStream_t st = sim->stream;
-  // The compact image (4 bytes and a bit per slot, 8 bytes per edge) goes up
-  // to a staging buffer; the placing kernels expand it into the records.
-  const uint64_t n_inh = I.slot_inh.size(), o_jq = (I.nslots + n_inh + 1) & ~1ull;
+  // The image, in network-local indices, goes up to a staging buffer in one
+  // piece (through pinned memory when it is small); the placing kernels expand
+  // and relocate it.
+  std::vector<nc::Segment> seg;  // dev: offset in the staging buffer
+  uint64_t at = 0;
+  auto stage = [&](const void* host, uint64_t bytes) {
+    const uint64_t o = at;
+    if (bytes) seg.push_back(nc::Segment{const_cast<void*>(host), (void*)(uintptr_t)o, bytes});
+    at += (bytes + 15) / 16 * 16;
+    return o / 4;
+  };
+  const bool drive_tables = r.ngrp && !tables_placed;
+  const uint64_t o_w = stage(I.slot_w.data(), I.nslots * 4), o_inh = stage(I.slot_inh.data(), I.slot_inh.size() * 4);
+  const uint64_t o_jq = stage(I.edge_jq.data(), S * sizeof(uint2)), o_row = stage(I.out_row.data(), npos * 8ull);
+  const uint64_t o_deg = stage(I.degw.data(), npos * 4ull), o_nid = stage(I.nid.data(), npos * 4ull);
+  const uint64_t o_soff = stage(I.slice_off.data(), I.nq * 4ull), o_moff = stage(I.slice_moff.data(), I.nq * 4ull);
+  const uint64_t o_idp = stage(M.pos_of_id.data(), net->n * 4ull), o_ptr = stage(M.in_ptr.data(), net->n * 8ull);
+  const uint64_t o_in = stage(inputs.data(), inputs.size() * sizeof(uint2));
+  const uint64_t o_grp = drive_tables ? stage(sim->groups.data() + r.grp0, r.ngrp * sizeof(nc_group)) : 0;
+  const uint64_t o_thr = drive_tables ? stage(sim->thr.data() + r.thr0, r.nthr * 4ull) : 0;
   {
-    nc_status sg = grow(&sim->d_stage, std::max<uint64_t>({o_jq + 2 * S + 2, 3ull * net->n + 4 * S + 4, digest_words(net->n, S)}), st);
+    nc_status sg = grow(&sim->d_stage, std::max<uint64_t>({at / 4, 3ull * net->n + 4 * S + 4, digest_words(net->n, S)}), st);
     if (sg != NC_OK) {
       if (r.has_drive) {
         const nc_group dead{0u, 1u, 0u, sim->max_nets};
@@ -1163,46 +1138,52 @@ extern "C" nc_status nc_sim_add(nc_sim* sim, const nc_net* net, const nc_params*
   }
   uint32_t* const stg = sim->d_stage.p;
   auto blocks = [](uint64_t n) { return dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 4096)); };
-  NC_HIP(hipMemcpyAsync(sim->slice_off + q0, slice_off.data(), I.nq * 4, hipMemcpyHostToDevice, st));
-  NC_HIP(hipMemcpyAsync(sim->slice_moff + q0, slice_moff.data(), I.nq * 4, hipMemcpyHostToDevice, st));
+  if (at <= kPinBytes) {
+    for (const nc::Segment& g : seg) memcpy(sim->h_pin + (uintptr_t)g.dev, g.host, g.bytes);
+    if (at) NC_HIP(hipMemcpyAsync(stg, sim->h_pin, at, hipMemcpyHostToDevice, st));
+  } else {
+    for (nc::Segment& g : seg) g.dev = (unsigned char*)stg + (uintptr_t)g.dev;
+    NC_HIP(nc::upload(sim->device, st, seg.data(), seg.size()));
+  }
+  nc_placing pl{};
+  pl.out_row = (const uint2*)(stg + o_row);
+  pl.degw = stg + o_deg, pl.nid = stg + o_nid;
+  pl.slice_off = stg + o_soff, pl.slice_moff = stg + o_moff;
+  pl.id_pos = stg + o_idp, pl.in_ptr = (const int64_t*)(stg + o_ptr);
+  pl.npos = npos, pl.nq = I.nq, pl.n = net->n, pl.nmwords = I.nmwords;
+  pl.pos0 = pos0, pl.q0 = (uint32_t)q0, pl.slot0 = (uint32_t)sl0, pl.mask0 = (uint32_t)mk0, pl.out0 = (uint32_t)o0;
+  pl.V = sim->V, pl.last_fire = sim->last_fire, pl.firings = sim->firings, pl.d_nid = sim->nid;
+  pl.asum = sim->asum, pl.amask = sim->amask, pl.bcnt = sim->bcnt, pl.pend_cnt = sim->pend_cnt;
+  pl.d_slice_off = sim->slice_off, pl.d_slice_moff = sim->slice_moff;
+  pl.d_id_pos = sim->id_pos, pl.d_id_row = sim->id_row, pl.ndw = sim->ndw, pl.d_out_row = sim->out_row;
+  if (drive_tables) {
+    pl.groups = stg + o_grp, pl.n_groups = r.ngrp * (uint32_t)(sizeof(nc_group) / 4);
+    pl.thr = stg + o_thr, pl.n_thr = r.nthr;
+    pl.d_groups = (uint32_t*)(sim->d_groups.p + r.grp0), pl.d_thr = sim->d_thr.p + r.thr0;
+  }
+  hipLaunchKernelGGL(k_place_net, blocks(std::max<uint64_t>({npos, I.nmwords, pl.n_thr, pl.n_groups, 1})), dim3(256), 0,
+                     st, pl);
+  NC_HIP(hipGetLastError());
+  if (!inputs.empty()) {
+    hipLaunchKernelGGL(k_place_inputs, dim3((uint32_t)((inputs.size() + 255) / 256)), dim3(256), 0, st,
+                       sim->ndw + pos0, (const uint2*)(stg + o_in), (uint32_t)inputs.size());
+    NC_HIP(hipGetLastError());
+  }
   if (I.nslots) {
-    NC_HIP(hipMemcpyAsync(stg, I.slot_w.data(), I.nslots * 4, hipMemcpyHostToDevice, st));
-    NC_HIP(hipMemcpyAsync(stg + I.nslots, I.slot_inh.data(), n_inh * 4, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_place_slots, blocks(I.nslots), dim3(256), 0, st, sim->slots + sl0, (const float*)stg,
-                       (const uint32_t*)(stg + I.nslots), (uint64_t)I.nslots);
+    hipLaunchKernelGGL(k_place_slots, blocks(I.nslots), dim3(256), 0, st, sim->slots + sl0, (const float*)(stg + o_w),
+                       (const uint32_t*)(stg + o_inh), (uint64_t)I.nslots);
     NC_HIP(hipGetLastError());
   }
   if (S) {
-    NC_HIP(hipMemcpyAsync(stg + o_jq, I.edge_jq.data(), S * sizeof(uint2), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_place_edges, blocks(S), dim3(256), 0, st, sim->edges + o0, (const uint2*)(stg + o_jq), S,
                        (uint32_t)sl0, (uint32_t)q0, (const uint32_t*)sim->slice_off);
     NC_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(k_place_neurons, blocks(npos), dim3(256), 0, st, sim->V + pos0, sim->last_fire + pos0,
-                     sim->firings + pos0, (uint64_t)npos);
-  NC_HIP(hipGetLastError());
-  NC_HIP(hipMemsetAsync(sim->amask + mk0, 0, I.nmwords * 4, st));
-  NC_HIP(hipMemsetAsync(sim->asum + pos0, 0, npos * 4, st));
-  NC_HIP(hipMemcpyAsync(sim->ndw + pos0, ndwv.data(), npos * sizeof(uint2), hipMemcpyHostToDevice, st));
-  NC_HIP(hipMemcpyAsync(sim->nid + pos0, I.nid.data(), npos * 4, hipMemcpyHostToDevice, st));
-  // the export maps: weights are read in export order on the device
-  std::vector<uint32_t> idrow(net->n);
-  for (uint32_t i = 0; i < net->n; ++i) idrow[i] = (uint32_t)M.in_ptr[i];
-  if (net->n) {
-    NC_HIP(hipMemcpyAsync(sim->id_pos + pos0, M.pos_of_id.data(), net->n * 4ull, hipMemcpyHostToDevice, st));
-    NC_HIP(hipMemcpyAsync(sim->id_row + pos0, idrow.data(), net->n * 4ull, hipMemcpyHostToDevice, st));
-  }
-  NC_HIP(hipMemcpyAsync(sim->out_row + pos0, orow.data(), npos * sizeof(uint2), hipMemcpyHostToDevice, st));
-  NC_HIP(hipMemsetAsync(sim->pend_cnt + q0, 0, I.nq * sizeof(uint2), st));
-  // no spike of a network that held these slices before may arrive here
-  NC_HIP(hipMemsetAsync(sim->bcnt + (size_t)q0 * NC_NB, 0, (size_t)I.nq * NC_NB * 4, st));
-  NC_HIP(hipMemcpyAsync(sim->slice_net + q0, snet.data(), I.nq * 4, hipMemcpyHostToDevice, st));
-  NC_HIP(hipMemcpyAsync(sim->d_nets + id, &nd, sizeof(nd), hipMemcpyHostToDevice, st));
   NC_HIP(hipStreamSynchronize(st));
   for (uint32_t q = 0; q < I.nq; ++q) {
     sim->slice_net_host[q0 + q] = (uint32_t)id;
-    sim->slice_off_host[q0 + q] = slice_off[q];
-    sim->slice_moff_host[q0 + q] = slice_moff[q];
+    sim->slice_off_host[q0 + q] = (uint32_t)sl0 + I.slice_off[q];
+    sim->slice_moff_host[q0 + q] = (uint32_t)mk0 + I.slice_moff[q];
   }
   r.live = true;
   sim->active_dirty = true;
@@ -1217,8 +1198,6 @@ extern "C" nc_status nc_sim_remove(nc_sim* sim, int32_t net_id) try {
   if (stt != NC_OK) return stt;
   NC_HIP(hipSetDevice(sim->device));
   NC_HIP(hipStreamSynchronize(sim->stream));
-  std::vector<uint32_t> none(r->nq, NC_SLICE_NONE);
-  NC_HIP(hipMemcpy(sim->slice_net + r->q0, none.data(), r->nq * 4, hipMemcpyHostToDevice));
   for (uint32_t q = 0; q < r->nq; ++q) sim->slice_net_host[r->q0 + q] = NC_SLICE_NONE;
   sim->a_slices.release(r->q0, r->nq);
   sim->a_slots.release(r->slot0 / 256, r->nslots / 256);

@@ -347,14 +347,61 @@ __global__ __launch_bounds__(256) void k_place_slots(nc_slot* s, const float* w,
     s[i] = nc_slot{w[i], 0.0f, NC_NEVER, 2 * NC_NEVER + (int32_t)((inh[i >> 5] >> (i & 31)) & 1u)};
 }
 
-// Fresh neuron state: potential at the base level, never fired, no firings.
-__global__ __launch_bounds__(256) void k_place_neurons(float* V, int32_t* last_fire, uint32_t* firings, uint64_t n) {
+// The rest of a network being added, from its staged image in network-local
+// indices: per-neuron rows and fresh state (potential at the base level, never
+// fired, no firings), slice tables, the maps between ids and positions, the
+// drive's groups and thresholds; active masks, their summaries, pending counts
+// and bucket counts cleared (no spike of a network that held these slices
+// before may arrive here).  One launch and one copy: as sixteen copies and
+// fills of their own these took most of the 0.5 ms of adding a small network.
+struct nc_placing {
+  const uint2* out_row;  // staged, per position: out-edges, degree words, ids
+  const uint32_t *degw, *nid;
+  const uint32_t *slice_off, *slice_moff, *id_pos;  // per slice, per neuron id
+  const int64_t* in_ptr;
+  const uint32_t *groups, *thr;
+  uint32_t npos, nq, n, n_groups, n_thr;  // n_groups, n_thr in words
+  uint32_t pos0, q0, slot0, mask0, out0;
+  uint64_t nmwords;
+  float* V;  // the simulation's
+  int32_t* last_fire;
+  uint32_t *firings, *d_nid, *asum, *amask, *d_slice_off, *d_slice_moff, *d_id_pos, *d_id_row, *bcnt, *d_groups, *d_thr;
+  uint2 *ndw, *d_out_row, *pend_cnt;
+};
+__global__ __launch_bounds__(256) void k_place_net(nc_placing a) {
+  static_assert(NC_NB == 64u, "a bucket count per position");
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    V[i] = NC_BASELEVEL;
-    last_fire[i] = NC_NEVER;
-    firings[i] = 0u;
+  const uint64_t t0 = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (uint64_t i = t0; i < a.npos; i += stride) {
+    const uint64_t p = a.pos0 + i;
+    a.V[p] = NC_BASELEVEL;
+    a.last_fire[p] = NC_NEVER;
+    a.firings[p] = 0u;
+    a.asum[p] = 0u;
+    a.bcnt[p] = 0u;
+    a.ndw[p] = make_uint2(a.degw[i], 0u);
+    a.d_nid[p] = a.nid[i];
+    const uint2 o = a.out_row[i];
+    a.d_out_row[p] = make_uint2(a.out0 + o.x, o.y);
   }
+  for (uint64_t i = t0; i < a.nq; i += stride) {
+    a.d_slice_off[a.q0 + i] = a.slot0 + a.slice_off[i];
+    a.d_slice_moff[a.q0 + i] = a.mask0 + a.slice_moff[i];
+    a.pend_cnt[a.q0 + i] = make_uint2(0u, 0u);
+  }
+  for (uint64_t i = t0; i < a.n; i += stride) {
+    a.d_id_pos[a.pos0 + i] = a.id_pos[i];
+    a.d_id_row[a.pos0 + i] = (uint32_t)a.in_ptr[i];
+  }
+  for (uint64_t i = t0; i < a.nmwords; i += stride) a.amask[a.mask0 + i] = 0u;
+  for (uint64_t i = t0; i < a.n_groups; i += stride) a.d_groups[i] = a.groups[i];
+  for (uint64_t i = t0; i < a.n_thr; i += stride) a.d_thr[i] = a.thr[i];
+}
+
+// Input neurons, (local position, group) each.
+__global__ __launch_bounds__(256) void k_place_inputs(uint2* ndw, const uint2* inputs, uint32_t n) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) ndw[inputs[i].x] = make_uint2(ndw[inputs[i].x].x | NC_DEG_INPUT, inputs[i].y);
 }
 
 // Group spike trains of steps c0 .. c0 + gridDim.y - 1 of a call (at most

@@ -5,7 +5,7 @@
 // before and a third of that into fresh ones.  Here each thread moves every
 // so-many-th chunk -- by DMA to or from its own pinned chunk, by memcpy to or
 // from the caller's memory -- so that first touches and copies of several
-// chunks overlap the DMA of others: 23 MB into a warm array 1.4 ms -> 0.82, a
+// chunks overlap the DMA of others: 23 MB into a warm array 1.4 ms -> 0.70, a
 // wired network of 190 MB and its export 29.3 -> 11.6, a checkpoint of 18 MB
 // saved and restored 4.1 -> 2.6.
 #include <hip/hip_runtime.h>
@@ -21,8 +21,10 @@
 namespace nc {
 namespace {
 
-constexpr size_t kChunk = 1u << 20;
-constexpr unsigned kThreads = 8;
+// A chunk costs about 20 us beside its DMA: 23 MB in chunks of 256 KiB 1.7 ms,
+// 512 KiB 1.15, 1 MiB 0.82, 2 MiB 0.70, whatever the threads from four on.
+constexpr size_t kChunk = 2u << 20;
+constexpr unsigned kThreads = 4;
 constexpr size_t kIdleMost = 6;  // pinned buffers kept between calls (a server builds on four threads)
 
 struct PinnedChunks {
