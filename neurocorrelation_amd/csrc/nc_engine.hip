@@ -24,6 +24,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <mutex>
 #include <map>
 #include <numeric>
@@ -507,7 +508,8 @@ struct nc_sim {
   unsigned char* h_pin = nullptr;
   nc_netdesc* h_nds = nullptr;
   uint32_t* h_ev = nullptr;
-  uint32_t* h_words = nullptr;
+  uint32_t* h_words = nullptr;  // (the third: the last read's tag, nc_done)
+  uint32_t read_tag = 0;
   DevBuf<uint32_t> d_thr;
   DevBuf<uint32_t> d_ev_pos;
   DevBuf<uint8_t> d_ev_kind;
@@ -720,20 +722,45 @@ nc_place place_of(const nc_sim* sim, const NetRec& r) {
 
 dim3 row_blocks(const NetRec& r) { return dim3((uint32_t)(((uint64_t)r.n * NC_ROW_LANES + 255) / 256)); }
 
-// `bytes` of results for the caller: `fill` enqueues the kernel that writes
-// them to the address that it is given.  dev: device staging of that size.
+// What a read kernel of `blocks` workgroups signals with, and the wait for it:
+// by the flag when they are few, else by the stream.
+constexpr uint32_t kFlagBlocks = 16;
+nc_done signal_of(nc_sim* sim, uint32_t blocks) {
+  if (blocks == 0 || blocks > kFlagBlocks) return nc_done{nullptr, nullptr, 0u};
+  if (++sim->read_tag == 0u) ++sim->read_tag;
+  return nc_done{sim->d_chunk_off + 208, sim->h_words + 2, sim->read_tag};
+}
+nc_status wait_for(nc_sim* sim, const nc_done& d) {
+  if (d.flag) {
+    // bounded: behind steps still running, or a kernel that failed, the stream
+    // is waited for
+    const auto t0 = std::chrono::steady_clock::now();
+    for (;;) {
+      for (int i = 0; i < 64; ++i)
+        if (__atomic_load_n(d.flag, __ATOMIC_ACQUIRE) == d.tag) return check_barrier(sim);
+      if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(100)) break;
+    }
+  }
+  NC_HIP(hipStreamSynchronize(sim->stream));
+  return check_barrier(sim);
+}
+
+// `bytes` of results for the caller: `fill` enqueues the kernel of `blocks`
+// workgroups that writes them to the address that it is given.  dev: device
+// staging of that size.
 template <class F>
-nc_status deliver(nc_sim* sim, void* out, size_t bytes, void* dev, F fill) {
+nc_status deliver(nc_sim* sim, void* out, size_t bytes, void* dev, uint32_t blocks, F fill) {
   const bool pinned = bytes <= kPinBytes;
-  fill(pinned ? (void*)sim->h_pin : dev);
+  const nc_done d = signal_of(sim, pinned ? blocks : 0u);
+  fill(pinned ? (void*)sim->h_pin : dev, d);
   NC_HIP(hipGetLastError());
   if (!pinned) {
     const nc::Segment g{out, dev, bytes};
     NC_HIP(nc::download(sim->device, sim->stream, &g, 1));
   }
-  NC_HIP(hipStreamSynchronize(sim->stream));
-  if (pinned) memcpy(out, sim->h_pin, bytes);
-  return check_barrier(sim);
+  const nc_status st = wait_for(sim, d);
+  if (st == NC_OK && pinned) memcpy(out, sim->h_pin, bytes);
+  return st;
 }
 
 // The caller's `bytes` at an address that kernels can read.
@@ -752,8 +779,8 @@ nc_status fetch(nc_sim* sim, const void* in, size_t bytes, const void** at) {
 // A network's first n weights in export order; dev: device staging of n floats.
 nc_status export_weights(nc_sim* sim, NetRec& r, float* dev, float* out, uint64_t n) {
   const nc_place N = place_of(sim, r);
-  return deliver(sim, out, 4 * n, dev, [&](void* to) {
-    hipLaunchKernelGGL(k_read_weights, row_blocks(r), dim3(256), 0, sim->stream, N, (float*)to, (uint32_t)n);
+  return deliver(sim, out, 4 * n, dev, row_blocks(r).x, [&](void* to, const nc_done& d) {
+    hipLaunchKernelGGL(k_read_weights, row_blocks(r), dim3(256), 0, sim->stream, N, (float*)to, (uint32_t)n, d);
   });
 }
 
@@ -862,7 +889,8 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
     // word 0: chunk offset; word 32: grid-barrier arrivals of the call;
     // word 128: zero, the group-spike-train word read when there are no
     // groups; word 192: a checkpoint's faults (nc_sim_restore); words
-    // 200-203: a result's digest and firings (sim_result)
+    // 200-203: a result's digest and firings (sim_result); word 208: workgroups
+    // done of a read (nc_done)
     R.want(&sim->d_chunk_off, 256);
     // one more, never written: the (never live) network of hole records
     R.want(&sim->d_nets, sim->max_nets + 1ull);
@@ -884,7 +912,7 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
       sim->h_words = (uint32_t*)(sim->h_pin + kPinBytes);
       sim->h_nds = (nc_netdesc*)(sim->h_pin + kPinBytes + 64);
       sim->h_ev = (uint32_t*)(sim->h_nds + sim->max_nets);
-      sim->h_words[0] = sim->h_words[1] = 0u;
+      sim->h_words[0] = sim->h_words[1] = sim->h_words[2] = 0u;
     }
   }
   if (st == NC_OK) {
@@ -1703,9 +1731,11 @@ nc_status read_pos_array(nc_sim* sim, NetRec& r, const T* dev, T* out, uint32_t 
   if (!out) return fail(NC_ERR_ARG, "null argument");
   if (n > r.n) return fail(NC_ERR_RANGE, "more neurons requested than the network has");
   const nc_place N = place_of(sim, r);
-  return deliver(sim, out, 4ull * n, sim->d_stage.p, [&](void* to) {
-    if (n) hipLaunchKernelGGL(k_read_neurons, dim3((n + 255) / 256), dim3(256), 0, sim->stream, N, (const uint32_t*)dev, n,
-                       (uint32_t*)to);
+  const uint32_t blocks = (n + 255) / 256;
+  return deliver(sim, out, 4ull * n, sim->d_stage.p, blocks, [&](void* to, const nc_done& d) {
+    if (n)
+      hipLaunchKernelGGL(k_read_neurons, dim3(blocks), dim3(256), 0, sim->stream, N, (const uint32_t*)dev, n,
+                         (uint32_t*)to, d);
   });
 }
 }  // namespace
@@ -1898,10 +1928,12 @@ extern "C" nc_status nc_read_synapse_state(nc_sim* sim, int32_t net_id, int32_t*
   const bool pinned = 4 * n * m <= kPinBytes;
   uint32_t* const to = pinned ? (uint32_t*)sim->h_pin : sim->d_stage.p;
   auto at = [&](int i) { return want[i] ? to + of[i] * n : nullptr; };
+  nc_done d{nullptr, nullptr, 0u};
   if (n && m) {
+    d = signal_of(sim, pinned ? row_blocks(*r).x : 0u);
     hipLaunchKernelGGL(k_read_spikes, row_blocks(*r), dim3(256), 0, sim->stream, place_of(sim, *r),
                        (int32_t)r->steps_done, sim->T.r_rel, (int32_t*)at(0), (int32_t*)at(1), (float*)at(2),
-                       (uint32_t)n);
+                       (uint32_t)n, d);
     NC_HIP(hipGetLastError());
     std::vector<nc::Segment> seg;
     if (!pinned)
@@ -1909,11 +1941,11 @@ extern "C" nc_status nc_read_synapse_state(nc_sim* sim, int32_t net_id, int32_t*
         if (want[i]) seg.push_back(nc::Segment{want[i], at(i), 4 * n});
     NC_HIP(nc::download(sim->device, sim->stream, seg.data(), seg.size()));
   }
-  NC_HIP(hipStreamSynchronize(sim->stream));
-  if (pinned && n)
+  st = wait_for(sim, d);
+  if (st == NC_OK && pinned && n)
     for (int i = 0; i < 3; ++i)
       if (want[i]) memcpy(want[i], at(i), 4 * n);
-  return check_barrier(sim);
+  return st;
 }
 NC_ABI_CATCH
 
@@ -2002,7 +2034,7 @@ extern "C" nc_status nc_sim_save(nc_sim* sim, int32_t net_id, void* buf, uint64_
   h.digest = r->maps->digest;
   NC_HIP(hipSetDevice(sim->device));
   const uint64_t state = 12ull * r->n + 16ull * r->S;
-  st = deliver(sim, p + sizeof h, state, sim->d_stage.p, [&](void* to) {
+  st = deliver(sim, p + sizeof h, state, sim->d_stage.p, 0, [&](void* to, const nc_done&) {
     if (r->n)
       hipLaunchKernelGGL(k_pack, row_blocks(*r), dim3(256), 0, sim->stream, place_of(sim, *r), sim->V, sim->last_fire,
                          sim->firings, (int32_t)r->steps_done, (uint32_t*)to);

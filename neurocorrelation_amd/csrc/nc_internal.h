@@ -66,8 +66,12 @@ struct Segment {
 };
 hipError_t download(int device, hipStream_t st, const Segment* seg, size_t n_seg);
 hipError_t upload(int device, hipStream_t st, const Segment* seg, size_t n_seg);
+// A stream for a piece of work of its own: taken, and given back idle (making
+// and destroying one takes 80-100 us).
+hipError_t stream_take(int device, hipStream_t* out);
+void stream_give(int device, hipStream_t st);
 // A simulation came (+1) or went (-1): the last one's end frees the pinned
-// memory kept between copies.
+// memory and the streams kept between calls.
 void xfer_user(int change);
 #endif
 

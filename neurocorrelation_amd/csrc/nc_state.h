@@ -16,6 +16,25 @@
 
 #define NC_ROW_LANES 16u
 
+// Tells the host that a kernel of a few workgroups has written its results to
+// pinned memory, sooner than a stream synchronisation does (a read of 750
+// neurons 12.0 -> 8.2 us with its launch; from about 40 workgroups on the
+// fences cost more than it gains).  count: 0 between kernels; flag == null:
+// nobody waits so.
+struct nc_done {
+  uint32_t *count, *flag, tag;
+};
+__device__ __forceinline__ void nc_tell(const nc_done& d) {
+  if (!d.flag) return;
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  if (atomicAdd(d.count, 1u) + 1u != gridDim.x) return;
+  *d.count = 0u;
+  __threadfence_system();
+  __hip_atomic_store(d.flag, d.tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // A network on the device, for these kernels.
 struct nc_place {
   nc_slot* slots;
@@ -43,17 +62,20 @@ __device__ __forceinline__ bool nc_row_of(const nc_place& N, uint32_t t, nc_row&
 }
 
 // One value per neuron, by id.
-__global__ __launch_bounds__(256) void k_read_neurons(nc_place N, const uint32_t* v, uint32_t n, uint32_t* out) {
+__global__ __launch_bounds__(256) void k_read_neurons(nc_place N, const uint32_t* v, uint32_t n, uint32_t* out,
+                                                      nc_done done) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = v[N.pos0 + N.id_pos[N.pos0 + i]];
+  nc_tell(done);
 }
 
 // The first n_syn synapses' weights.
-__global__ __launch_bounds__(256) void k_read_weights(nc_place N, float* out, uint32_t n_syn) {
+__global__ __launch_bounds__(256) void k_read_weights(nc_place N, float* out, uint32_t n_syn, nc_done done) {
   nc_row r;
-  if (!nc_row_of(N, blockIdx.x * blockDim.x + threadIdx.x, r)) return;
-  for (uint32_t k = r.sub; k < r.deg && r.row + k < n_syn; k += NC_ROW_LANES)
-    out[r.row + k] = N.slots[r.slot(k)].w;
+  if (nc_row_of(N, blockIdx.x * blockDim.x + threadIdx.x, r))
+    for (uint32_t k = r.sub; k < r.deg && r.row + k < n_syn; k += NC_ROW_LANES)
+      out[r.row + k] = N.slots[r.slot(k)].w;
+  nc_tell(done);
 }
 
 // The first n_syn synapses' spike state at step s (a null array is not wanted):
@@ -63,16 +85,17 @@ __global__ __launch_bounds__(256) void k_read_weights(nc_place N, float* out, ui
 // moved to last_arr, or one restored without a latched spike; the latched
 // depolarisation.
 __global__ __launch_bounds__(256) void k_read_spikes(nc_place N, int32_t s, int32_t rel, int32_t* arrival,
-                                                     int32_t* last, float* depol, uint32_t n_syn) {
+                                                     int32_t* last, float* depol, uint32_t n_syn, nc_done done) {
   nc_row r;
-  if (!nc_row_of(N, blockIdx.x * blockDim.x + threadIdx.x, r)) return;
-  for (uint32_t k = r.sub; k < r.deg && r.row + k < n_syn; k += NC_ROW_LANES) {
-    const nc_slot x = N.slots[r.slot(k)];
-    const int32_t a = x.arr_inh >> 1;
-    if (arrival) arrival[r.row + k] = (a != NC_NEVER && s < a + rel) ? a : 0;
-    if (last) last[r.row + k] = (a != NC_NEVER && a <= s) ? a : x.last_arr;
-    if (depol) depol[r.row + k] = x.depol;
-  }
+  if (nc_row_of(N, blockIdx.x * blockDim.x + threadIdx.x, r))
+    for (uint32_t k = r.sub; k < r.deg && r.row + k < n_syn; k += NC_ROW_LANES) {
+      const nc_slot x = N.slots[r.slot(k)];
+      const int32_t a = x.arr_inh >> 1;
+      if (arrival) arrival[r.row + k] = (a != NC_NEVER && s < a + rel) ? a : 0;
+      if (last) last[r.row + k] = (a != NC_NEVER && a <= s) ? a : x.last_arr;
+      if (depol) depol[r.row + k] = x.depol;
+    }
+  nc_tell(done);
 }
 
 // Synapse::setWeight (src/NeuCor.cpp:576-579): the weight and its sign class.

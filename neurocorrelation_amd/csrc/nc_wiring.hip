@@ -428,14 +428,12 @@ extern "C" nc_status nc_net_generate_device(const nc_wiring_spec* spec, int32_t 
   const int ncell = nc_cells_per_axis(s.side, s.radius);
   const uint64_t ncells = (uint64_t)ncell * ncell * ncell;
   hipStream_t st = nullptr;
-  NW_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+  NW_HIP(nc::stream_take(device, &st));
   struct StreamGuard {
+    int device;
     hipStream_t s;
-    ~StreamGuard() {
-      (void)hipStreamSynchronize(s);  // the buffers' frees, queued on it
-      (void)hipStreamDestroy(s);
-    }
-  } sg{st};
+    ~StreamGuard() { nc::stream_give(device, s); }  // waits for the buffers' frees, queued on it
+  } sg{device, st};
   Bufs B{st, {}};
   float *px, *py, *pz, *X, *Y, *Z, *xyz;
   uint32_t *cell_d, *cell, *cmem, *cstart, *cend, *meta;

@@ -40,6 +40,7 @@ struct PinnedChunks {
 
 std::mutex g_mu;
 std::vector<PinnedChunks*> g_idle;
+std::vector<std::pair<int, hipStream_t>> g_streams;  // idle ones, with their device
 unsigned g_users = 0;  // simulations alive
 
 hipError_t take(int device, PinnedChunks** out) {
@@ -152,14 +153,44 @@ hipError_t upload(int device, hipStream_t st, const Segment* seg, size_t n_seg) 
   return move(device, st, seg, n_seg, false);
 }
 
+hipError_t stream_take(int device, hipStream_t* out) {
+  {
+    std::lock_guard<std::mutex> g(g_mu);
+    for (size_t i = 0; i < g_streams.size(); ++i)
+      if (g_streams[i].first == device) {
+        *out = g_streams[i].second;
+        g_streams.erase(g_streams.begin() + i);
+        return hipSuccess;
+      }
+  }
+  return hipStreamCreateWithFlags(out, hipStreamNonBlocking);
+}
+
+void stream_give(int device, hipStream_t st) {
+  (void)hipStreamSynchronize(st);
+  {
+    std::lock_guard<std::mutex> g(g_mu);
+    if (g_streams.size() < kIdleMost) {
+      g_streams.push_back({device, st});
+      return;
+    }
+  }
+  (void)hipStreamDestroy(st);
+}
+
 void xfer_user(int change) {
   std::vector<PinnedChunks*> gone;
+  std::vector<std::pair<int, hipStream_t>> streams;
   {
     std::lock_guard<std::mutex> g(g_mu);
     g_users += (unsigned)change;
-    if (g_users == 0) gone.swap(g_idle);
+    if (g_users == 0) {
+      gone.swap(g_idle);
+      streams.swap(g_streams);
+    }
   }
   for (PinnedChunks* b : gone) delete b;
+  for (auto& s : streams) (void)hipStreamDestroy(s.second);
 }
 
 }  // namespace nc
