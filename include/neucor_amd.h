@@ -198,7 +198,8 @@ nc_status nc_sim_remove(nc_sim* sim, int32_t net_id);
  * the per-call network windows and due host events to buffers sized by
  * nc_sim_create, nc_sim_add and nc_push_forced: it never allocates device
  * memory (under a graph launch shape it captures and instantiates a graph
- * when the shape or the set of networks changed). */
+ * when the shape or the set of networks changed; at the default shape, where
+ * captured chunks pay, from the second call with the same launches on). */
 nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps);
 
 /* Steps each network has completed and has left (0 = finished when it was
@@ -272,7 +273,7 @@ nc_status nc_reset_activities(nc_sim* sim, int32_t net_id);
  * [2] active slot-steps, [3] arrivals, [4] fired neurons,
  * [5] in-degree of fired, [6] out-degree of fired, [7] accepted spikes,
  * [8] pending-list entries scanned (spikes whose delays exceed the
- * arrival ring), [9] mask words of every stepped neuron, ceil(in-degree /
+ * arrival buckets', and those past a bucket's first 64), [9] mask words of every stepped neuron, ceil(in-degree /
  * 32) each, [10] active-mask words
  * written back, [11] fired-list records (per 64-neuron slice with fired
  * neurons, one per share of its out-edges given to a fan-out wave: up to 16,
@@ -344,7 +345,9 @@ nc_status nc_set_counting(nc_sim* sim, int enable);
  * that cannot complete (a grid not wholly resident, as when another
  * simulation's kernels hold part of the device) gives up after 2 s and the
  * next synchronising call fails with NC_ERR_STATE.  Results do not depend
- * on the launch shape.  Default {4, 0, 0, 0, 0, 0}; nc_sim_tune keeps
+ * on the launch shape.  Default {4, 0, 0, 0, 0, 0}, at which
+ * nc_sim_step chooses the form of its kernels by the simulation's size and
+ * the activity last seen; any other shape is used as given.  nc_sim_tune keeps
  * fanout_waves as it finds it. */
 typedef struct nc_launch_cfg {
   uint32_t waves_per_block;

@@ -1553,31 +1553,44 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
         (void)hipGraphExecDestroy(sim->graph);
         sim->graph = nullptr;
       }
-      NC_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-      nc_status cs = NC_OK;
-      for (uint32_t c = 0; c < G && cs == NC_OK; ++c) {
-        a.chunk_i = (int32_t)c;
-        uint32_t* bar_arg = bar;
-        void* args[] = {&a, &bar_arg};
-        if (fn_step ? hipLaunchKernel(fn_step, dim3(pgrid), dim3(64 * wpb), args, lds, st) != hipSuccess
-                    : (hipLaunchKernel(fn_neuron, dim3(n_grid), dim3(n_block), args, lds, st) != hipSuccess ||
-                       hipLaunchKernel(fn_fanout, dim3(fan_grid), dim3(64 * wpb), args, 0, st) != hipSuccess))
-          cs = fail(NC_ERR_HIP, "kernel launch during capture failed");
-      }
-      hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, st, sim->d_chunk_off, G);
-      hipGraph_t g = nullptr;
-      const hipError_t ce = hipStreamEndCapture(st, &g);
-      if (cs != NC_OK) {
-        if (g) (void)hipGraphDestroy(g);
-        return cs;
-      }
-      NC_HIP(ce);
-      const hipError_t ie = hipGraphInstantiate(&sim->graph, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      NC_HIP(ie);
+      auto capture = [&]() -> nc_status {
+        NC_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+        nc_status cs = NC_OK;
+        for (uint32_t c = 0; c < G && cs == NC_OK; ++c) {
+          a.chunk_i = (int32_t)c;
+          uint32_t* bar_arg = bar;
+          void* args[] = {&a, &bar_arg};
+          if (fn_step ? hipLaunchKernel(fn_step, dim3(pgrid), dim3(64 * wpb), args, lds, st) != hipSuccess
+                      : (hipLaunchKernel(fn_neuron, dim3(n_grid), dim3(n_block), args, lds, st) != hipSuccess ||
+                         hipLaunchKernel(fn_fanout, dim3(fan_grid), dim3(64 * wpb), args, 0, st) != hipSuccess))
+            cs = fail(NC_ERR_HIP, "kernel launch during capture failed");
+        }
+        hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, st, sim->d_chunk_off, G);
+        hipGraph_t g = nullptr;
+        const hipError_t ce = hipStreamEndCapture(st, &g);
+        if (cs != NC_OK) {
+          if (g) (void)hipGraphDestroy(g);
+          return cs;
+        }
+        NC_HIP(ce);
+        const hipError_t ie = hipGraphInstantiate(&sim->graph, g, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(g);
+        NC_HIP(ie);
+        return NC_OK;
+      };
+      const nc_status cs = capture();
       a.chunk_i = 0;
-      sim->graph_args = a;
-      memcpy(sim->graph_key, key, sizeof key);
+      if (cs == NC_OK) {
+        sim->graph_args = a;
+        memcpy(sim->graph_key, key, sizeof key);
+      } else if (!own) {
+        return cs;
+      } else {
+        // the call's own idea: its steps are launched one by one instead
+        (void)hipGetLastError();
+        sim->graph = nullptr;
+        G = 0;
+      }
     }
   }
   // The call in sub-chunks of at most NC_GRING steps (whole graph chunks):

@@ -25,6 +25,7 @@ void split_bytes(size_t bytes, F f) {
   const unsigned nt = bytes < kParallelBytes ? 1u : std::min(8u, std::max(1u, std::thread::hardware_concurrency()));
   const size_t part = (bytes / nt + kPage) / kPage * kPage;
   std::vector<std::thread> th;
+  th.reserve(nt);
   size_t at = 0;
   try {
     for (unsigned t = 0; t + 1 < nt && at + part < bytes; ++t, at += part) th.emplace_back(f, at, at + part);

@@ -85,6 +85,8 @@ hipError_t move(int device, hipStream_t st, const Segment* seg, size_t n_seg, bo
   if (chunks.empty()) return hipSuccess;
   size_t total = 0;
   for (const Segment& c : chunks) total += c.bytes;
+  std::vector<std::thread> th;
+  th.reserve(kThreads);
   PinnedChunks* b = nullptr;
   hipError_t e = take(device, &b);
   if (e != hipSuccess) return e;
@@ -130,8 +132,6 @@ hipError_t move(int device, hipStream_t st, const Segment* seg, size_t n_seg, bo
   };
   const unsigned nt = (unsigned)std::min<size_t>(
       {chunks.size(), kThreads, std::max<size_t>(1, std::thread::hardware_concurrency())});
-  std::vector<std::thread> th;
-  th.reserve(nt);
   try {
     for (unsigned t = 1; t < nt; ++t) th.emplace_back(work, t);
   } catch (const std::system_error&) {
