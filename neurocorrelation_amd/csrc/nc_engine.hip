@@ -529,6 +529,7 @@ struct nc_sim {
   uint64_t raster_read = 0;
   bool act_identity = false;  // active record i is slice act_q0 + i
   uint32_t act_q0 = 0;
+  uint32_t net_all = ~0u;  // the only live network, or ~0u
   uint64_t host_neuron_steps = 0, host_synapse_steps = 0, host_mword_steps = 0;
   // Host staging of a call's events; reused only after upload_done.
   std::vector<uint32_t> h_ev_pos;
@@ -578,6 +579,7 @@ nc_step_args base_args(nc_sim* sim) {
   a.n_active_slices = (uint32_t)sim->active_host.size();
   a.act_identity = sim->act_identity ? 1u : 0u;
   a.act_q0 = sim->act_q0;
+  a.net_all = sim->net_all;
   a.nets = sim->d_nets;
   a.groups = sim->d_groups.p;
   a.thr = sim->d_thr.p;
@@ -690,6 +692,7 @@ nc_status rebuild_active(nc_sim* sim) {
     sim->live_nq = std::max(sim->live_nq, r.nq);
     sim->live_mw = std::max(sim->live_mw, r.max_mw);
   }
+  sim->net_all = sim->net_recs_host.size() == 1 ? sim->net_recs_host[0].net : ~0u;
   if (!sim->net_recs_host.empty())
     NC_HIP(hipMemcpy(sim->net_recs, sim->net_recs_host.data(), sim->net_recs_host.size() * sizeof(nc_net_rec),
                      hipMemcpyHostToDevice));
@@ -1472,11 +1475,16 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   const uint32_t lds = a.tabs_in_lds ? (uint32_t)a.len_pre * 4 : 0u;
   const void* fn_neuron = nullptr;
   const void* fn_fanout = nullptr;
+  const bool tabs = a.tabs_in_lds != 0;
+  auto pick = [&](const void* plain, const void* staged, const void* fan) {
+    fn_neuron = tabs ? staged : plain;
+    fn_fanout = fan;
+  };
   switch (wpb) {
-    case 1: fn_neuron = (const void*)k_neuron<1>, fn_fanout = (const void*)k_fanout<1>; break;
-    case 2: fn_neuron = (const void*)k_neuron<2>, fn_fanout = (const void*)k_fanout<2>; break;
-    case 8: fn_neuron = (const void*)k_neuron<8>, fn_fanout = (const void*)k_fanout<8>; break;
-    default: fn_neuron = (const void*)k_neuron<4>, fn_fanout = (const void*)k_fanout<4>; break;
+    case 1: pick((const void*)k_neuron<1, false>, (const void*)k_neuron<1, true>, (const void*)k_fanout<1>); break;
+    case 2: pick((const void*)k_neuron<2, false>, (const void*)k_neuron<2, true>, (const void*)k_fanout<2>); break;
+    case 8: pick((const void*)k_neuron<8, false>, (const void*)k_neuron<8, true>, (const void*)k_fanout<8>); break;
+    default: pick((const void*)k_neuron<4, false>, (const void*)k_neuron<4, true>, (const void*)k_fanout<4>); break;
   }
   // The persistent form: one launch per step of a grid the device holds at
   // once (every workgroup resident, so that the grid barrier can end).

@@ -26,10 +26,12 @@
 //     records past the cache, rows) on a device that k_neuron's one wave per
 //     slice leaves mostly idle, where each of a slice's 16 fired lanes and 6
 //     batches of spikes added its own.  20 000 neurons, a quarter firing:
-//     the neuron phase 50.4 -> 17.9, of which about 4 is the launch.  For many
+//     the neuron phase 50.4 -> 17.0, of which about 4 is the launch.  (With
+//     the owner's masks read beside the entries, the entries' records in
+//     flight over the charge and no barrier before it: 18.2 -> 17.0.)  For many
 //     slices (19 200) it is the traffic of the fired lanes' rows: 301 -> 264.
 //   k_net_steps: quiet networks the barrier and the LDS round trips of one
-//     step (300 neurons: 6.9 -> 2.1); busy ones one compute unit's misses and
+//     step (300 neurons: 6.9 -> 1.9); busy ones one compute unit's misses and
 //     instructions (1000 neurons: 53 -> 23.6, of which the rows' records take
 //     a quarter at about 12 bytes a clock).
 #pragma once
@@ -66,14 +68,17 @@ struct nc_gsh {
   float tpre[RES ? NC_GTAB + 1 : 1], tpost[RES ? NC_GTAB : 1];
 };
 
-// A bucket entry of the step, with the record of its slot where its weight
-// may be stale.
+// A bucket entry of the step, its target's last fire, and its slot's weight
+// (where the entry's may be stale) and sign class.
 struct nc_gent {
   uint2 be;
   float w;
   uint32_t inh;
-  bool on;
+  int32_t lf;
+  bool on, stale;
 };
+// Step of the fire behind an entry taken up at step s.
+__device__ __forceinline__ int32_t nc_gent_fire(uint32_t x, int32_t s) { return s - (int32_t)(((x >> 24) & 63u) + 1u); }
 
 __device__ __forceinline__ void nc_gent_slot(uint32_t rel, uint32_t& tl, uint32_t& k) {
   tl = (rel & (64u * NC_CHUNK - 1u)) >> NC_CHUNK_LOG;
@@ -109,17 +114,21 @@ struct nc_glane {
 };
 
 // The step s (step ci of the call) of the group's nsl slices.  gword: the
-// owner lane's group-spike-train word; f_in, f_bg: its host-scheduled fires.
+// owner lane's group-spike-train word; f_in, f_bg: its host-scheduled fires;
+// rec_i, soff0, b_n0: the slice's place among the active ones, its first slot
+// and its bucket's count (not resident).
 template <int NSL, int W, bool RES>
 __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL, W, RES>& sh, const nc_netdesc& nd,
                                               uint32_t nsl, uint32_t q0, uint32_t wv, uint32_t lane, int32_t s,
                                               int32_t ci, nc_glane& L, uint32_t sm, uint32_t* mrow,
                                               uint32_t pend_n, uint32_t gword, bool f_in, bool f_bg,
-                                              const float* tpre, const float* tpost, uint32_t rec_i) {
+                                              const float* tpre, const float* tpost, uint32_t rec_i, uint32_t soff0,
+                                              uint32_t b_n0) {
   const uint32_t par = (uint32_t)ci & 1u, ph = (uint32_t)ci % 3u;
   const bool owner = wv < nsl;
-  // the waves of slice xs: xs, xs + nsl, ...
-  const uint32_t xs = wv % nsl, sub = wv / nsl, nsub = (W - 1u - xs) / nsl + 1u;
+  // the waves of slice xs: xs, xs + nsl, ...; the owner takes the last share of
+  // its entries, as it has the charge to sum
+  const uint32_t xs = wv % nsl, nsub = (W - 1u - xs) / nsl + 1u, sub = wv < nsl ? nsub - 1u : wv / nsl - 1u;
   const uint32_t xq = q0 + xs;
   const size_t bi = (size_t)xq * NC_NB + ((uint32_t)s & (NC_NB - 1u));
   uint32_t* const pl = (((uint32_t)s >> NC_PEND_LOG_W) & 1u) ? a.pend1 : a.pend0;
@@ -131,34 +140,50 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
   // it) is read now, beside the owners' charge: what may still change it in
   // this step is the post-side STDP of a target that fires now, whose trace
   // is 0 and which does not use it.
-  uint32_t b_n;
+  uint32_t b_n = b_n0;
   if constexpr (RES) b_n = sh.bcnt[xs][(uint32_t)s & (NC_NB - 1u)];
-  else b_n = a.bcnt[bi];
   const uint32_t b_take = min(b_n, NC_BCAP);
-  auto entry = [&](uint32_t i) {
+  // (No branch around the reads: an entry whose record is not needed reads its
+  // own place again.  They are first used after the fire.)
+  auto place = [&](uint32_t i) { return a.bent + (bi * NC_BCAP + min(i, NC_BCAP - 1u)); };
+  auto entry_of = [&](uint32_t i, uint2 be) {
     nc_gent g;
+    const uint2* const own = place(i);
     g.on = i < b_take;
-    g.be = a.bent[bi * NC_BCAP + min(i, NC_BCAP - 1u)];
+    g.be = be;
     uint32_t tl, k;
     nc_gent_slot(g.be.x & 0xFFFFFFu, tl, k);
-    const int32_t sf = s - (int32_t)(((g.be.x >> 24) & 63u) + 1u);
-    int32_t lf;
-    if constexpr (RES) lf = sh.lfo[xs][tl];
-    else if constexpr (W == 1) lf = __shfl(lf0, (int)tl);
-    else lf = a.last_fire[xq * 64u + tl];
-    g.w = __uint_as_float(g.be.y);
+    const int32_t sf = nc_gent_fire(g.be.x, s);
+    if constexpr (RES) g.lf = sh.lfo[xs][tl];
+    else if constexpr (W == 1) g.lf = __shfl(lf0, (int)tl);
+    else g.lf = a.last_fire[xq * 64u + tl];
+    // (with several waves, beside the last fire that says whether it is needed)
+    constexpr bool late = !RES && W > 1;
+    if constexpr (!late) g.stale = g.on && (g.lf > sf || sf < nd.whost);
+    const bool rd = late ? g.on : g.stale;
+    const nc_slot* const r = a.slots + nc_slot_of(RES ? sh.soff[xs] : soff0, tl, k);
+    g.w = *(rd ? &r->w : reinterpret_cast<const float*>(&own->y));
     g.inh = g.be.x >> 31;
-    if (g.on && (lf > sf || sf < nd.whost)) {
-      const nc_slot r = a.slots[nc_slot_of(sh.soff[xs], tl, k)];
-      g.w = r.w;
-      g.inh = (uint32_t)r.arr_inh & 1u;
-    }
+    if (g.on && sf < nd.whost) g.inh = (uint32_t)r->arr_inh & 1u;  // a host write may have changed it
     return g;
   };
+  auto entry = [&](uint32_t i) { return entry_of(i, *place(i)); };
+  constexpr bool kOne = !RES && W <= 2;  // every wave has a share of the bucket
+  uint2 be0 = make_uint2(0u, 0u);
+  if constexpr (kOne) be0 = *place(sub * 64u + lane);
+  // The owner's mask words, read beside the entries.
+  uint32_t mx[RES ? 1 : NC_GW];
+  if constexpr (!RES) {
+    if (owner) {
+#pragma unroll
+      for (uint32_t w = 0; w < NC_GW; ++w) mx[w] = ((sm >> w) & 1u) ? mrow[w * 64] : 0u;
+    }
+  }
   nc_gent g0;
   g0.on = false;
   // resident counts are at hand; else the entries are read beside the count
-  if (sub * 64u < (RES ? b_take : NC_BCAP)) g0 = entry(sub * 64u + lane);
+  if constexpr (kOne) g0 = entry_of(sub * 64u + lane, be0);
+  else if (sub * 64u < (RES ? b_take : NC_BCAP)) g0 = entry(sub * 64u + lane);
 
   static_assert(NC_BCAP == 128u, "at most two entries per lane of one wave");
   nc_gent g1;
@@ -171,7 +196,7 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
   uint32_t nk[NC_ACACHE] = {0u, 0u, 0u}, nv[NC_ACACHE] = {0u, 0u, 0u}, ncnt = 0, smk = 0, dirty = 0;
   bool cache_dirty = false, fire = false;
   if (owner) {
-    const uint32_t soff = sh.soff[wv];
+    const uint32_t soff = RES ? sh.soff[wv] : soff0;
     const uint2 ac[NC_ACACHE] = {make_uint2(L.cache.x, (uint32_t)s - (((uint32_t)s - L.cache.w) & 255u)),
                                  make_uint2(L.cache.y, (uint32_t)s - (((uint32_t)s - (L.cache.w >> 8)) & 255u)),
                                  make_uint2(L.cache.z, (uint32_t)s - (((uint32_t)s - (L.cache.w >> 16)) & 255u))};
@@ -179,13 +204,8 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
     int32_t lf = L.lf;
     uint32_t idx = 0;
     if constexpr (!RES) {
-      for (uint32_t w0 = 0; w0 < ((L.nmw + 1u) & ~1u); w0 += 4) {
-        uint32_t x[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) x[u] = ((sm >> (w0 + u)) & 1u) ? mrow[(w0 + u) * 64] : 0u;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) sh.keepw[wv][w0 + u][lane] = x[u];
-      }
+      for (uint32_t w = 0; w < NC_GW; ++w) sh.keepw[wv][w][lane] = mx[w];
     }
     for (uint32_t w0 = 0; w0 < L.nmw; w0 += 2) {
       const uint32_t mw[2] = {sh.keepw[wv][w0][lane], sh.keepw[wv][w0 + 1][lane]};  // zero past the lane's words
@@ -399,8 +419,10 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
       if (g.on) {
         uint32_t tl, k;
         nc_gent_slot(g.be.x & 0xFFFFFFu, tl, k);
-        nc_gtake<NSL, W, RES>(a, sh, xs, tl, k, g.w, g.inh, __float_as_uint(a.depol_k * __uint_as_float(g.be.y)), pre_f,
-                           post_f, lr);
+        const int32_t sf = nc_gent_fire(g.be.x, s);
+        const bool stale = (!RES && W > 1) ? g.lf > sf || sf < nd.whost : g.stale;
+        nc_gtake<NSL, W, RES>(a, sh, xs, tl, k, stale ? g.w : __uint_as_float(g.be.y),
+                              g.inh, __float_as_uint(a.depol_k * __uint_as_float(g.be.y)), pre_f, post_f, lr);
       }
     }
     if (owner && pend_n) {
@@ -543,16 +565,13 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
 
 // The neuron phase of one step, a workgroup of W waves per active slice.
 template <int W>
-__global__ __launch_bounds__(64 * W) void k_neuron_wide(nc_step_args a) {
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6))) void k_neuron_wide(nc_step_args a) {
   __shared__ nc_gsh<1, W, false> sh;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t i = blockIdx.x;
-  const int32_t ci = (int32_t)*a.chunk_off + a.chunk_i;
+  const uint32_t i = blockIdx.x + nc_have_neuron_args(a);
   const nc_slice_rec rec = a.active_slices[i];
-  const uint32_t q = a.act_identity ? a.act_q0 + i : rec.q;
-  const uint32_t par = (uint32_t)ci & 1u;
-  if (i == 0 && threadIdx.x < NC_FLISTS) a.fired_cnt[((par ^ 1u) * NC_FLISTS + threadIdx.x) * NC_FCNT_STRIDE] = 0u;
+  const uint32_t q = nc_slice_of(a, rec, i);
   nc_glane L;
   L.pos = q * 64u + lane;
   uint32_t sm = 0;
@@ -566,9 +585,14 @@ __global__ __launch_bounds__(64 * W) void k_neuron_wide(nc_step_args a) {
     sm = a.asum[L.pos];
     pc = a.pend_cnt[q];
   }
-  const nc_netdesc nd = a.nets[rec.net];
-  if (ci >= nd.remaining) return;  // the whole workgroup: one network
+  const nc_netdesc nd = a.nets[nc_net_of(a, rec)];
+  const int32_t ci = (int32_t)*a.chunk_off + a.chunk_i;
+  const uint32_t par = (uint32_t)ci & 1u;
   const int32_t s = nd.base_step + ci + 1;
+  const uint32_t b_n = a.bcnt[(size_t)q * NC_NB + ((uint32_t)s & (NC_NB - 1u))];
+  // (after the uniform reads: a store before them would make them vector reads)
+  if (i == 0 && threadIdx.x < NC_FLISTS) a.fired_cnt[((par ^ 1u) * NC_FLISTS + threadIdx.x) * NC_FCNT_STRIDE] = 0u;
+  if (ci >= nd.remaining) return;  // the whole workgroup: one network
   uint32_t gword = 0;
   bool f_in = false, f_bg = false;
   L.fires = 0;
@@ -592,10 +616,11 @@ __global__ __launch_bounds__(64 * W) void k_neuron_wide(nc_step_args a) {
     for (int i = 0; i < 3; ++i) sh.nrow[i] = sh.any[i] = 0u;
     sh.soff[0] = rec.slot_off;
   }
-  __syncthreads();
+  // No barrier: before the step's first one, only wave 0 reads these (the
+  // other waves have rec.slot_off itself).
   const uint32_t pend_n = (((uint32_t)s >> NC_PEND_LOG_W) & 1u) ? pc.y : pc.x;
   nc_group_step<1, W, false>(a, sh, nd, 1u, q, wv, lane, s, ci, L, sm, a.amask + rec.mask_off + lane, pend_n, gword,
-                             f_in, f_bg, a.t_pre, a.t_post, i);
+                             f_in, f_bg, a.t_pre, a.t_post, i, rec.slot_off, b_n);
   if (wv == 0 && (L.nw.x & NC_DEG_VALID)) {
     if (__float_as_uint(L.V) != __float_as_uint(L.V_in)) a.V[L.pos] = L.V;
     if (L.fires) {
@@ -686,7 +711,7 @@ __global__ __launch_bounds__(64 * W) void k_net_steps(nc_step_args a, const nc_n
     }
     const uint32_t pend_n = owner ? sh.pcnt[wv][((uint32_t)s >> NC_PEND_LOG_W) & 1u] : 0u;
     nc_group_step<NSL, W, true>(a, sh, nd, nsl, q0, wv, lane, s, (int32_t)c, L, 0u, mrow, pend_n, gword, f_in, f_bg,
-                                sh.tpre, sh.tpost, 0u);
+                                sh.tpre, sh.tpost, 0u, 0u, 0u);
   }
   __syncthreads();
   if (threadIdx.x == 0) nc_report(a, sh.nrow[(end - 1u) % 3u] >= NC_BUSY_LANES * nsl);

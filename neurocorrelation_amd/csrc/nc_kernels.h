@@ -146,6 +146,7 @@ struct nc_step_args {
   uint32_t n_active_slices;
   uint32_t act_identity;  // active record i is slice act_q0 + i (one contiguous run)
   uint32_t act_q0;
+  uint32_t net_all;  // the network of every active slice, or ~0u: of several
   const nc_netdesc* nets;
   const nc_group* groups;
   const uint32_t* thr;
@@ -285,9 +286,42 @@ __device__ __forceinline__ void nc_count32(unsigned long long* ctr, uint32_t row
 // its spatially close fan-out targets in one L2.
 __device__ __forceinline__ uint32_t nc_block_id(uint32_t swizzle) {
   const uint32_t b = blockIdx.x;
-  if (!swizzle) return b;
   const uint32_t nb = gridDim.x, q = nb >> 3, r = nb & 7u, x = b & 7u, i = b >> 3;
-  return x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
+  return swizzle ? x * q + min(x, r) + i : b;
+}
+
+// An active slice and its network, without waiting for the slice's record
+// where the arguments give them (the asm keeps each branch a branch, as a
+// select would wait, and its result out of the register that the record's read
+// fills).
+__device__ __forceinline__ uint32_t nc_slice_of(const nc_step_args& a, const nc_slice_rec& rec, uint32_t i) {
+  uint32_t q = a.act_q0 + i;
+  if (!a.act_identity)
+    asm("s_mov_b32 %0, %1" : "=&s"(q) : "s"(__builtin_amdgcn_readfirstlane(rec.q)));
+  return q;
+}
+__device__ __forceinline__ uint32_t nc_net_of(const nc_step_args& a, const nc_slice_rec& rec) {
+  uint32_t net = a.net_all;
+  if (net == ~0u)
+    asm("s_mov_b32 %0, %1" : "=&s"(net) : "s"(__builtin_amdgcn_readfirstlane(rec.net)));
+  return net;
+}
+
+// The arguments that a neuron kernel's first reads take, in registers at once:
+// left to itself the compiler reads each where it is first used, and the
+// branches in between make that one round of reads after the other.  (With
+// the slice and network known early and k_fanout's first record read beside
+// its count, us per step: 20 000 quiet neurons 9.5 -> 8.7, 60 000 11.1 -> 10.3,
+// plain-1m 84.4 -> 82.2.)  Returns
+// zero, which what follows has to depend on (a volatile asm would count as a
+// store, and turn the uniform reads after it into vector reads).
+__device__ __forceinline__ uint32_t nc_have_neuron_args(const nc_step_args& a) {
+  uint32_t zero = 0u;
+  asm("" : "+s"(zero) : "s"(a.n_active_slices), "s"(a.act_identity), "s"(a.act_q0), "s"(a.net_all), "s"(a.active_slices),
+               "s"(a.nets), "s"(a.chunk_off), "s"(a.chunk_i), "s"(a.xcd_swizzle), "s"(a.ndw), "s"(a.V),
+               "s"(a.last_fire), "s"(a.pend_cnt), "s"(a.asum), "s"(a.acache), "s"(a.nid), "s"(a.bcnt), "s"(a.bent),
+               "s"(a.gfire), "s"(a.gwords), "s"(a.t_post), "s"(a.len_post));
+  return zero;
 }
 
 // Advances the device-side chunk offset by the chunk's step count (the last
@@ -449,9 +483,7 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
   const bool wave_in = wave < a.n_active_slices;
   const uint32_t widx = wave_in ? wave : 0u;
   const nc_slice_rec rec = a.active_slices[widx];
-  // With one contiguous run of slices the per-neuron loads need not wait
-  // for the slice record.
-  const uint32_t q = a.act_identity ? a.act_q0 + widx : rec.q;
+  const uint32_t q = nc_slice_of(a, rec, widx);
   const uint32_t pos = q * 64 + lane;
   uint2 nw = a.ndw[pos];
   float V = a.V[pos];
@@ -470,7 +502,7 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
   // the others; gfire points at a zero word when there are no groups).
   const uint4 cache = a.acache[pos];
   const uint32_t my_nid = a.nid[pos];
-  const nc_netdesc nd = a.nets[rec.net];
+  const nc_netdesc nd = a.nets[nc_net_of(a, rec)];
   const bool live = wave_in && ci < nd.remaining;
   const int32_t s = nd.base_step + ci + 1;
   const size_t bi = (size_t)q * NC_NB + ((uint32_t)s & (NC_NB - 1u));
@@ -696,7 +728,7 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
       f_tag = tag | ((n_frec - 1u) << 28);
       f_n = n_frec;
       f_b = b;
-      if (a.ctr) atomicAdd(&a.ctr[(size_t)blk * NC_NCTR + 11], (unsigned long long)n_frec);
+      if (a.ctr) atomicAdd(&a.ctr[(size_t)(blk % a.ctr_rows) * NC_NCTR + 11], (unsigned long long)n_frec);
     }
   }
   if (fm) {
@@ -755,7 +787,8 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
         n_pw += (uint32_t)__builtin_popcountll(__ballot(ch0)) + (uint32_t)__builtin_popcountll(__ballot(ch1));
       }
     }
-    if (a.ctr && lane == 0 && n_pw) atomicAdd(&a.ctr[(size_t)blk * NC_NCTR + 18], (unsigned long long)n_pw);
+    if (a.ctr && lane == 0 && n_pw)
+      atomicAdd(&a.ctr[(size_t)(blk % a.ctr_rows) * NC_NCTR + 18], (unsigned long long)n_pw);
     // the arrivals below read records the row passes may have written
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -905,6 +938,7 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
     }
   }
   if (a.ctr) {
+    blk %= a.ctr_rows;
     nc_count32(a.ctr, blk, 2, n_active);
     nc_count32(a.ctr, blk, 3, n_arr);
     if (lane == 0 && fm) {
@@ -936,12 +970,12 @@ __device__ __forceinline__ const float* nc_trace_tables(const nc_step_args& a) {
 
 // The neuron phase of one step for every active slice, one wave per slice,
 // WPB waves per workgroup.
-template <int WPB>
+template <int WPB, bool TABS>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) void k_neuron(nc_step_args a) {
-  const uint32_t blk = nc_block_id(a.xcd_swizzle);
+  const uint32_t blk = nc_block_id(a.xcd_swizzle + nc_have_neuron_args(a));
   const uint32_t wave = __builtin_amdgcn_readfirstlane(blk * WPB + (threadIdx.x >> 6));
-  const float* tpre = nc_trace_tables<WPB>(a);
-  nc_neuron_slice<WPB>(a, blk % a.ctr_rows, wave, (int32_t)*a.chunk_off + a.chunk_i, tpre);
+  const float* tpre = TABS ? nc_trace_tables<WPB>(a) : a.t_pre;
+  nc_neuron_slice<WPB>(a, blk, wave, (int32_t)*a.chunk_off + a.chunk_i, tpre);
 }
 
 // Synapse::fire (src/NeuCor.cpp:727-738) on every outgoing synapse of every
@@ -996,16 +1030,22 @@ __device__ __forceinline__ void nc_fanout_wave(const nc_step_args& a, uint32_t b
                                                uint32_t per, int32_t ci) {
   const uint32_t lane = threadIdx.x & 63;
   uint32_t n_acc = 0, n_out = 0;
-  const uint32_t nf = first < per ? __builtin_amdgcn_readfirstlane(
-                                        a.fired_cnt[((((uint32_t)ci & 1u) * NC_FLISTS) + lst) * NC_FCNT_STRIDE])
-                                  : 0u;
+  // The list's lengths of both parities and the wave's first record, read
+  // beside the step's number (the record before its list is known to reach
+  // that far: a place of the list all the same).
+  const uint32_t n0 = a.fired_cnt[lst * NC_FCNT_STRIDE], n1 = a.fired_cnt[(NC_FLISTS + lst) * NC_FCNT_STRIDE];
   const uint4* const flist = a.fired + lst * a.fcap;
+  uint4 fl = make_uint4(0u, 0u, 0u, 0u);
+  if (lane == 0 && first < a.fcap) fl = flist[first];
+  uint32_t nf = __builtin_amdgcn_readfirstlane(((uint32_t)ci & 1u) ? n1 : n0);
+  nf = first < per ? nf : 0u;
   // busy: two records per slice, or (unsplit: one per slice) most slices fired
   if (a.call_tag && first == 0u && lane == 0)
     nc_report(a, nf * (NC_FLISTS / 2u) >= a.n_active_slices * (a.fsplit_od ? 1.0f : 0.375f));
   for (uint32_t fb = first; fb < nf; fb += 64 * per) {
     const uint32_t fi = fb + lane * per;
-    const uint4 fl = fi < nf ? flist[fi] : make_uint4(0u, 0u, 0u, 0u);
+    if (fi >= nf) fl = make_uint4(0u, 0u, 0u, 0u);
+    else if (fi != first) fl = flist[fi];
     unsigned long long has = __ballot((fl.x | fl.y) != 0u);
     while (has) {
       const uint32_t fsrc = (uint32_t)__builtin_ctzll(has);
@@ -1064,6 +1104,7 @@ __device__ __forceinline__ void nc_fanout_wave(const nc_step_args& a, uint32_t b
     }
   }
   if (a.ctr) {
+    blk %= a.ctr_rows;
     if (lane == 0 && n_out) atomicAdd(&a.ctr[(size_t)blk * NC_NCTR + 6], (unsigned long long)n_out);
     nc_count32(a.ctr, blk, 7, n_acc);
   }
@@ -1073,13 +1114,18 @@ __device__ __forceinline__ void nc_fanout_wave(const nc_step_args& a, uint32_t b
 // fired-slice records.
 template <int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_fanout(nc_step_args a) {
-  const uint32_t blk = nc_block_id(a.xcd_swizzle);
+  // the arguments in one round of reads, as in nc_have_neuron_args
+  uint32_t zero = 0u;
+  asm("" : "+s"(zero) : "s"(a.chunk_off), "s"(a.chunk_i), "s"(a.xcd_swizzle), "s"(a.xcd_lists), "s"(a.fired),
+               "s"(a.fired_cnt), "s"(a.fcap), "s"(a.call_tag), "s"(a.n_active_slices), "s"(a.edges), "s"(a.out_row),
+               "s"(a.slots), "s"(a.bcnt), "s"(a.bent), "s"(a.r_rel), "s"(a.depol_k), "s"(a.ctr));
+  const uint32_t blk = nc_block_id(a.xcd_swizzle) + zero;
   const uint32_t per = gridDim.x * WPB / NC_FLISTS;
   uint32_t lst, first;
   if (a.xcd_lists) {
     // the lists of this workgroup's XCD (the grid holds the same number of
     // waves on every XCD, a multiple of 8)
-    const uint32_t wx = (blockIdx.x >> 3) * WPB + (threadIdx.x >> 6);
+    const uint32_t wx = (blockIdx.x >> 3) * WPB + (threadIdx.x >> 6) + zero;
     lst = (blockIdx.x & 7u) * 8u + (wx & 7u);
     first = wx >> 3;
   } else {
@@ -1087,7 +1133,7 @@ __global__ __launch_bounds__(64 * WPB) void k_fanout(nc_step_args a) {
     lst = wave % NC_FLISTS;
     first = wave / NC_FLISTS;
   }
-  nc_fanout_wave(a, blk % a.ctr_rows, lst, first, per, (int32_t)*a.chunk_off + a.chunk_i);
+  nc_fanout_wave(a, blk, lst, first, per, (int32_t)*a.chunk_off + a.chunk_i);
 }
 
 // Grid-wide barrier of the persistent step kernel: each workgroup adds one
@@ -1125,7 +1171,7 @@ __device__ __forceinline__ void nc_grid_barrier(uint32_t* bar, uint32_t target, 
 // arrivals in this call (zeroed at its start).
 template <int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_step(nc_step_args a, uint32_t* bar) {
-  const uint32_t blk = blockIdx.x % a.ctr_rows;
+  const uint32_t blk = blockIdx.x;
   const uint32_t nwaves = gridDim.x * WPB;
   const uint32_t w0 = __builtin_amdgcn_readfirstlane(blockIdx.x * WPB + (threadIdx.x >> 6));
   const int32_t ci = (int32_t)*a.chunk_off + a.chunk_i;

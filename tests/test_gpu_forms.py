@@ -161,3 +161,39 @@ def test_own_graphs_from_the_second_equal_call():
         m = 20 if i == 3 else 0
         return np.arange(m) % 30 + 1, np.arange(m), np.zeros(m)
     _both(net, _drive(3000, seed=6, bg=0.003), 1.0, [40, 40, 33, 40, 17, 40, 1100, 5, 40], events=events)
+
+
+# where the networks lie: one alone past the first slice, two in one run of
+# slices, two with a hole between them that the active list covers (small) or
+# leaves out (large); weights written with spikes in flight change sign class
+@pytest.mark.parametrize("keep,hole", [((2,), 300), ((1, 2), 300), ((0, 2), 100), ((0, 2), 9000)])
+@pytest.mark.parametrize("n,k", [(1500, 30), (24_000, 25)])
+def test_where_networks_lie(keep, hole, n, k):
+    nets = [_net(n, k, seed=1), _net(hole, 10, seed=2), _net(n + 65, k, seed=3)]
+
+    def run(sim, ids):
+        out = []
+        for c in range(3):
+            sim.step(25)
+            for j, i in ids.items():
+                w = sim.weights(i, nets[j].n_syn)
+                out += [w, sim.potential(i, nets[j].n), sim.firings(i, nets[j].n)]
+                if c == 1:
+                    sim.write_weights(i, np.where(np.arange(w.size) % 3 == 0, -w, w))
+        return out + [x for j, i in ids.items() for x in _state(sim, i, nets[j])]
+
+    sim = nc.Simulation(sum(m.n + 64 for m in nets), sum(m.n_syn for m in nets), 4)
+    ids = [sim.add(m, None, _drive(m.n, j)) for j, m in enumerate(nets)]
+    for j in range(3):
+        if j not in keep:
+            sim.remove(ids[j])
+    got = run(sim, {j: ids[j] for j in keep})
+    sim.close()
+    want = {}
+    for j in keep:
+        sim = nc.Simulation.for_network(nets[j])
+        sim.set_launch(**PER_SLICE)
+        want[j] = run(sim, {j: sim.add(nets[j], None, _drive(nets[j].n, j))})
+        sim.close()
+    calls = [x for c in range(3) for j in keep for x in want[j][3 * c:3 * c + 3]]  # three arrays a call
+    _same(got, calls + [x for j in keep for x in want[j][9:]])
