@@ -38,7 +38,9 @@
 #include "nc_kernels.h"
 
 #define NC_GW 8       // active-mask words per lane: in-degrees up to 256
-#define NC_GARR 4     // arrivals of a lane and step kept for the next cache (more: read back from the records)
+// arrivals of a lane and step kept for the next cache (more: read back from the records)
+// (eight where waves wait for one another and the LDS holds them)
+#define NC_GARR(w, res) ((res) || (w) == 1 ? 4 : 8)
 #define NC_GREC 6     // slot records past the cache an owner lane reads together
 #define NC_GTAB 2048  // trace-table entries k_net_steps stages in LDS, per table
 
@@ -52,9 +54,9 @@ struct nc_gsh {
   uint32_t keepw[NSL][NC_GW][64];  // active-mask words
   uint32_t dirty[NSL][64];         // words that differ from memory's
   float trt[NSL][64];              // target trace at the step (0: none)
-  int32_t lfo[RES ? NSL : 1][64];  // last fire before the step
+  int32_t lfo[RES ? NSL : 1][RES ? 64 : 1];  // last fire before the step
   uint32_t narr[NSL][64];          // arrivals of the step
-  uint2 arr[NSL][64][NC_GARR];     // the first of them: {in-slot, depolarisation}
+  uint2 arr[NSL][64][NC_GARR(W, RES)];  // the first of them: {in-slot, depolarisation}
   uint32_t nrow[3];                // fired lanes, by the step modulo 3 (see below)
   uint32_t row[NSL * 64];          // fired lanes: slice << 6 | lane
   uint32_t rdeg[NSL * 64];         // their in-degrees
@@ -62,9 +64,9 @@ struct nc_gsh {
   uint32_t soff[NSL];              // first slot of each slice
   unsigned long long fm;           // (one slice) its fired lanes
   uint2 rout[RES ? NSL * 64 : 1];  // fired lanes' out-rows
-  uint32_t bcnt[RES ? NSL : 1][NC_NB];
+  uint32_t bcnt[RES ? NSL : 1][RES ? NC_NB : 1];
   uint32_t pcnt[RES ? NSL : 1][2];
-  uint32_t que[RES ? W : 1][320];  // per wave: edges to fire (at most 63 left over and 4 * 64 new)
+  uint32_t que[RES ? W : 1][RES ? 320 : 1];  // per wave: edges to fire (at most 63 left over and 4 * 64 new)
   float tpre[RES ? NC_GTAB + 1 : 1], tpost[RES ? NC_GTAB : 1];
 };
 
@@ -99,7 +101,7 @@ __device__ __forceinline__ void nc_gtake(const nc_step_args& a, nc_gsh<NSL, W, R
   atomicOr(&sh.keepw[sl][k >> 5][tl], 1u << (k & 31u));
   if (!RES) atomicOr(&sh.dirty[sl][tl], 1u << (k >> 5));
   const uint32_t at = atomicAdd(&sh.narr[sl][tl], 1u);
-  if (at < NC_GARR) sh.arr[sl][tl][at] = make_uint2(k, depol);
+  if (at < NC_GARR(W, RES)) sh.arr[sl][tl][at] = make_uint2(k, depol);
 }
 
 // What an owner lane keeps of its neuron.
@@ -350,21 +352,25 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
   }
 
   // Post-side STDP (Neuron::fire's inSynapses loop): two rows per wave, 128
-  // slots of each in a round; or, when more lanes fired, 16 lanes per row,
-  // eight rows per wave, 32 slots of each in a round.
+  // slots of each in a round; or, when more lanes fired, 16 lanes per row:
+  // four rows per wave, 64 slots of each in a round, while that covers the
+  // rows, else eight rows per wave, 32 slots of each.
   const uint32_t lpr = nr <= 2u * W ? 6u : 4u, per = 64u >> lpr;
+  const bool deep = W > 1 && lpr == 4u && nr <= 4u * W;
   if (nr) {
     const uint32_t step = 64u << lpr;  // slots between in-slots k and k + (1 << lpr) of a lane
+    const uint32_t pass = deep ? 4u : 2u;  // slots of a row a lane takes in a round
     for (uint32_t r0 = wv; r0 < nr; r0 += 2u * W * per) {
-      uint32_t j0[2], dg[2];  // the lane's first slot of each row
+      uint32_t j0[2], dg[2], kb[2];  // the lane's first slot of each row (deep: its first and third of one)
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        const uint32_t r = r0 + W * (per * u + (lane >> lpr)), rr = min(r, nr - 1u), code = sh.row[rr];
-        j0[u] = nc_slot_of(sh.soff[code >> 6], code & 63u, lane & ((1u << lpr) - 1u));
+        const uint32_t r = r0 + W * ((deep ? 0u : per * u) + (lane >> lpr)), rr = min(r, nr - 1u), code = sh.row[rr];
+        kb[u] = deep ? 2u * u << lpr : 0u;
+        j0[u] = nc_slot_of(sh.soff[code >> 6], code & 63u, lane & ((1u << lpr) - 1u)) + (deep ? 2u * u * step : 0u);
         dg[u] = r < nr ? sh.rdeg[rr] : 0u;
       }
       for (uint32_t k0 = lane & ((1u << lpr) - 1u); __ballot(k0 < max(dg[0], dg[1]));
-           k0 += 2u << lpr, j0[0] += 2u * step, j0[1] += 2u * step) {
+           k0 += pass << lpr, j0[0] += pass * step, j0[1] += pass * step) {
         nc_slot x[4];
         uint32_t j[4];
         bool in[4];
@@ -372,7 +378,7 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
         // no branch around the reads (slot 0 stands in past a row's end)
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const uint32_t k = k0 + ((uint32_t)(u & 1) << lpr);
+          const uint32_t k = k0 + kb[u >> 1] + ((uint32_t)(u & 1) << lpr);
           in[u] = k < dg[u >> 1];
           // 16 or 64 slots on: whole chunks
           j[u] = in[u] ? j0[u >> 1] + ((u & 1) ? step : 0u) : 0u;
@@ -459,20 +465,31 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
     const uint32_t na = (b_take || pend_n) ? sh.narr[wv][lane] : 0u;
     if (na) {
       cache_dirty = true;
-      if (na <= NC_GARR) {
+      if (na <= NC_GARR(W, RES)) {
         for (uint32_t i = 0; i < na; ++i) {
           const uint2 e = sh.arr[wv][lane][i];
           nc_push(nk, nv, ncnt, e.x, (uint32_t)s, e.y);
         }
       } else {
-        // the first active slots from their records
+        // the first active slots (more arrived than the cache holds) from
+        // their records, read together
+        uint32_t k[NC_ACACHE];
         ncnt = 0;
         for (uint32_t w = 0; w < L.nmw && ncnt < NC_ACACHE; ++w)
           for (uint32_t m = sh.keepw[wv][w][lane]; m && ncnt < NC_ACACHE; m &= m - 1) {
-            const uint32_t k = 32u * w + (uint32_t)__builtin_ctz(m);
-            const nc_slot r = a.slots[nc_slot_of(sh.soff[wv], lane, k)];
-            nc_push(nk, nv, ncnt, k, (uint32_t)(r.arr_inh >> 1), __float_as_uint(r.depol));
+            const uint32_t at = 32u * w + (uint32_t)__builtin_ctz(m);
+#pragma unroll
+            for (int e = 0; e < NC_ACACHE; ++e) k[e] = ncnt == (uint32_t)e || ncnt == 0u ? at : k[e];
+            ++ncnt;
           }
+        nc_slot r[NC_ACACHE];
+#pragma unroll
+        for (int e = 0; e < NC_ACACHE; ++e) r[e] = a.slots[nc_slot_of(sh.soff[wv], lane, k[e])];
+#pragma unroll
+        for (int e = 0; e < NC_ACACHE; ++e) {
+          nk[e] = k[e] | ((uint32_t)(r[e].arr_inh >> 1) << 24);
+          nv[e] = __float_as_uint(r[e].depol);
+        }
       }
     }
     if (cache_dirty)
@@ -524,21 +541,22 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
           (plist ? a.pend1 : a.pend0)[ed.j - ed.rel + pt] = (ed.rel << 8) | ((uint32_t)arr & 255u);
         }
       };
+      const uint32_t pass = deep ? 4u : 2u;
       for (uint32_t r0 = wv; r0 < nr; r0 += 2u * W * per) {
         uint2 o[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-          const uint32_t r = r0 + W * (per * u + (lane >> lpr));
+          const uint32_t r = r0 + W * ((deep ? 0u : per * u) + (lane >> lpr));
           o[u] = sh.rout[min(r, nr - 1u)];
           if (r >= nr) o[u].y = 0u;
         }
-        for (uint32_t i0 = lane & ((1u << lpr) - 1u); __ballot(i0 < max(o[0].y, o[1].y)); i0 += 2u << lpr) {
+        for (uint32_t i0 = lane & ((1u << lpr) - 1u); __ballot(i0 < max(o[0].y, o[1].y)); i0 += pass << lpr) {
           uint32_t e[4];
           bool in[4];
           int32_t lat[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
-            const uint32_t i = i0 + ((uint32_t)(u & 1) << lpr);
+            const uint32_t i = i0 + ((deep ? (uint32_t)u : (uint32_t)(u & 1)) << lpr);
             in[u] = i < o[u >> 1].y;
             e[u] = in[u] ? o[u >> 1].x + i : 0u;
             lat[u] = a.edges[e[u]].arr;
