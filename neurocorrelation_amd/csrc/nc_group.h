@@ -49,6 +49,14 @@ struct nc_net_rec {
   uint32_t act0, nq, net, pad;
 };
 
+// A workgroup barrier for what its waves hand over in LDS: reads from memory
+// stay in flight across it, and stores are not waited for.
+__device__ __forceinline__ void nc_lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 template <int NSL, int W, bool RES>
 struct nc_gsh {
   uint32_t keepw[NSL][NC_GW][64];  // active-mask words
@@ -310,8 +318,13 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
     if (fm) {
       const uint32_t nfl = (uint32_t)__builtin_popcountll(fm);
       uint32_t at = 0;
-      if (lane == 0) at = atomicAdd(&sh.nrow[ph], nfl);
-      at = (uint32_t)__shfl((int)at, 0) + (uint32_t)__builtin_popcountll(fm & ((1ull << lane) - 1ull));
+      if constexpr (NSL == 1) {
+        if (lane == 0) sh.nrow[ph] = nfl;
+      } else {
+        if (lane == 0) at = atomicAdd(&sh.nrow[ph], nfl);
+        at = (uint32_t)__shfl((int)at, 0);
+      }
+      at += (uint32_t)__builtin_popcountll(fm & ((1ull << lane) - 1ull));
       if (fire) {
         sh.row[at] = (wv << 6) | lane;
         sh.rdeg[at] = dw & NC_DEG_MASK;
@@ -327,7 +340,9 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
       }
     }
   }
-  __syncthreads();
+  // Every store to memory of the step before is behind a full barrier of that
+  // step (or of the kernel): only LDS is handed over here.
+  nc_lds_barrier();
   const uint32_t nr = sh.nrow[ph];
   const bool any = sh.any[ph] != 0u;
   // The counts of the step after next, which were last read before this
@@ -403,7 +418,8 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
         }
       }
     }
-    __syncthreads();
+    // No barrier: the arrivals below write no weight of a lane that fired now,
+    // and k_net_steps has one before its fan-out reads these.
   }
 
   if (!RES && f_n) {
@@ -456,7 +472,10 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
         else reinterpret_cast<uint32_t*>(&a.pend_cnt[q0 + wv])[plist] = kept;
       }
     }
-    __syncthreads();
+    // the weights written above are read in this kernel only where it goes on
+    // to the next step
+    if constexpr (RES) __syncthreads();
+    else nc_lds_barrier();
   }
 
   // The owners: the next cache and, unless the group stays resident, the
@@ -466,9 +485,13 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
     if (na) {
       cache_dirty = true;
       if (na <= NC_GARR(W, RES)) {
-        for (uint32_t i = 0; i < na; ++i) {
-          const uint2 e = sh.arr[wv][lane][i];
-          nc_push(nk, nv, ncnt, e.x, (uint32_t)s, e.y);
+        for (uint32_t i = 0; i < na; i += 4u) {
+          uint2 e[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) e[u] = sh.arr[wv][lane][i + u];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (i + u < na) nc_push(nk, nv, ncnt, e[u].x, (uint32_t)s, e[u].y);
         }
       } else {
         // the first active slots (more arrived than the cache holds) from
@@ -499,10 +522,13 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
       sh.lfo[wv][lane] = L.lf;
     } else {
       if (b_take || pend_n) dirty |= sh.dirty[wv][lane];
-      for (uint32_t w = 0; w < L.nmw; ++w) {
-        const uint32_t x = sh.keepw[wv][w][lane];
-        if ((dirty >> w) & 1u) mrow[w * 64] = x;
-        if (x) smk |= 1u << w;
+      uint32_t x[NC_GW];
+#pragma unroll
+      for (uint32_t w = 0; w < NC_GW; ++w) x[w] = sh.keepw[wv][w][lane];  // zero past the lane's words
+#pragma unroll
+      for (uint32_t w = 0; w < NC_GW; ++w) {
+        if ((dirty >> w) & 1u) mrow[w * 64] = x[w];
+        if (x[w]) smk |= 1u << w;
       }
       if (cache_dirty) a.acache[L.pos] = L.cache;
       if (smk != sm) a.asum[L.pos] = smk;
