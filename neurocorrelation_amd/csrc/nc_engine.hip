@@ -91,8 +91,11 @@ inline uint64_t digest_words(uint64_t n, uint64_t S) {
 constexpr size_t kPinBytes = 1u << 20;
 // Host events a call passes through pinned memory (more: copied).
 constexpr size_t kPinEvents = 4096;
-// nc_sim_step's own graphs: steps in one, and the most slices they are for.
-constexpr uint32_t kGraphSteps = 16, kGraphSlices = 2048;
+// nc_sim_step's own graphs: steps in one, and the most slices they are for;
+// calls of how many steps update the graph at hand for other launches, and
+// after how many steps of its launches, with how many to come, a call makes
+// the first one.
+constexpr uint32_t kGraphSteps = 16, kGraphSlices = 2048, kGraphUpdate = 48, kGraphAfter = 96, kGraphLeft = 48;
 
 // First-fit allocator over [0, cap) in units.
 struct RangeAlloc {
@@ -490,6 +493,7 @@ struct nc_sim {
   hipGraphExec_t graph = nullptr;
   nc_step_args graph_args{};
   uint32_t graph_key[5] = {0, 0, 0, 0, 0};
+  const void* graph_fn[2] = {nullptr, nullptr};  // its two kernels
   nc_step_args last_args{};  // the last call's launches (nc_sim_step's own graphs)
   uint32_t last_key[4] = {0, 0, 0, 0};
   nc_netdesc* d_nets = nullptr;
@@ -1360,6 +1364,9 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     if (s0 != NC_OK) return s0;
   }
   const Form form = step_form(sim);
+  // no launch of the graph at hand is still running: it may be updated
+  const bool idle = sim->graph && hipStreamQuery(st) == hipSuccess;
+  if (!idle) (void)hipGetLastError();
 
   // Host-scheduled events for steps [1, max_run] of this call, per step.
   std::vector<uint32_t>& ev_pos = sim->h_ev_pos;
@@ -1538,9 +1545,13 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   // of cfg.graph_steps steps, or, at the default shape, of kGraphSteps for
   // quiet simulations of few slices, whose launches' gaps count: us per step
   // of 20 000 neurons 11.2 -> 9.6, 60 000 12.3 -> 11.0, 99 991 12.5 -> 11.5;
-  // from 300 000 on, and for busy ones, nothing.  As a capture costs about
-  // what 200 steps gain, it waits for a second call with the same launches;
-  // the last step stays a launch of its own, which reports the activity.
+  // from 300 000 on, and for busy ones, nothing.  (And the host launches 16
+  // steps in 20 us instead of 90: the server's loop, which keeps several
+  // lanes busy, is bound by that.)  Making a graph takes the host 400 us, so
+  // a call makes it behind kGraphAfter of its own steps, or up front when it
+  // repeats the launches of the last one; giving it other launches takes 40
+  // us, up front, for which it has to be idle.  The last step stays a launch
+  // of its own, which reports the activity.
   const bool plain_steps = !form.network && ev_pos.empty() && sim->kernel_timing == 0;
   uint32_t G = plain_steps && sim->cfg.graph_steps && max_run >= sim->cfg.graph_steps ? sim->cfg.graph_steps : 0u;
   const uint32_t key_of[4] = {wpb | form.wide_waves << 8, n_grid, lds,
@@ -1550,61 +1561,79 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     sim->last_args = a;
     memcpy(sim->last_key, key_of, sizeof key_of);
   }
-  const bool own = plain_steps && !sim->cfg.graph_steps && !sim->cfg.persistent && same && !sim->busy &&
-                   a.n_active_slices <= kGraphSlices && max_run > kGraphSteps;
+  bool own = plain_steps && !sim->cfg.graph_steps && !sim->cfg.persistent && !sim->busy &&
+             a.n_active_slices <= kGraphSlices && max_run > kGraphSteps;
+  const uint32_t key[5] = {own ? kGraphSteps : G, key_of[0], key_of[1], key_of[2], key_of[3]};
+  const bool fits = sim->graph && memcmp(&sim->graph_args, &a, sizeof a) == 0 &&
+                    memcmp(sim->graph_key, key, sizeof key) == 0;
+  bool update = false, later = false;
+  if (own && !fits) {
+    update = sim->graph && sim->graph_key[0] == kGraphSteps && sim->graph_fn[0] == fn_neuron &&
+             sim->graph_fn[1] == fn_fanout;
+    if (update) own = idle && max_run >= kGraphUpdate;
+    else if (!same) {
+      own = false;
+      later = max_run >= kGraphAfter + kGraphLeft;
+    }
+  }
   if (own) G = kGraphSteps;
-  if (G) {
-    a.chunk_i = 0;
-    const uint32_t key[5] = {G, key_of[0], key_of[1], key_of[2], key_of[3]};
-    if (!sim->graph || memcmp(&sim->graph_args, &a, sizeof a) != 0 || memcmp(sim->graph_key, key, sizeof key) != 0) {
-      if (sim->graph) {
-        (void)hipGraphExecDestroy(sim->graph);
-        sim->graph = nullptr;
-      }
-      auto capture = [&]() -> nc_status {
-        NC_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        nc_status cs = NC_OK;
-        for (uint32_t c = 0; c < G && cs == NC_OK; ++c) {
-          a.chunk_i = (int32_t)c;
-          uint32_t* bar_arg = bar;
-          void* args[] = {&a, &bar_arg};
-          if (fn_step ? hipLaunchKernel(fn_step, dim3(pgrid), dim3(64 * wpb), args, lds, st) != hipSuccess
-                      : (hipLaunchKernel(fn_neuron, dim3(n_grid), dim3(n_block), args, lds, st) != hipSuccess ||
-                         hipLaunchKernel(fn_fanout, dim3(fan_grid), dim3(64 * wpb), args, 0, st) != hipSuccess))
-            cs = fail(NC_ERR_HIP, "kernel launch during capture failed");
-        }
-        hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, st, sim->d_chunk_off, G);
-        hipGraph_t g = nullptr;
-        const hipError_t ce = hipStreamEndCapture(st, &g);
-        if (cs != NC_OK) {
-          if (g) (void)hipGraphDestroy(g);
-          return cs;
-        }
-        NC_HIP(ce);
-        const hipError_t ie = hipGraphInstantiate(&sim->graph, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        NC_HIP(ie);
-        return NC_OK;
-      };
-      const nc_status cs = capture();
-      a.chunk_i = 0;
-      if (cs == NC_OK) {
-        sim->graph_args = a;
-        memcpy(sim->graph_key, key, sizeof key);
-      } else if (!own) {
-        return cs;
-      } else {
-        // the call's own idea: its steps are launched one by one instead
-        (void)hipGetLastError();
-        sim->graph = nullptr;
-        G = 0;
-      }
+  const nc_step_args plain = a;  // as every captured launch takes it but for chunk_i
+  // The graph of the call's launches into sim->graph, anew or by an update.
+  auto capture = [&](uint32_t steps) -> nc_status {
+    if (sim->graph && !update) {
+      (void)hipGraphExecDestroy(sim->graph);
+      sim->graph = nullptr;
+    }
+    nc_step_args c = plain;
+    NC_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+    nc_status cs = NC_OK;
+    for (uint32_t i = 0; i < steps && cs == NC_OK; ++i) {
+      c.chunk_i = (int32_t)i;
+      uint32_t* bar_arg = bar;
+      void* args[] = {&c, &bar_arg};
+      if (fn_step ? hipLaunchKernel(fn_step, dim3(pgrid), dim3(64 * wpb), args, lds, st) != hipSuccess
+                  : (hipLaunchKernel(fn_neuron, dim3(n_grid), dim3(n_block), args, lds, st) != hipSuccess ||
+                     hipLaunchKernel(fn_fanout, dim3(fan_grid), dim3(64 * wpb), args, 0, st) != hipSuccess))
+        cs = fail(NC_ERR_HIP, "kernel launch during capture failed");
+    }
+    hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, st, sim->d_chunk_off, steps);
+    hipGraph_t g = nullptr;
+    const hipError_t ce = hipStreamEndCapture(st, &g);
+    hipError_t ie = ce;
+    if (cs == NC_OK && ce == hipSuccess) {
+      hipGraphNode_t node;
+      hipGraphExecUpdateResult res;
+      ie = update ? hipGraphExecUpdate(sim->graph, g, &node, &res)
+                  : hipGraphInstantiate(&sim->graph, g, nullptr, nullptr, 0);
+    }
+    if (g) (void)hipGraphDestroy(g);
+    if (cs != NC_OK || ie != hipSuccess) {
+      if (update) (void)hipGraphExecDestroy(sim->graph);
+      sim->graph = nullptr;
+      return cs != NC_OK ? cs : fail(NC_ERR_HIP, hipGetErrorString(ie));
+    }
+    sim->graph_args = plain;
+    memcpy(sim->graph_key, key, sizeof key);
+    sim->graph_key[0] = steps;
+    sim->graph_fn[0] = fn_neuron;
+    sim->graph_fn[1] = fn_fanout;
+    return NC_OK;
+  };
+  if (G && !fits) {
+    const nc_status cs = capture(G);
+    if (cs != NC_OK) {
+      if (!own) return cs;
+      // the call's own idea: its steps are launched one by one instead
+      (void)hipGetLastError();
+      own = false;
+      G = 0;
     }
   }
   // The call in sub-chunks of at most NC_GRING steps (whole graph chunks):
   // the group spike trains of a sub-chunk are drawn into the ring first.
   // The device chunk offset holds the steps launched before the running
   // graph chunk or run of direct launches.
+  static_assert(NC_GRING % kGraphSteps == 0 && NC_GRING >= kGraphAfter + kGraphLeft, "own graphs fit the ring");
   const uint32_t L = G ? (NC_GRING / G) * G : NC_GRING;
   for (uint32_t c0 = 0; c0 < max_run; c0 += L) {
     const uint32_t len = std::min(L, max_run - c0);
@@ -1623,34 +1652,55 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       if (s1 != NC_OK) return s1;
       continue;
     }
-    uint32_t j = 0;
+    uint32_t j = 0;  // steps of the sub-chunk in the device chunk offset
+    auto direct = [&](uint32_t to) -> nc_status {
+      for (uint32_t i = c0 + j; i < c0 + to; ++i) {
+        a.chunk_i = (int32_t)(i - (c0 + j));
+        a.n_ev = ev_ptr[i + 1] - ev_ptr[i];
+        a.ev_pos = sim->d_ev_pos.p + ev_ptr[i];
+        a.ev_kind = sim->d_ev_kind.p + ev_ptr[i];
+        a.use_forced = ev_pos.empty() ? 0 : 1;
+        nc_status s1 = NC_OK;
+        if (a.n_ev) {
+          void* args[] = {&a};
+          hipError_t e = hipLaunchKernel((const void*)k_drive, dim3((a.n_ev + 255) / 256), dim3(256), args, 0, st);
+          if (e != hipSuccess) s1 = fail(NC_ERR_HIP, hipGetErrorString(e));
+        }
+        if (fn_step) {
+          if (s1 == NC_OK) s1 = launch(1, fn_step, pgrid, 64 * wpb, lds);
+        } else {
+          if (s1 == NC_OK) s1 = launch(1, fn_neuron, n_grid, n_block, lds);
+          if (i + 1 == max_run) a.call_tag = sim->calls;
+          if (s1 == NC_OK) s1 = launch(3, fn_fanout, fan_grid, 64 * wpb, 0);
+        }
+        if (s1 != NC_OK) return s1;
+        sim->timing_step++;
+      }
+      return NC_OK;
+    };
+    auto advance = [&](uint32_t steps) -> nc_status {
+      hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, st, sim->d_chunk_off, steps);
+      NC_HIP(hipGetLastError());
+      return NC_OK;
+    };
+    if (later) {
+      // the graph is made while the device runs the call's first steps
+      later = false;
+      nc_status s1 = direct(kGraphAfter);
+      if (s1 == NC_OK) s1 = advance(kGraphAfter);
+      if (s1 != NC_OK) return s1;
+      j = kGraphAfter;
+      own = capture(kGraphSteps) == NC_OK;
+      if (own) G = kGraphSteps;
+      else (void)hipGetLastError();
+    }
     if (G)
       for (; len - j >= G + (own && c0 + len == max_run ? 1u : 0u); j += G) NC_HIP(hipGraphLaunch(sim->graph, st));
-    for (uint32_t i = c0 + j; i < c0 + len; ++i) {
-      a.chunk_i = (int32_t)(i - (c0 + j));
-      a.n_ev = ev_ptr[i + 1] - ev_ptr[i];
-      a.ev_pos = sim->d_ev_pos.p + ev_ptr[i];
-      a.ev_kind = sim->d_ev_kind.p + ev_ptr[i];
-      a.use_forced = ev_pos.empty() ? 0 : 1;
-      nc_status s1 = NC_OK;
-      if (a.n_ev) {
-        void* args[] = {&a};
-        hipError_t e = hipLaunchKernel((const void*)k_drive, dim3((a.n_ev + 255) / 256), dim3(256), args, 0, st);
-        if (e != hipSuccess) s1 = fail(NC_ERR_HIP, hipGetErrorString(e));
-      }
-      if (fn_step) {
-        if (s1 == NC_OK) s1 = launch(1, fn_step, pgrid, 64 * wpb, lds);
-      } else {
-        if (s1 == NC_OK) s1 = launch(1, fn_neuron, n_grid, n_block, lds);
-        if (i + 1 == max_run) a.call_tag = sim->calls;
-        if (s1 == NC_OK) s1 = launch(3, fn_fanout, fan_grid, 64 * wpb, 0);
-      }
-      if (s1 != NC_OK) return s1;
-      sim->timing_step++;
-    }
+    const nc_status s1 = direct(len);
+    if (s1 != NC_OK) return s1;
     if (j < len && c0 + len < max_run) {
-      hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, st, sim->d_chunk_off, len - j);
-      NC_HIP(hipGetLastError());
+      const nc_status s2 = advance(len - j);
+      if (s2 != NC_OK) return s2;
     }
   }
   sim->gstep += max_run;

@@ -197,3 +197,32 @@ def test_where_networks_lie(keep, hole, n, k):
         sim.close()
     calls = [x for c in range(3) for j in keep for x in want[j][3 * c:3 * c + 3]]  # three arrays a call
     _same(got, calls + [x for j in keep for x in want[j][9:]])
+
+
+@pytest.mark.parametrize("sync", [True, False])
+def test_own_graphs_made_and_updated(sync):
+    # a long first call makes the graph behind its first steps (96); networks
+    # that join, stop and leave change its launches, which later calls of 48
+    # steps or more give it when the device is idle, and launch directly when
+    # the calls before still run
+    nets = [_net(n, 40, delay_max=40, seed=n, inhib=0.2, w=(0.05, 0.3)) for n in (3000, 1500, 9000, 2000)]
+    got = []
+    for shape in ({}, PER_SLICE):
+        sim = nc.Simulation(sum(m.n + 64 for m in nets), sum(m.n_syn for m in nets), 4)
+        sim.set_launch(**shape)
+        add = lambda j, steps=0: sim.add(nets[j], None, _drive(nets[j].n, j, bg=0.002), steps=steps)
+        ids = {0: add(0)}
+        out = []
+        for steps, join, left in ((143, None, None), (144, 1, None), (200, 2, None), (48, None, 1), (47, 3, None),
+                                  (1300, None, None), (60, None, 0), (60, 1, None), (15, None, None)):
+            sim.step(steps)
+            if left is not None:
+                out += _state(sim, ids[left], nets[left])
+                sim.remove(ids.pop(left))
+            if join is not None:
+                ids[join] = add(join, 250 if join == 2 else 0)
+            if sync:
+                out += [sim.potential(i, nets[j].n) for j, i in ids.items()]
+        got.append(out + [x for j, i in ids.items() for x in _state(sim, i, nets[j])])
+        sim.close()
+    _same(*got)
