@@ -234,8 +234,11 @@ __global__ __launch_bounds__(256) void k_restore_latches(nc_edge* e, const nc_sl
 //   k_fnv_sum    a thread per piece, its low byte now known, adds its terms.
 // The host hashes a byte per four to five clocks, after copying the results:
 // 18 ms of the server's loop for 24 jobs of 4.4e6 words in all, 4.8 so.
+// A segment's chain is what k_fnv_maps takes for all but the largest results
+// (those take the arithmetic, 256 chains): segments of 1024 words 71 us a job
+// of that burst, of 256 words 26.
 #define NC_FNV_PIECE 64u
-#define NC_FNV_SEG 1024u
+#define NC_FNV_SEG 256u
 #define NC_FNV_GROUP 64u
 #define NC_FNV_P 1099511628211ull
 

@@ -1,7 +1,7 @@
 """The digest of a served job's result, computed on the device, against
 nc_digest (FNV-1a, pinned to published vectors in test_serve_wire.py) of the
 same job's arrays read from a run alone: sizes on either side of where the
-device takes it up, of a segment (1024 words) and of a group of 64."""
+device takes it up, of a segment (256 words) and of a group of 64."""
 import pytest
 
 from neurocorrelation_amd import serve, workloads as W
