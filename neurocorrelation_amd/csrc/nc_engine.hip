@@ -1262,26 +1262,27 @@ namespace {
 // fires, the activity that the device last reported (no form changes a
 // result).  The lines, us per step of either side (a network's slices are
 // 64 neurons each; "busy": a fifth of the neurons fire):
-//   - networks of up to 16 slices, a workgroup each: 300 neurons 2.1 against
-//     6.9 (k_neuron and k_fanout launches), 1000 quiet neurons 3.3 against
-//     8.2, 1024 busy networks of 200-1000 neurons 108 against 181.  One
+//   - networks of up to 16 slices, a workgroup each: 300 neurons 1.9 against
+//     5.7 (k_neuron and k_fanout launches), 1000 quiet neurons 3.0 against
+//     7.2, 1024 busy networks of 200-1000 neurons 103 against 194.  One
 //     compute unit per network bounds it: a busy network of 10 slices takes
-//     15.2 here and 21.2 in the wide form, one of 16 slices 23.6 and 21.7,
-//     64 of 3-16 slices 41 and 35, 256 of them 47 and 54.
-//   - up to 1024 slices, four waves a slice: 20 000 busy neurons 26.9 against
-//     49.8 of k_neuron, 60 000 quiet ones 11.5 against 12.4.
-//   - up to 4096 slices, two waves, if busy (2700 slices: 85 against 113);
-//     1563 quiet slices take 13.6 against 12.0 of k_neuron.
-//   - above, one wave, if busy (19 200 slices: 464 against 487); 10^6 quiet
-//     neurons take 91.7 against 87.4 of k_neuron.
-//   - above 8192 slices, quiet: k_neuron and k_fanout of one wave per
-//     workgroup in XCD order: 84.2 against 87.5 at 10^6 neurons (an XCD's L2
-//     then holds a run of slices and most of its fan-out targets), 56.0
-//     against 56.2 at 600 000; at 300 000 nothing, below it costs.
+//     14.9 here and 18.0 in the wide form, one of 16 slices 21.7 and 18.4,
+//     64 of 3-16 slices 34.0 and 32.2, 256 of them 45 and 48.
+//   - up to 1024 slices, four waves a slice: 20 000 busy neurons 24.3 against
+//     51.2 of k_neuron, 60 000 quiet ones 9.6 either way.
+//   - up to 4096 slices, two waves, if busy (2700 slices: 81 against 112);
+//     1563 quiet slices take 10.5 against 10.2 of k_neuron.
+//   - above, one wave, if busy (19 200 slices: 401 against 454).
+//   - above 8192 slices, quiet: one wave, k_neuron_wide and k_fanout in XCD
+//     order (an XCD's L2 then holds a run of slices and most of its fan-out
+//     targets): 77.9 at 10^6 neurons against 79.2 in launch order, 82.5 of
+//     k_neuron in XCD order and 85.4 without; 600 000 51.7 against 54.1, or,
+//     of a tenth of the activity, 18.7 against 19.6.  300 000 such take 13.8
+//     against k_neuron's 13.4.
 struct Form {
   bool network = false;     // k_net_steps
   uint32_t wide_waves = 0;  // k_neuron_wide with this many waves per slice (0: k_neuron)
-  bool xcd = false;         // k_neuron and k_fanout of one wave per workgroup, in XCD order
+  bool xcd = false;         // workgroups in XCD order, those of k_fanout of one wave
 };
 
 Form step_form(const nc_sim* sim) {
@@ -1298,7 +1299,7 @@ Form step_form(const nc_sim* sim) {
   }
   if (slices <= 1024) f.wide_waves = 4;
   else if (sim->busy) f.wide_waves = slices <= 4096 ? 2 : 1;
-  else f.xcd = slices > 8192;
+  else if (slices > 8192) f.wide_waves = 1, f.xcd = true;
   return f;
 }
 

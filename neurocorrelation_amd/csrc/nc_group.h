@@ -361,8 +361,9 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
     f_n = a.fsplit_od ? min(NC_FSPLIT, (nr * a.fsplit_od + 63u) >> 6) : 1u;
     // the list whose readers run on this workgroup's XCD: k_fanout's block of
     // four waves takes lists 4b .. 4b + 3 modulo 64, and blocks go round the
-    // eight XCDs in turn
-    const uint32_t b = 4u * (rec_i & 7u) + ((rec_i >> 3) & 3u) + (rec_i & 32u);
+    // eight XCDs in turn; in XCD order, one of the XCD's eight
+    const uint32_t b = a.xcd_lists ? 8u * (blockIdx.x & 7u) + ((blockIdx.x >> 3) & 7u)
+                                   : 4u * (rec_i & 7u) + ((rec_i >> 3) & 3u) + (rec_i & 32u);
     f_at = b * a.fcap + atomicAdd(&a.fired_cnt[(par * NC_FLISTS + b) * NC_FCNT_STRIDE], f_n);
   }
 
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6))) voi
   __shared__ nc_gsh<1, W, false> sh;
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t i = blockIdx.x + nc_have_neuron_args(a);
+  const uint32_t i = nc_block_id(a.xcd_swizzle + nc_have_neuron_args(a));
   const nc_slice_rec rec = a.active_slices[i];
   const uint32_t q = nc_slice_of(a, rec, i);
   nc_glane L;
