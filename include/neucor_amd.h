@@ -198,8 +198,8 @@ nc_status nc_sim_remove(nc_sim* sim, int32_t net_id);
  * the per-call network windows and due host events to buffers sized by
  * nc_sim_create, nc_sim_add and nc_push_forced: it never allocates device
  * memory (under a graph launch shape it captures and instantiates a graph
- * when the shape or the set of networks changed; at the default shape, where
- * captured chunks pay, from the second call with the same launches on). */
+ * when the shape or the set of networks changed; at the default shape it does
+ * so of its own where captured chunks pay, or updates the graph it has). */
 nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps);
 
 /* Steps each network has completed and has left (0 = finished when it was
