@@ -11,8 +11,8 @@
 // lane per neuron, which sums the charge, decides the fire and writes the
 // neuron's state.  What a wave of k_neuron does one fired lane and one batch
 // of 64 arrivals after the other is shared by all waves through LDS:
-//   post-side STDP  two fired lanes' rows per wave at a time, or eight when
-//                   many fired
+//   post-side STDP  two fired lanes' rows per wave at a time, or four or
+//                   eight when many fired
 //   arrivals        a lane per bucket entry, whose record's weight was read
 //                   while the owners summed the charge; mask bits and the new
 //                   active slots go to their owner through LDS

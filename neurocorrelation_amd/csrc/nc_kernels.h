@@ -495,10 +495,10 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
   // so that the wave waits for each one alone (a load under a branch makes
   // the wait before the next use cover every load in flight): the active-slot
   // cache (read only while the walk is within it), the id (used by the
-  // background draw), all NC_BCAP entry places of the arrival bucket of step
-  // s (the first b_n hold this step's arrivals: spikes with delays up to NC_NB
+  // background draw), the first 64 entry places of the arrival bucket of step
+  // s (its first b_n hold this step's arrivals: spikes with delays up to NC_NB
   // that found room in it; the others wait in the pending list of s's arrival
-  // window) and the group-spike-train word of an input's group (word 0 for
+  // window, where entries past the 64 join them) and the group-spike-train word of an input's group (word 0 for
   // the others; gfire points at a zero word when there are no groups).
   const uint4 cache = a.acache[pos];
   const uint32_t my_nid = a.nid[pos];
