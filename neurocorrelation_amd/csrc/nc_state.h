@@ -168,13 +168,18 @@ __global__ __launch_bounds__(256) void k_check_checkpoint(const uint32_t* in, ui
 // rel steps: a lane per neuron lays out its neuron, its slot records and,
 // from their arrivals, its active mask words and their summary, its cache of
 // the first active slots and its spikes in flight (in the pending list of
-// their window: their buckets are not theirs to fill in order).
+// their window: their buckets are not theirs to fill in order).  The lists
+// start empty: they hold the spikes of a checkpoint restored here before, if
+// that one was taken before its first step.
 __global__ __launch_bounds__(64) void k_unpack(nc_place N, const uint32_t* nid, const uint32_t* slice_moff,
                                                const uint32_t* in, int32_t s, int32_t rel, float* V,
                                                int32_t* last_fire, uint32_t* firings, uint32_t* amask, uint32_t* asum,
                                                uint4* acache, uint32_t* pend0, uint32_t* pend1, uint2* pend_cnt) {
   const uint32_t q = N.q0 + blockIdx.x, lane = threadIdx.x, pos = q * 64u + lane;
   const uint32_t dw = N.ndw[pos].x;
+  if (lane == 0) pend_cnt[q] = make_uint2(0u, 0u);
+  __threadfence();
+  __syncthreads();
   if (!(dw & NC_DEG_VALID)) return;
   const uint32_t id = nid[pos], deg = dw & NC_DEG_MASK, row = N.id_row[N.pos0 + id], so = N.slice_off[q];
   V[pos] = __uint_as_float(in[3ull * id]);
