@@ -239,9 +239,9 @@ nc_status nc_read_firings(nc_sim* sim, int32_t net_id, uint32_t* out, uint32_t n
 nc_status nc_read_weights(nc_sim* sim, int32_t net_id, float* out, uint64_t n);
 nc_status nc_write_weights(nc_sim* sim, int32_t net_id, const float* w, uint64_t n);
 
-/* nc_read_weights without any device allocation.  No counterpart in the
- * reference: for callers that cannot allocate device memory (code under HIP
- * graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
+/* nc_read_weights without any allocation (nor any thread of its own).  No
+ * counterpart in the reference: for callers that cannot allocate (code under
+ * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * weights are gathered in export order into a static per-GPU scratch array
  * of 16,777,216 floats (64 MiB, held by every GPU the library runs on until
  * the process ends; reads of up to 1 MiB into the simulation's pinned host

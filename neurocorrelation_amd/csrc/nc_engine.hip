@@ -1864,9 +1864,17 @@ extern "C" nc_status nc_read_weights_noalloc(nc_sim* sim, int32_t net_id, float*
   if (!scr) return fail(NC_ERR_STATE, "the static scratch of this device is not set up");
   NC_HIP(hipSetDevice(sim->device));
   if (r->S == 0 || n == 0) return NC_OK;
-  // the export kernel writes every entry that the copy reads: nothing needs
-  // clearing first
-  return export_weights(sim, *r, scr, out, n);
+  // Nothing here allocates, starts a thread or takes from the pinned chunks:
+  // small results go through the simulation's own pinned buffer, others from
+  // the scratch (whose every entry the kernel writes first) to `out` in one
+  // copy.
+  if (4 * n <= kPinBytes) return export_weights(sim, *r, scr, out, n);
+  hipLaunchKernelGGL(k_read_weights, row_blocks(*r), dim3(256), 0, sim->stream, place_of(sim, *r), scr, (uint32_t)n,
+                     nc_done{nullptr, nullptr, 0u});
+  NC_HIP(hipGetLastError());
+  NC_HIP(hipMemcpyAsync(out, scr, 4 * n, hipMemcpyDeviceToHost, sim->stream));
+  NC_HIP(hipStreamSynchronize(sim->stream));
+  return check_barrier(sim);
 }
 NC_ABI_CATCH
 
