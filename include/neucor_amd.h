@@ -360,6 +360,16 @@ typedef struct nc_launch_cfg {
 nc_status nc_sim_set_launch(nc_sim* sim, const nc_launch_cfg* cfg);
 nc_status nc_sim_get_launch(const nc_sim* sim, nc_launch_cfg* cfg);
 
+/* How the last nc_sim_step with steps to take launched them: a diagnostic of
+ * what the default shape chose. */
+typedef struct nc_launch_info {
+  uint32_t networks;        /* 1: a workgroup per network, all steps of the call in one launch */
+  uint32_t waves_per_slice; /* of the neuron kernel's several-wave form (0: its form of a wave per slice) */
+  uint32_t graph_steps;     /* steps of a captured chunk it launched (0: none) */
+  uint32_t graph_made;      /* 1: it captured a graph, or gave the one at hand other launches */
+} nc_launch_info;
+nc_status nc_sim_last_launch(const nc_sim* sim, nc_launch_info* info);
+
 /* Autotuner of the launch shape over 38 shapes: {1, 2, 4, 8 slices per
  * workgroup} x {XCD order off/on} x {LDS tables off/on} x {no graph, graph
  * chunks of steps_per_trial steps}, and the persistent form with {2, 4, 8}

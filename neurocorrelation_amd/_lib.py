@@ -53,6 +53,11 @@ class LaunchCfg(C.Structure):
                 ("stage_tables", C.c_uint32), ("fanout_waves", C.c_uint32), ("persistent", C.c_uint32)]
 
 
+class LaunchInfo(C.Structure):
+    _fields_ = [("networks", C.c_uint32), ("waves_per_slice", C.c_uint32), ("graph_steps", C.c_uint32),
+                ("graph_made", C.c_uint32)]
+
+
 class ServerSpec(C.Structure):
     _fields_ = [
         ("device", C.c_int32), ("lanes", C.c_uint32), ("chunk", C.c_uint32), ("builders", C.c_uint32),
@@ -133,6 +138,7 @@ SIGNATURES = {
     "nc_sim_restore": (C.c_int, [P, C.c_int32, C.c_void_p, C.c_uint64]),
     "nc_sim_set_launch": (C.c_int, [P, C.POINTER(LaunchCfg)]),
     "nc_sim_get_launch": (C.c_int, [P, C.POINTER(LaunchCfg)]),
+    "nc_sim_last_launch": (C.c_int, [P, C.POINTER(LaunchInfo)]),
     "nc_sim_tune": (C.c_int, [P, C.c_uint32, C.POINTER(LaunchCfg)]),
     "nc_sim_tune_list": (C.c_int, [P, C.POINTER(LaunchCfg), C.c_uint32, C.c_uint32, C.c_uint32,
                                    C.POINTER(LaunchCfg), C.POINTER(C.c_float)]),

@@ -496,6 +496,7 @@ struct nc_sim {
   const void* graph_fn[2] = {nullptr, nullptr};  // its two kernels
   nc_step_args last_args{};  // the last call's launches (nc_sim_step's own graphs)
   uint32_t last_key[4] = {0, 0, 0, 0};
+  nc_launch_info info{};  // of the last call
   nc_netdesc* d_nets = nullptr;
   float *t_pre = nullptr, *t_post = nullptr, *w_ap = nullptr;
   uint32_t calls = 0;   // nc_sim_step calls, numbering the activity reports (never 0 in a report)
@@ -1285,11 +1286,14 @@ struct Form {
   bool xcd = false;         // workgroups in XCD order, those of k_fanout of one wave
 };
 
+bool default_shape(const nc_launch_cfg& c) {
+  return c.waves_per_block == 4 && !c.xcd_swizzle && !c.graph_steps && !c.stage_tables && !c.fanout_waves &&
+         !c.persistent;
+}
+
 Form step_form(const nc_sim* sim) {
   Form f;
-  const nc_launch_cfg& c = sim->cfg;
-  if (c.waves_per_block != 4 || c.xcd_swizzle || c.graph_steps || c.stage_tables || c.fanout_waves || c.persistent)
-    return f;
+  if (!default_shape(sim->cfg)) return f;
   if (sim->counting || sim->live_mw > NC_GW) return f;
   const size_t slices = sim->active_host.size();
   if (sim->live_nq <= 16 && !sim->kernel_timing && sim->T.t_pre.size() <= NC_GTAB &&
@@ -1365,6 +1369,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     if (s0 != NC_OK) return s0;
   }
   const Form form = step_form(sim);
+  sim->info = nc_launch_info{form.network ? 1u : 0u, form.wide_waves, 0u, 0u};
   // no launch of the graph at hand is still running: it may be updated
   const bool idle = sim->graph && hipStreamQuery(st) == hipSuccess;
   if (!idle) (void)hipGetLastError();
@@ -1562,8 +1567,8 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     sim->last_args = a;
     memcpy(sim->last_key, key_of, sizeof key_of);
   }
-  bool own = plain_steps && !sim->cfg.graph_steps && !sim->cfg.persistent && !sim->busy &&
-             a.n_active_slices <= kGraphSlices && max_run > kGraphSteps;
+  bool own = plain_steps && default_shape(sim->cfg) && !sim->busy && a.n_active_slices <= kGraphSlices &&
+             max_run > kGraphSteps;
   const uint32_t key[5] = {own ? kGraphSteps : G, key_of[0], key_of[1], key_of[2], key_of[3]};
   const bool fits = sim->graph && memcmp(&sim->graph_args, &a, sizeof a) == 0 &&
                     memcmp(sim->graph_key, key, sizeof key) == 0;
@@ -1581,6 +1586,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   const nc_step_args plain = a;  // as every captured launch takes it but for chunk_i
   // The graph of the call's launches into sim->graph, anew or by an update.
   auto capture = [&](uint32_t steps) -> nc_status {
+    sim->info.graph_made = 1u;
     if (sim->graph && !update) {
       (void)hipGraphExecDestroy(sim->graph);
       sim->graph = nullptr;
@@ -1696,7 +1702,10 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       else (void)hipGetLastError();
     }
     if (G)
-      for (; len - j >= G + (own && c0 + len == max_run ? 1u : 0u); j += G) NC_HIP(hipGraphLaunch(sim->graph, st));
+      for (; len - j >= G + (own && c0 + len == max_run ? 1u : 0u); j += G) {
+        NC_HIP(hipGraphLaunch(sim->graph, st));
+        sim->info.graph_steps = G;
+      }
     const nc_status s1 = direct(len);
     if (s1 != NC_OK) return s1;
     if (j < len && c0 + len < max_run) {
@@ -2334,6 +2343,13 @@ NC_ABI_CATCH
 extern "C" nc_status nc_sim_get_launch(const nc_sim* sim, nc_launch_cfg* cfg) try {
   if (!sim || !cfg) return fail(NC_ERR_ARG, "null argument");
   *cfg = sim->cfg;
+  return NC_OK;
+}
+NC_ABI_CATCH
+
+extern "C" nc_status nc_sim_last_launch(const nc_sim* sim, nc_launch_info* info) try {
+  if (!sim || !info) return fail(NC_ERR_ARG, "null argument");
+  *info = sim->info;
   return NC_OK;
 }
 NC_ABI_CATCH

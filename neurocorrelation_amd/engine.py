@@ -236,6 +236,12 @@ class Simulation:
         check(lib().nc_sim_get_launch(self._h, C.byref(cfg)))
         return _cfg_dict(cfg)
 
+    def last_launch(self):
+        """How the last step call launched its steps (nc_launch_info)."""
+        info = _lib.LaunchInfo()
+        check(lib().nc_sim_last_launch(self._h, C.byref(info)))
+        return {f: getattr(info, f) for f, _ in info._fields_}
+
     def tune(self, steps_per_trial=32):
         """Autotunes the launch shape over the engine's 38 candidate shapes,
         every trial from the same saved state; the simulation is left where
