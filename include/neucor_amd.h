@@ -382,7 +382,8 @@ nc_status nc_sim_tune(nc_sim* sim, uint32_t steps_per_trial, nc_launch_cfg* chos
  * trial starts from that state -- a warm-up trial of steps_per_trial steps,
  * which also captures the candidate's graph, the state put back, then the
  * timed trial of the same steps -- so that every candidate times the same
- * work.  `rounds` rounds visit the candidates in rotated order; each
+ * work (the default shape warms up three times: its launches follow what the
+ * calls before them reported).  `rounds` rounds visit the candidates in rotated order; each
  * candidate's median device time is its score, written to ms_out[i] (may be
  * NULL).  The fastest becomes the launch shape and is reported in *chosen.
  * Afterwards the simulation is exactly where it was before the call (no

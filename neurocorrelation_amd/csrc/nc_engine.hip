@@ -1795,11 +1795,17 @@ extern "C" nc_status nc_push_forced(nc_sim* sim, int32_t net_id, uint32_t n_even
 NC_ABI_CATCH
 
 namespace {
-// After a synchronisation: did a grid barrier of the persistent form time out
-// (a grid whose workgroups were not all resident) since the last check?
-nc_status check_barrier(nc_sim* sim) {
+// After a synchronisation: the activity that the last call reported.
+void read_report(nc_sim* sim) {
   volatile uint32_t* const w = sim->h_words;
   sim->busy = sim->calls && w[0] == sim->calls;
+}
+
+// After a synchronisation: that, and did a grid barrier of the persistent form
+// time out (a grid whose workgroups were not all resident) since the last check?
+nc_status check_barrier(nc_sim* sim) {
+  read_report(sim);
+  volatile uint32_t* const w = sim->h_words;
   if (!w[1]) return NC_OK;
   w[1] = 0u;
   return fail(NC_ERR_STATE, "a grid barrier of the persistent launch timed out: the steps since the last check "
@@ -2384,13 +2390,26 @@ extern "C" nc_status nc_sim_tune_list(nc_sim* sim, const nc_launch_cfg* cands, u
   std::vector<std::vector<float>> ms((size_t)n_cands);
   // Every trial starts from the saved state: a warm-up trial (which also
   // captures the candidate's graph), the state put back, then the timed
-  // trial.  Rounds visit the candidates in rotated order.
+  // trial.  The default shape's launches depend on the activity last reported
+  // and, for its own graph, on the call before: it warms up until they are
+  // those that repeated calls have (the report; its launches; their graph), so
+  // that neither another candidate's report nor a capture (400 us) is timed.
+  // Rounds visit the candidates in rotated order.
+  auto settled = [&]() -> nc_status {
+    NC_HIP(hipStreamSynchronize(sim->stream));
+    read_report(sim);
+    return NC_OK;
+  };
   for (uint32_t rd = 0; rd < rounds && st == NC_OK; ++rd)
     for (uint32_t k = 0; k < n_cands && st == NC_OK; ++k) {
       const uint32_t i = (k + rd * (n_cands / rounds + 1)) % n_cands;
       sim->cfg = cands[i];
-      st = state_restore(sim, saved);
-      if (st == NC_OK) st = nc_sim_step(sim, steps_per_trial);
+      for (int w = default_shape(cands[i]) ? 3 : 1; w > 0 && st == NC_OK; --w) {
+        st = state_restore(sim, saved);
+        if (st == NC_OK) st = settled();
+        if (st == NC_OK) st = nc_sim_step(sim, steps_per_trial);
+        if (st == NC_OK) st = settled();
+      }
       if (st == NC_OK) st = state_restore(sim, saved);
       if (st != NC_OK) break;
       if (hipEventRecord(e0, sim->stream) != hipSuccess) {

@@ -55,3 +55,33 @@ def test_the_default_shape_captures_its_own():
     sim.step(40)
     assert sim.last_launch() == dict(networks=1, waves_per_slice=0, graph_steps=0, graph_made=0)
     sim.close()
+
+
+def test_the_tuner_times_the_default_shape_as_repeated_calls_run():
+    # no capture in the timed trial (the last launch that the tuner made), a
+    # chunk captured before it, also with another shape's graph at hand
+    sim, _ = _quiet(3000)
+    for before in ((), (dict(waves_per_block=4, graph_steps=16),)):
+        for steps in (40, 100):
+            sim.tune_list(list(before) + [{}], steps_per_trial=steps, rounds=1)
+            info = sim.last_launch()
+            assert (info["graph_steps"], info["graph_made"], info["waves_per_slice"]) == (16, 0, 4)
+    sim.close()
+
+
+def test_the_tuner_times_the_form_of_the_activity_it_has():
+    # busy networks of more than 1024 slices: two waves per slice once a report
+    # is read, which no call before the tuner does
+    n, count = 1500, 48
+    nets = [nc.Network.generate(n, W.side_for(n), W.radius_for_degree(25), 1, 20, 0.2, 0.8, seed=i, device=0)
+            for i in range(count)]
+    drive = W.drive_spec(dict(n_inputs=75, n_groups=2, n_correlated=2, period=200, p0=0.05, amp_corr=1.0,
+                              amp_ind=0.5), seed=1)
+    sim = nc.Simulation(count * (n + 64), sum(m.n_syn for m in nets), count)
+    for m in nets:
+        sim.add(m, None, drive)
+    sim.step(80)
+    assert sim.last_launch()["waves_per_slice"] == 0
+    sim.tune_list([dict(waves_per_block=2), {}], steps_per_trial=16, rounds=1)
+    assert sim.last_launch()["waves_per_slice"] == 2
+    sim.close()
