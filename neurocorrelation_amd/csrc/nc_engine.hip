@@ -1368,6 +1368,26 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     nc_status s0 = rebuild_active(sim);
     if (s0 != NC_OK) return s0;
   }
+  // The steps are taken: counted when all of them are launched.
+  auto counted = [&]() {
+    sim->gstep += max_run;
+    for (size_t i = 0; i < sim->nets.size(); ++i) {
+      NetRec& r = sim->nets[i];
+      if (!r.live) continue;
+      uint32_t run = (uint32_t)nds[i].remaining;
+      sim->host_neuron_steps += (uint64_t)run * r.n;
+      sim->host_synapse_steps += (uint64_t)run * r.S;
+      sim->host_mword_steps += (uint64_t)run * r.mwords_step;
+      r.steps_done += run;
+      if (r.steps_left != UINT32_MAX) r.steps_left -= run;
+    }
+  };
+  if (sim->active_host.empty()) {
+    // no network has a neuron: there is nothing to launch
+    sim->info = nc_launch_info{0u, 0u, 0u, 0u};
+    counted();
+    return NC_OK;
+  }
   const Form form = step_form(sim);
   sim->info = nc_launch_info{form.network ? 1u : 0u, form.wide_waves, 0u, 0u};
   // no launch of the graph at hand is still running: it may be updated
@@ -1713,7 +1733,6 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       if (s2 != NC_OK) return s2;
     }
   }
-  sim->gstep += max_run;
   if (!timed_kinds.empty()) {
     NC_HIP(hipEventSynchronize(sim->ev_pool[nev_used - 1]));
     for (size_t q = 0; q < timed_kinds.size(); ++q) {
@@ -1722,16 +1741,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       sim->k_ms[timed_kinds[q]] += ms;
     }
   }
-  for (size_t i = 0; i < sim->nets.size(); ++i) {
-    NetRec& r = sim->nets[i];
-    if (!r.live) continue;
-    uint32_t run = (uint32_t)nds[i].remaining;
-    sim->host_neuron_steps += (uint64_t)run * r.n;
-    sim->host_synapse_steps += (uint64_t)run * r.S;
-    sim->host_mword_steps += (uint64_t)run * r.mwords_step;
-    r.steps_done += run;
-    if (r.steps_left != UINT32_MAX) r.steps_left -= run;
-  }
+  counted();
   return NC_OK;
 }
 NC_ABI_CATCH
