@@ -1394,36 +1394,50 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   const bool idle = sim->graph && hipStreamQuery(st) == hipSuccess;
   if (!idle) (void)hipGetLastError();
 
-  // Host-scheduled events for steps [1, max_run] of this call, per step.
+  // Host-scheduled events for steps [1, max_run] of this call: counted per
+  // step, then each placed among those of its step, in queue order (a sort of
+  // 10^6 in no order took 108 ms, this 15).
   std::vector<uint32_t>& ev_pos = sim->h_ev_pos;
   std::vector<uint8_t>& ev_kind = sim->h_ev_kind;
   std::vector<uint32_t>& ev_step = sim->h_ev_step;
-  ev_step.clear();
-  ev_pos.clear();
-  ev_kind.clear();
-  std::vector<uint32_t> ev_ptr(max_run + 1, 0);
+  std::vector<uint32_t> ev_ptr(max_run + 1, 0);  // the first event of each step
+  size_t n_ev = 0;
+  for (size_t i = 0; i < sim->nets.size(); ++i) {
+    const NetRec& r = sim->nets[i];
+    if (!r.live) continue;
+    const uint32_t run = (uint32_t)nds[i].remaining;
+    for (const auto& ev : r.events) {
+      const uint32_t k = ev.first - r.steps_done;  // 1-based offset in this call
+      if (k >= 1 && k <= run) ++ev_ptr[k], ++n_ev;
+    }
+  }
+  ev_pos.resize(n_ev);
+  ev_kind.resize(n_ev);
+  ev_step.resize(n_ev);
+  if (n_ev)
+    for (uint32_t k = 0; k < max_run; ++k) ev_ptr[k + 1] += ev_ptr[k];
   {
-    std::vector<std::pair<uint32_t, std::pair<uint32_t, uint8_t>>> due;  // by step of the call, in queue order
+    std::vector<uint32_t> at;
+    if (n_ev) at.assign(ev_ptr.begin(), ev_ptr.end() - 1);
     for (size_t i = 0; i < sim->nets.size(); ++i) {
       NetRec& r = sim->nets[i];
       if (!r.live || r.events.empty()) continue;
-      std::vector<std::pair<uint32_t, std::pair<uint32_t, uint8_t>>> keep;
       const uint32_t run = (uint32_t)nds[i].remaining;
-      for (auto& ev : r.events) {
-        uint32_t k = ev.first - r.steps_done;  // 1-based offset in this call
-        if (k >= 1 && k <= run) due.push_back({k - 1, ev.second});
-        else if (k > run) keep.push_back(ev);
+      size_t kept = 0;
+      for (size_t e = 0; e < r.events.size(); ++e) {
+        const auto ev = r.events[e];
+        const uint32_t k = ev.first - r.steps_done;
+        if (k >= 1 && k <= run) {
+          const uint32_t o = at[k - 1]++;
+          ev_pos[o] = ev.second.first;
+          ev_kind[o] = ev.second.second;
+          ev_step[o] = k - 1;
+        } else if (k > run) {
+          r.events[kept++] = ev;
+        }
       }
-      r.events.swap(keep);
+      r.events.resize(kept);
     }
-    std::stable_sort(due.begin(), due.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
-    for (auto& e : due) {
-      ++ev_ptr[e.first + 1];
-      ev_pos.push_back(e.second.first);
-      ev_kind.push_back(e.second.second);
-      ev_step.push_back(e.first);
-    }
-    for (uint32_t k = 0; k < max_run; ++k) ev_ptr[k + 1] += ev_ptr[k];
   }
   nc_begin b;
   memset(&b, 0, sizeof b);
@@ -1436,7 +1450,6 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     b.n[p] = (uint32_t)words;
   };
   part(0, sim->d_nets, nds, sim->nets.size() * (sizeof(nc_netdesc) / 4));
-  const size_t n_ev = ev_pos.size();
   if (n_ev) {
     // nc_push_forced and nc_sim_restore reserve room for every queued event
     if (sim->d_ev_pos.n < n_ev || sim->d_ev_kind.n < n_ev || sim->d_ev_step.n < n_ev)
