@@ -1396,7 +1396,8 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
 
   // Host-scheduled events for steps [1, max_run] of this call: counted per
   // step, then each placed among those of its step, in queue order (a sort of
-  // 10^6 in no order took 108 ms, this 15).
+  // 10^6 in no order took 108 ms, this 15).  The workgroup-per-network form
+  // takes them network by network, each network's by step.
   std::vector<uint32_t>& ev_pos = sim->h_ev_pos;
   std::vector<uint8_t>& ev_kind = sim->h_ev_kind;
   std::vector<uint32_t>& ev_step = sim->h_ev_step;
@@ -1406,37 +1407,55 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     const NetRec& r = sim->nets[i];
     if (!r.live) continue;
     const uint32_t run = (uint32_t)nds[i].remaining;
+    nds[i].ev0 = (uint32_t)n_ev;
     for (const auto& ev : r.events) {
       const uint32_t k = ev.first - r.steps_done;  // 1-based offset in this call
       if (k >= 1 && k <= run) ++ev_ptr[k], ++n_ev;
     }
+    nds[i].ev1 = (uint32_t)n_ev;
   }
   ev_pos.resize(n_ev);
   ev_kind.resize(n_ev);
   ev_step.resize(n_ev);
-  if (n_ev)
+  if (n_ev) {
     for (uint32_t k = 0; k < max_run; ++k) ev_ptr[k + 1] += ev_ptr[k];
-  {
-    std::vector<uint32_t> at;
-    if (n_ev) at.assign(ev_ptr.begin(), ev_ptr.end() - 1);
+    std::vector<uint32_t> at(ev_ptr.begin(), ev_ptr.end() - 1), pos, step;
+    std::vector<uint8_t> kind;
     for (size_t i = 0; i < sim->nets.size(); ++i) {
       NetRec& r = sim->nets[i];
       if (!r.live || r.events.empty()) continue;
-      const uint32_t run = (uint32_t)nds[i].remaining;
+      const uint32_t run = (uint32_t)nds[i].remaining, e0 = nds[i].ev0, e1 = nds[i].ev1;
       size_t kept = 0;
+      uint32_t next = e0, last = 0;
+      bool ascending = true;
       for (size_t e = 0; e < r.events.size(); ++e) {
         const auto ev = r.events[e];
         const uint32_t k = ev.first - r.steps_done;
         if (k >= 1 && k <= run) {
-          const uint32_t o = at[k - 1]++;
+          const uint32_t o = form.network ? next++ : at[k - 1]++;
           ev_pos[o] = ev.second.first;
           ev_kind[o] = ev.second.second;
           ev_step[o] = k - 1;
+          ascending &= k >= last;
+          last = k;
         } else if (k > run) {
           r.events[kept++] = ev;
         }
       }
       r.events.resize(kept);
+      if (!form.network || ascending) continue;
+      pos.assign(ev_pos.begin() + e0, ev_pos.begin() + e1);
+      kind.assign(ev_kind.begin() + e0, ev_kind.begin() + e1);
+      step.assign(ev_step.begin() + e0, ev_step.begin() + e1);
+      at.assign(run + 1, 0);
+      for (uint32_t k : step) ++at[k + 1];
+      for (uint32_t k = 0; k < run; ++k) at[k + 1] += at[k];
+      for (size_t e = 0; e < step.size(); ++e) {
+        const uint32_t o = e0 + at[step[e]]++;
+        ev_pos[o] = pos[e];
+        ev_kind[o] = kind[e];
+        ev_step[o] = step[e];
+      }
     }
   }
   nc_begin b;
@@ -1683,7 +1702,6 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     }
     if (form.network) {
       if (c0 + len == max_run) a.call_tag = sim->calls;
-      a.n_ev = (uint32_t)ev_pos.size();
       a.ev_pos = sim->d_ev_pos.p;
       a.ev_kind = sim->d_ev_kind.p;
       const nc_status s1 = sim->live_nq <= 4   ? launch_networks<4, 8>(sim, a, c0, len)

@@ -104,7 +104,8 @@ struct nc_netdesc {
   uint32_t bg_thr;              // background threshold on a u32 draw (0 = off)
   uint32_t bg_lo, bg_hi;        // background seed
   int32_t whost;                // first step after the last host weight write
-  uint32_t pad[5];
+  uint32_t ev0, ev1;            // its host events of the call, by step (k_net_steps)
+  uint32_t pad[3];
 };
 
 // One record per active slice (one wave).
