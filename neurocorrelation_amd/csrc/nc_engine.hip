@@ -488,7 +488,7 @@ struct nc_sim {
   bool counting = false;
   uint32_t* d_chunk_off = nullptr;  // steps of the current call before the running chunk
   nc_launch_cfg cfg{4, 0, 0, 0, 0, 0};
-  int resident[9] = {0};  // persistent form: workgroups of 1..8 waves the device holds at once (0 = not known)
+  int cus = 256;  // the device's compute units
   // captured chunk of cfg.graph_steps steps and the launch it was captured for
   hipGraphExec_t graph = nullptr;
   nc_step_args graph_args{};
@@ -873,6 +873,7 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
   };
   H(hipSetDevice(spec->device), "hipSetDevice");
   if (st == NC_OK) st = scratch_setup(spec->device);  // once per device, with it current
+  H(hipDeviceGetAttribute(&sim->cus, hipDeviceAttributeMultiprocessorCount, spec->device), "hipDeviceGetAttribute");
   H(hipStreamCreateWithFlags(&sim->stream, hipStreamNonBlocking), "hipStreamCreate");
   H(hipEventCreateWithFlags(&sim->upload_done, hipEventDisableTiming), "hipEventCreate");
   sim->max_pos = (spec->max_neurons + 63) / 64 * 64 + 64 * (uint64_t)spec->max_nets;
@@ -1269,6 +1270,16 @@ namespace {
 //     compute unit per network bounds it: a busy network of 10 slices takes
 //     14.9 here and 18.0 in the wide form, one of 16 slices 21.7 and 18.4,
 //     64 of 3-16 slices 34.0 and 32.2, 256 of them 45 and 48.
+//     More networks than the device holds workgroups (two of 8 waves or one of
+//     16 per compute unit) follow in rounds, of which each takes a step's time
+//     for every step and about 8 us of its own.  Both sides' times, by a
+//     network's slices and in all (see the code), so that a call of n steps
+//     goes the shorter way.  Quiet, 50 steps: 1024 of 64 neurons 6.4 against
+//     11.6, 2048 10.7 and 12.6, 4096 18.9 and 13.0; 1024 of 300 11.3 and 14.3,
+//     4096 43.8 and 31.5; 1000 of 64 and one of 1000 10.8 and 11.1, 2000 18.9
+//     and 12.6; 1024 of 1000 19.4 and 28.5.  Calls of one step: 1024 of 64 43
+//     and 37, 2048 of 600 118 and 66.  Busy, 50 steps: 4096 of 64 24.4 and
+//     17.0, 2048 of 300 59 and 52, 2048 of 600 85 and 118.
 //   - up to 1024 slices, four waves a slice: 20 000 busy neurons 24.3 against
 //     51.2 of k_neuron, 60 000 quiet ones 9.6 either way.
 //   - up to 4096 slices, two waves, if busy (2700 slices: 81 against 112);
@@ -1291,15 +1302,21 @@ bool default_shape(const nc_launch_cfg& c) {
          !c.persistent;
 }
 
-Form step_form(const nc_sim* sim) {
+Form step_form(const nc_sim* sim, uint32_t steps) {
   Form f;
   if (!default_shape(sim->cfg)) return f;
   if (sim->counting || sim->live_mw > NC_GW) return f;
-  const size_t slices = sim->active_host.size();
+  const size_t slices = sim->active_host.size(), nets = sim->net_recs_host.size();
   if (sim->live_nq <= 16 && !sim->kernel_timing && sim->T.t_pre.size() <= NC_GTAB &&
       sim->T.t_post.size() <= NC_GTAB && !(sim->busy && sim->live_nq > 12 && slices <= 1024)) {
-    f.network = true;
-    return f;
+    const double held = (double)sim->cus * (sim->live_nq <= 4 ? 2 : 1), rounds = ceil((double)nets / held);
+    const double size = (double)slices / (double)nets;
+    const double one = sim->busy ? 2.0 + 1.05 * size : 2.4 + 0.16 * size;
+    const double two = sim->busy ? 11.0 + 0.0045 * slices : 10.0 + 0.0012 * slices;
+    if (rounds <= 1.0 || 8.0 * (rounds - 1.0) + steps * one * rounds < steps * two) {
+      f.network = true;
+      return f;
+    }
   }
   if (slices <= 1024) f.wide_waves = 4;
   else if (sim->busy) f.wide_waves = slices <= 4096 ? 2 : 1;
@@ -1388,7 +1405,7 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
     counted();
     return NC_OK;
   }
-  const Form form = step_form(sim);
+  const Form form = step_form(sim, max_run);
   sim->info = nc_launch_info{form.network ? 1u : 0u, form.wide_waves, 0u, 0u};
   // no launch of the graph at hand is still running: it may be updated
   const bool idle = sim->graph && hipStreamQuery(st) == hipSuccess;
@@ -1563,10 +1580,9 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
       case 8: fn_step = (const void*)k_step<8>; break;
       default: fn_step = (const void*)k_step<4>; break;
     }
-    int per_cu = 0, cus = 0;
+    int per_cu = 0;
     NC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn_step, (int)(64 * wpb), lds));
-    NC_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, sim->device));
-    pgrid = std::min<uint32_t>((uint32_t)std::max(per_cu, 0) * (uint32_t)std::max(cus, 0), std::max(grid, fan_grid));
+    pgrid = std::min<uint32_t>((uint32_t)std::max(per_cu, 0) * (uint32_t)sim->cus, std::max(grid, fan_grid));
     if (pgrid * wpb < NC_FLISTS) return fail(NC_ERR_STATE, "the device holds too few workgroups for the persistent form");
   }
   switch (form.wide_waves) {

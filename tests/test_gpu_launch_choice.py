@@ -1,5 +1,6 @@
 """What the default launch shape chooses, by nc_sim_last_launch, and that any
 other shape is launched as it was given."""
+import numpy as np
 import pytest
 
 import neurocorrelation_amd as nc
@@ -85,3 +86,34 @@ def test_the_tuner_times_the_form_of_the_activity_it_has():
     sim.tune_list([dict(waves_per_block=2), {}], steps_per_trial=16, rounds=1)
     assert sim.last_launch()["waves_per_slice"] == 2
     sim.close()
+
+
+# networks of a slice (the device holds 512 of their workgroups), of a slice
+# with one of 16 among them (256), of 5 slices: a round, a few, many
+@pytest.mark.parametrize("count,n,one,forms", [(500, 64, 0, (1, 1, 1)), (6000, 64, 0, (0, 0, 0)),
+                                               (2500, 64, 1000, (0, 0, 0)), (300, 300, 0, (1, 0, 1))])
+def test_many_small_networks(count, n, one, forms):
+    # a workgroup per network while the rounds they follow one another in are
+    # few; whatever is chosen, a network's state is that of an explicit shape
+    made = [nc.Network.generate(m, W.side_for(m), W.radius_for_degree(20), 1, 20, 0.05, 0.3, 0.2, seed=m + i)
+            for i in range(4) for m in (n, one) if m]
+    drive = W.drive_spec(dict(n_inputs=6, n_groups=2, n_correlated=2, period=200, p0=0.05, amp_corr=1.0,
+                              amp_ind=1.0), seed=1)
+    nets = [made[i % len(made)] if not one or i == 7 else made[2 * (i % 4)] for i in range(count)]
+    if one:
+        nets[7] = made[1]
+    states = []
+    for shape in ({}, dict(waves_per_block=2)):
+        sim = nc.Simulation(sum(m.n + 64 for m in nets), sum(m.n_syn for m in nets), count,
+                            max_slots=sum(m.device_size()[1] for m in nets))
+        ids = [sim.add(m, None, drive) for m in nets]
+        sim.set_launch(**shape)
+        out = []
+        for steps, form in zip((50, 1, 50), forms):
+            sim.step(steps)
+            assert sim.last_launch()["networks"] == (0 if shape else form), steps
+            out += [sim.save(ids[i]) for i in (0, 7, count // 2, count - 1)]
+        out += [sim.firings(i, m.n) for i, m in zip(ids, nets)]
+        states.append(out)
+        sim.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*states))
