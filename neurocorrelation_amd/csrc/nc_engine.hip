@@ -2030,36 +2030,58 @@ extern "C" nc_status nc_set_weights(nc_sim* sim, int32_t net_id, uint64_t n, con
   if (n && (!syn || !w)) return fail(NC_ERR_ARG, "null argument");
   for (uint64_t i = 0; i < n; ++i)
     if (syn[i] >= r->S) return fail(NC_ERR_RANGE, "synapse index out of range");
-  // Of a synapse listed more than once the last weight holds: the entries in
-  // order of their synapse, then of the list, and of each the last.
-  std::vector<uint64_t> order(n);
-  std::iota(order.begin(), order.end(), 0ull);
-  std::stable_sort(order.begin(), order.end(), [&](uint64_t a, uint64_t b) { return syn[a] < syn[b]; });
+  // Of a synapse listed more than once the last weight holds.  A short list
+  // goes to the device as slots and weights, sorted by synapse; a longer one as
+  // a table of the network's weights and a bit for each listed (the lines cross
+  // near S / 256).  Of 1.06e6 synapses, ms: 10 000 sorted 0.57, by the table
+  // 0.23; 100 000 6.2, 0.46; all of them in no order 88, 1.0.
   std::vector<uint2> sw;
-  sw.reserve(n);
-  const nc::NetMaps& M = *r->maps;
-  uint32_t t = 0;  // target whose row holds the synapse
-  for (uint64_t i = 0; i < n; ++i) {
-    const uint64_t k = syn[order[i]];
-    if (i + 1 < n && syn[order[i + 1]] == k) continue;
-    if ((uint64_t)M.in_ptr[t + 1] <= k)
-      t = (uint32_t)(std::upper_bound(M.in_ptr.begin() + t, M.in_ptr.end(), (int64_t)k) - M.in_ptr.begin() - 1);
-    const uint32_t p = M.pos_of_id[t];
-    uint32_t bits;
-    memcpy(&bits, &w[order[i]], 4);
-    sw.push_back(make_uint2((uint32_t)r->slot0 + nc_slot_of(M.slice_off[p / 64], p % 64, (uint32_t)(k - M.in_ptr[t])), bits));
+  nc::RawVec<float> table;
+  std::vector<uint32_t> listed;
+  if (n <= r->S / 256) {
+    std::vector<uint64_t> order(n);
+    std::iota(order.begin(), order.end(), 0ull);
+    std::stable_sort(order.begin(), order.end(), [&](uint64_t a, uint64_t b) { return syn[a] < syn[b]; });
+    sw.reserve(n);
+    const nc::NetMaps& M = *r->maps;
+    uint32_t t = 0;  // target whose row holds the synapse
+    for (uint64_t i = 0; i < n; ++i) {
+      const uint64_t k = syn[order[i]];
+      if (i + 1 < n && syn[order[i + 1]] == k) continue;
+      if ((uint64_t)M.in_ptr[t + 1] <= k)
+        t = (uint32_t)(std::upper_bound(M.in_ptr.begin() + t, M.in_ptr.end(), (int64_t)k) - M.in_ptr.begin() - 1);
+      const uint32_t p = M.pos_of_id[t];
+      uint32_t bits;
+      memcpy(&bits, &w[order[i]], 4);
+      sw.push_back(make_uint2((uint32_t)r->slot0 + nc_slot_of(M.slice_off[p / 64], p % 64, (uint32_t)(k - M.in_ptr[t])), bits));
+    }
+  } else {
+    table.resize(r->S);
+    listed.assign((r->S + 31) / 32, 0u);
+    for (uint64_t i = 0; i < n; ++i) {
+      table[syn[i]] = w[i];
+      listed[syn[i] / 32] |= 1u << (syn[i] % 32);
+    }
   }
   NC_HIP(hipSetDevice(sim->device));
   NC_HIP(hipStreamSynchronize(sim->stream));
   st = check_barrier(sim);
   if (st != NC_OK) return st;
   r->whost = r->steps_done + 1;
-  if (sw.empty()) return NC_OK;
-  const void* at = nullptr;
-  st = fetch(sim, sw.data(), sw.size() * sizeof(uint2), &at);
-  if (st != NC_OK) return st;
-  hipLaunchKernelGGL(k_set_weights, dim3((uint32_t)((sw.size() + 255) / 256)), dim3(256), 0, sim->stream, sim->slots,
-                     (const uint2*)at, (uint32_t)sw.size());
+  if (n == 0) return NC_OK;
+  if (!table.empty()) {
+    float* const d_table = (float*)sim->d_stage.p;
+    uint32_t* const d_listed = sim->d_stage.p + r->S;
+    const nc::Segment g[] = {{table.data(), d_table, 4 * r->S}, {listed.data(), d_listed, 4 * listed.size()}};
+    NC_HIP(nc::upload(sim->device, sim->stream, g, 2));
+    hipLaunchKernelGGL(k_write_listed, row_blocks(*r), dim3(256), 0, sim->stream, place_of(sim, *r), d_table, d_listed);
+  } else {
+    const void* at = nullptr;
+    st = fetch(sim, sw.data(), sw.size() * sizeof(uint2), &at);
+    if (st != NC_OK) return st;
+    hipLaunchKernelGGL(k_set_weights, dim3((uint32_t)((sw.size() + 255) / 256)), dim3(256), 0, sim->stream, sim->slots,
+                       (const uint2*)at, (uint32_t)sw.size());
+  }
   NC_HIP(hipGetLastError());
   NC_HIP(hipStreamSynchronize(sim->stream));
   return NC_OK;

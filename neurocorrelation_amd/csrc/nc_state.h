@@ -112,6 +112,16 @@ __global__ __launch_bounds__(256) void k_write_weights(nc_place N, const float* 
     nc_set_weight(&N.slots[r.slot(k)], w[r.row + k]);
 }
 
+// The weights of the synapses whose bits are set.
+__global__ __launch_bounds__(256) void k_write_listed(nc_place N, const float* w, const uint32_t* listed) {
+  nc_row r;
+  if (!nc_row_of(N, blockIdx.x * blockDim.x + threadIdx.x, r)) return;
+  for (uint32_t k = r.sub; k < r.deg; k += NC_ROW_LANES) {
+    const uint32_t i = r.row + k;
+    if ((listed[i >> 5] >> (i & 31u)) & 1u) nc_set_weight(&N.slots[r.slot(k)], w[i]);
+  }
+}
+
 // Listed slots' weights: (slot, weight bits), every slot once.
 __global__ __launch_bounds__(256) void k_set_weights(nc_slot* slots, const uint2* sw, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
