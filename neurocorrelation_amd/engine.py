@@ -12,6 +12,9 @@ from ._lib import LaunchCfg, Params, SimSpec, WiringSpec, check, lib, ptr
 
 NEVER = _lib.NC_NEVER_STEP
 
+# (a function object of its own: ctypes.pythonapi's attributes are every importer's)
+_new_bytes = C.PYFUNCTYPE(C.py_object, C.c_char_p, C.c_ssize_t)(("PyBytes_FromStringAndSize", C.pythonapi))
+
 
 def _cfg_dict(cfg):
     return {f: getattr(cfg, f) for f, _ in LaunchCfg._fields_}
@@ -268,9 +271,7 @@ class Simulation:
         size = C.c_uint64()
         check(lib().nc_sim_save(self._h, net_id, None, 0, C.byref(size)))
         # the call fills a new bytes object in place, before anything else holds it
-        new_bytes = C.pythonapi.PyBytes_FromStringAndSize
-        new_bytes.restype, new_bytes.argtypes = C.py_object, [C.c_char_p, C.c_ssize_t]
-        data = new_bytes(None, size.value)
+        data = _new_bytes(None, size.value)
         check(lib().nc_sim_save(self._h, net_id, C.cast(C.c_char_p(data), C.c_void_p), size.value, C.byref(size)))
         return data
 
