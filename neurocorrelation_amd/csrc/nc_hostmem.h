@@ -9,8 +9,8 @@
 #include <sys/mman.h>
 
 #include <algorithm>
+#include <exception>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -29,8 +29,9 @@ void split_bytes(size_t bytes, F f) {
   size_t at = 0;
   try {
     for (unsigned t = 0; t + 1 < nt && at + part < bytes; ++t, at += part) th.emplace_back(f, at, at + part);
-  } catch (const std::system_error&) {
-    // no thread to be had: the rest is this one's
+  } catch (const std::exception&) {
+    // no thread, or no memory for one, to be had: the rest is this one's (the
+    // threads started have to be joined whatever it was)
   }
   f(at, bytes);
   for (auto& t : th) t.join();

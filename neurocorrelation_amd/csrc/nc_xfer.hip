@@ -134,8 +134,9 @@ hipError_t move(int device, hipStream_t st, const Segment* seg, size_t n_seg, bo
       {chunks.size(), kThreads, std::max<size_t>(1, std::thread::hardware_concurrency())});
   try {
     for (unsigned t = 1; t < nt; ++t) th.emplace_back(work, t);
-  } catch (const std::system_error&) {
-    // no thread to be had: the others move all chunks
+  } catch (const std::exception&) {
+    // no thread, or no memory for one, to be had: the others move all chunks
+    // (those started have to be joined whatever it was)
   }
   work(0);
   for (auto& t : th) t.join();
