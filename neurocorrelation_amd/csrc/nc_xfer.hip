@@ -77,6 +77,17 @@ void give_back(PinnedChunks* b) {
   delete b;
 }
 
+// Without a pinned buffer.
+hipError_t move_direct(hipStream_t st, const Segment* seg, size_t n_seg, bool to_host) {
+  hipError_t e = hipSuccess;
+  for (size_t i = 0; i < n_seg && e == hipSuccess; ++i)
+    if (seg[i].bytes)
+      e = to_host ? hipMemcpyAsync(seg[i].host, seg[i].dev, seg[i].bytes, hipMemcpyDeviceToHost, st)
+                  : hipMemcpyAsync(seg[i].dev, seg[i].host, seg[i].bytes, hipMemcpyHostToDevice, st);
+  const hipError_t w = hipStreamSynchronize(st);
+  return e == hipSuccess ? w : e;
+}
+
 hipError_t move(int device, hipStream_t st, const Segment* seg, size_t n_seg, bool to_host) {
   std::vector<Segment> chunks;
   for (size_t i = 0; i < n_seg; ++i)
@@ -89,7 +100,12 @@ hipError_t move(int device, hipStream_t st, const Segment* seg, size_t n_seg, bo
   th.reserve(kThreads);
   PinnedChunks* b = nullptr;
   hipError_t e = take(device, &b);
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess) {
+    // the host has no more memory to pin, which the copies themselves can do
+    // without
+    (void)hipGetLastError();
+    return move_direct(st, seg, n_seg, to_host);
+  }
   if (total <= kChunk) {
     // one wait for all of it
     size_t at = 0;

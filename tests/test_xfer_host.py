@@ -127,3 +127,26 @@ int main() {
   return 0;
 }
 """ % (a, b))
+
+
+@pytest.mark.parametrize("what", ["h_no_pinned", "h_no_events"])
+def test_transfers_without_memory_to_pin(tmp_path, what):
+    run(tmp_path, r"""
+int main() {
+  %s = 1;
+  const size_t n[3] = {5u << 20, 0, 77};
+  for (int down = 0; down < 2; ++down) {
+    std::vector<char> host[3], dev[3];
+    Segment seg[3];
+    for (int i = 0; i < 3; ++i) {
+      host[i] = pattern(n[i], down ? 0 : i + 1), dev[i] = pattern(n[i], down ? i + 1 : 0);
+      seg[i] = Segment{host[i].data(), dev[i].data(), n[i]};
+    }
+    CHECK((down ? download(0, nullptr, seg, 3) : upload(0, nullptr, seg, 3)) == hipSuccess);
+    for (int i = 0; i < 3; ++i) CHECK(host[i] == pattern(n[i], i + 1) && dev[i] == host[i]);
+    CHECK(hipGetLastError() == hipSuccess);
+    CHECK(h_pinned == 0 && h_events == 0);
+  }
+  return 0;
+}
+""" % what)
