@@ -78,7 +78,8 @@ nc_status nc_net_generate(const nc_wiring_spec* spec, nc_net** out);
  * grid and the rows of sources within the radius, sorted by source id, then
  * the per-synapse delays, weights and sign classes (spec->n_threads is
  * ignored).  Also replaces Neuron::makeConnections' all-pairs scan
- * (src/NeuCor.cpp:418-444). */
+ * (src/NeuCor.cpp:418-444).  A process that has no simulation keeps one stream
+ * and 8 MiB of pinned memory for its next call. */
 nc_status nc_net_generate_device(const nc_wiring_spec* spec, int32_t device, nc_net** out);
 
 /* Replaces NeuCor::createNeuron / NeuCor::createSynapse

@@ -71,7 +71,8 @@ hipError_t upload(int device, hipStream_t st, const Segment* seg, size_t n_seg);
 hipError_t stream_take(int device, hipStream_t* out);
 void stream_give(int device, hipStream_t st);
 // A simulation came (+1) or went (-1): the last one's end frees the pinned
-// memory and the streams kept between calls.
+// memory and the streams kept between calls.  Without one, wiring keeps a
+// single buffer (8 MiB) and a single stream.
 void xfer_user(int change);
 #endif
 

@@ -14,6 +14,7 @@
 #include <atomic>
 #include <mutex>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "nc_internal.h"
@@ -25,7 +26,9 @@ namespace {
 // 512 KiB 1.15, 1 MiB 0.82, 2 MiB 0.70, whatever the threads from four on.
 constexpr size_t kChunk = 2u << 20;
 constexpr unsigned kThreads = 4;
-constexpr size_t kIdleMost = 6;  // pinned buffers kept between calls (a server builds on four threads)
+// Pinned buffers and streams kept between calls: while simulations live (a
+// server builds on four threads), and for programs that only wire networks.
+constexpr size_t kIdleMost = 6, kIdleAlone = 1;
 
 struct PinnedChunks {
   int device = 0;
@@ -38,20 +41,40 @@ struct PinnedChunks {
   }
 };
 
+// Idle things of a device each, no allocation to keep one.
+template <class T>
+struct Idle {
+  struct Item {
+    int device;
+    T x;
+  } item[kIdleMost] = {};
+  size_t n = 0;
+  bool take(int device, T* out) {
+    for (size_t i = 0; i < n; ++i)
+      if (item[i].device == device) {
+        *out = item[i].x;
+        item[i] = item[--n];
+        return true;
+      }
+    return false;
+  }
+  bool give(int device, T x, size_t most) {
+    if (n >= most) return false;
+    item[n++] = Item{device, x};
+    return true;
+  }
+};
+
 std::mutex g_mu;
-std::vector<PinnedChunks*> g_idle;
-std::vector<std::pair<int, hipStream_t>> g_streams;  // idle ones, with their device
+Idle<PinnedChunks*> g_idle;
+Idle<hipStream_t> g_streams;
 unsigned g_users = 0;  // simulations alive
+size_t idle_most() { return g_users ? kIdleMost : kIdleAlone; }
 
 hipError_t take(int device, PinnedChunks** out) {
   {
     std::lock_guard<std::mutex> g(g_mu);
-    for (size_t i = 0; i < g_idle.size(); ++i)
-      if (g_idle[i]->device == device) {
-        *out = g_idle[i];
-        g_idle.erase(g_idle.begin() + i);
-        return hipSuccess;
-      }
+    if (g_idle.take(device, out)) return hipSuccess;
   }
   PinnedChunks* b = new PinnedChunks();
   b->device = device;
@@ -69,10 +92,7 @@ hipError_t take(int device, PinnedChunks** out) {
 void give_back(PinnedChunks* b) {
   {
     std::lock_guard<std::mutex> g(g_mu);
-    if (g_idle.size() < kIdleMost) {
-      g_idle.push_back(b);
-      return;
-    }
+    if (g_idle.give(b->device, b, idle_most())) return;
   }
   delete b;
 }
@@ -173,12 +193,7 @@ hipError_t upload(int device, hipStream_t st, const Segment* seg, size_t n_seg) 
 hipError_t stream_take(int device, hipStream_t* out) {
   {
     std::lock_guard<std::mutex> g(g_mu);
-    for (size_t i = 0; i < g_streams.size(); ++i)
-      if (g_streams[i].first == device) {
-        *out = g_streams[i].second;
-        g_streams.erase(g_streams.begin() + i);
-        return hipSuccess;
-      }
+    if (g_streams.take(device, out)) return hipSuccess;
   }
   return hipStreamCreateWithFlags(out, hipStreamNonBlocking);
 }
@@ -187,27 +202,24 @@ void stream_give(int device, hipStream_t st) {
   (void)hipStreamSynchronize(st);
   {
     std::lock_guard<std::mutex> g(g_mu);
-    if (g_streams.size() < kIdleMost) {
-      g_streams.push_back({device, st});
-      return;
-    }
+    if (g_streams.give(device, st, idle_most())) return;
   }
   (void)hipStreamDestroy(st);
 }
 
 void xfer_user(int change) {
-  std::vector<PinnedChunks*> gone;
-  std::vector<std::pair<int, hipStream_t>> streams;
+  Idle<PinnedChunks*> gone;
+  Idle<hipStream_t> streams;
   {
     std::lock_guard<std::mutex> g(g_mu);
     g_users += (unsigned)change;
     if (g_users == 0) {
-      gone.swap(g_idle);
-      streams.swap(g_streams);
+      std::swap(gone, g_idle);
+      std::swap(streams, g_streams);
     }
   }
-  for (PinnedChunks* b : gone) delete b;
-  for (auto& s : streams) (void)hipStreamDestroy(s.second);
+  for (size_t i = 0; i < gone.n; ++i) delete gone.item[i].x;
+  for (size_t i = 0; i < streams.n; ++i) (void)hipStreamDestroy(streams.item[i].x);
 }
 
 }  // namespace nc

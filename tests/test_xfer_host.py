@@ -150,3 +150,58 @@ int main() {
   return 0;
 }
 """ % what)
+
+
+def test_what_is_kept_between_calls(tmp_path):
+    # several threads wire at once, with and without a simulation alive
+    run(tmp_path, r"""
+static void wire() {
+  hipStream_t st = nullptr;
+  if (stream_take(0, &st) != hipSuccess) abort();
+  std::vector<char> host(5 << 20), dev = pattern(5 << 20, 3);
+  const Segment seg{host.data(), dev.data(), host.size()};
+  if (download(0, st, &seg, 1) != hipSuccess || host != dev) abort();
+  stream_give(0, st);
+}
+static void wires(int n) {
+  std::vector<std::thread> th;
+  for (int i = 0; i < n; ++i) th.emplace_back([] { for (int k = 0; k < 5; ++k) wire(); });
+  for (auto& t : th) t.join();
+}
+int main() {
+  wires(8);
+  CHECK(h_pinned <= 1 && h_streams <= 1 && h_events <= 4);
+  const int calls = h_pin_calls;
+  for (int i = 0; i < 5; ++i) wire();
+  CHECK(h_pin_calls <= calls + 1);  // (one kept is used again)
+  xfer_user(1);
+  wires(8);
+  CHECK(h_pinned <= 6 && h_streams <= 6);
+  xfer_user(1), xfer_user(-1);
+  CHECK(h_pinned >= 1 && h_streams >= 1);
+  hipStream_t st = nullptr;
+  CHECK(stream_take(0, &st) == hipSuccess);
+  xfer_user(-1);
+  CHECK(h_pinned == 0 && h_events == 0 && h_streams == 1);
+  stream_give(0, st);  // after the last simulation went
+  wires(8);
+  CHECK(h_pinned <= 1 && h_streams <= 1);
+  // another device's are not handed out
+  hipStream_t a = nullptr, b = nullptr;
+  CHECK(stream_take(1, &a) == hipSuccess && stream_take(0, &b) == hipSuccess && a != b);
+  stream_give(1, a), stream_give(0, b);
+  CHECK(h_streams <= 1);
+  xfer_user(1), xfer_user(-1);
+  CHECK(h_pinned == 0 && h_events == 0 && h_streams == 0);
+  // and keeping one allocates nothing
+  xfer_user(1);
+  wire();
+  CHECK(stream_take(0, &a) == hipSuccess && stream_take(0, &b) == hipSuccess);
+  t_left = 0;
+  stream_give(0, a), stream_give(0, b);
+  t_left = -1;
+  xfer_user(-1);
+  CHECK(h_pinned == 0 && h_streams == 0);
+  return 0;
+}
+""")
