@@ -179,7 +179,8 @@ nc_status nc_net_prepare(nc_net* net);
 void nc_sim_destroy(nc_sim* sim);
 
 /* Bytes a network of this size takes on the device, and the free HBM the
- * admission policy sees (hipMemGetInfo). */
+ * admission policy sees (hipMemGetInfo).  A simulation of at most a quarter of
+ * the free memory takes 512 bytes more per neuron (larger arrival buckets). */
 nc_status nc_sim_footprint(uint64_t n_neurons, uint64_t n_syn, uint64_t* bytes);
 nc_status nc_sim_free_bytes(const nc_sim* sim, uint64_t* free_bytes);
 

@@ -471,7 +471,8 @@ struct nc_sim {
   uint32_t *pend0 = nullptr, *pend1 = nullptr;
   uint2* pend_cnt = nullptr;
   uint32_t* bcnt = nullptr;        // per slice: NC_NB arrival-bucket counts
-  uint2* bent = nullptr;           // per slice: NC_NB buckets of NC_BCAP entries
+  uint2* bent = nullptr;           // per slice: NC_NB buckets of bcap entries
+  uint32_t bcap = NC_BCAP_MOST;
   uint4* acache = nullptr;         // active-slot cache: one 16-byte entry per position
   uint32_t *id_pos = nullptr, *id_row = nullptr;  // per network, at its positions: neuron id -> local position, first synapse
   uint32_t* slice_moff = nullptr;  // per slice: first active-mask word
@@ -815,7 +816,7 @@ extern "C" nc_status nc_sim_footprint(uint64_t n_neurons, uint64_t n_syn, uint64
            + P * sizeof(uint4)                             // active-slot cache
            + Q * (8 + 4 + 4 + sizeof(nc_slice_rec))       // pend_cnt, slice_off, slice_moff, active
            + (Q + NC_FLISTS * 8) * NC_FSPLIT * 16          // fired lists
-           + Q * NC_NB * (4ull + 8ull * NC_BCAP) + Q * 4     // arrival buckets, slice mask offsets
+           + Q * NC_NB * (4ull + 8ull * NC_BCAP_LEAST) + Q * 4  // arrival buckets, slice mask offsets
            + slots * (sizeof(nc_slot) + 8) + mwords * 4    // slot records, pending lists, active masks
            + (n_syn + 64) * sizeof(nc_edge)                // out-edges
            + (Q + 2) * NC_NCTR * 8;                        // counters
@@ -888,29 +889,53 @@ extern "C" nc_status nc_sim_create(const nc_sim_spec* spec, nc_sim** out) try {
   sim->max_mwords = sim->max_slots / 32 + 64 * Q;
   if (st == NC_OK) {
     // One allocation, cut into the arrays: first those that start cleared.
-    Arena R;
     sim->ctr_rows = Q + 2;
-    R.want(&sim->amask, sim->max_mwords), R.want(&sim->asum, P), R.want(&sim->ndw, P);
-    R.want(&sim->forced_in, P / 32), R.want(&sim->forced_bg, P / 32);
-    R.want(&sim->fired, (Q + NC_FLISTS * 8ull) * NC_FSPLIT), R.want(&sim->fired_cnt, 2ull * NC_FLISTS * NC_FCNT_STRIDE);
-    R.want(&sim->pend_cnt, Q), R.want(&sim->bcnt, Q * NC_NB), R.want(&sim->acache, P);
-    R.want(&sim->raster_cnt, 16), R.want(&sim->ctr, sim->ctr_rows * NC_NCTR);
-    // word 0: chunk offset; word 32: grid-barrier arrivals of the call;
-    // word 128: zero, the group-spike-train word read when there are no
-    // groups; word 192: a checkpoint's faults (nc_sim_restore); words
-    // 200-203: a result's digest and firings (sim_result); word 208: workgroups
-    // done of a read (nc_done)
-    R.want(&sim->d_chunk_off, 256);
-    // one more, never written: the (never live) network of hole records
-    R.want(&sim->d_nets, sim->max_nets + 1ull);
-    const uint64_t cleared = R.bytes;
-    R.want(&sim->slots, sim->max_slots), R.want(&sim->edges, sim->max_out);
-    R.want(&sim->pend0, sim->max_slots), R.want(&sim->pend1, sim->max_slots), R.want(&sim->bent, Q * NC_NB * NC_BCAP);
-    R.want(&sim->V, P), R.want(&sim->last_fire, P), R.want(&sim->firings, P), R.want(&sim->nid, P);
-    R.want(&sim->out_row, P), R.want(&sim->id_pos, P), R.want(&sim->id_row, P);
-    R.want(&sim->slice_off, Q), R.want(&sim->slice_moff, Q), R.want(&sim->active, Q);
-    R.want(&sim->net_recs, sim->max_nets), R.want(&sim->raster, 2ull * sim->raster_cap);
-    H(hipMalloc(&sim->arena, R.bytes), "hipMalloc");
+    uint64_t cleared = 0;
+    auto cut = [&]() {
+      Arena R;
+      R.want(&sim->amask, sim->max_mwords), R.want(&sim->asum, P), R.want(&sim->ndw, P);
+      R.want(&sim->forced_in, P / 32), R.want(&sim->forced_bg, P / 32);
+      R.want(&sim->fired, (Q + NC_FLISTS * 8ull) * NC_FSPLIT), R.want(&sim->fired_cnt, 2ull * NC_FLISTS * NC_FCNT_STRIDE);
+      R.want(&sim->pend_cnt, Q), R.want(&sim->bcnt, Q * NC_NB), R.want(&sim->acache, P);
+      R.want(&sim->raster_cnt, 16), R.want(&sim->ctr, sim->ctr_rows * NC_NCTR);
+      // word 0: chunk offset; word 32: grid-barrier arrivals of the call;
+      // word 128: zero, the group-spike-train word read when there are no
+      // groups; word 192: a checkpoint's faults (nc_sim_restore); words
+      // 200-203: a result's digest and firings (sim_result); word 208: workgroups
+      // done of a read (nc_done)
+      R.want(&sim->d_chunk_off, 256);
+      // one more, never written: the (never live) network of hole records
+      R.want(&sim->d_nets, sim->max_nets + 1ull);
+      cleared = R.bytes;
+      R.want(&sim->slots, sim->max_slots), R.want(&sim->edges, sim->max_out);
+      R.want(&sim->pend0, sim->max_slots), R.want(&sim->pend1, sim->max_slots);
+      R.want(&sim->bent, Q * NC_NB * sim->bcap);
+      R.want(&sim->V, P), R.want(&sim->last_fire, P), R.want(&sim->firings, P), R.want(&sim->nid, P);
+      R.want(&sim->out_row, P), R.want(&sim->id_pos, P), R.want(&sim->id_row, P);
+      R.want(&sim->slice_off, Q), R.want(&sim->slice_moff, Q), R.want(&sim->active, Q);
+      R.want(&sim->net_recs, sim->max_nets), R.want(&sim->raster, 2ull * sim->raster_cap);
+      return R;
+    };
+    // Arrival buckets of 128 entries where the simulation is small beside the
+    // free memory (a quarter; below 1 GiB where there is room), else of 64:
+    // which sizes fit does not depend on the larger ones.
+    Arena R = cut();
+    auto fewer = [&]() {
+      sim->bcap = NC_BCAP_LEAST;
+      R = cut();
+    };
+    if (R.bytes >= (1ull << 30)) {
+      size_t free_b = 0, total = 0;
+      H(hipMemGetInfo(&free_b, &total), "hipMemGetInfo");
+      if (R.bytes > free_b / 4) fewer();
+    }
+    hipError_t e = hipMalloc(&sim->arena, R.bytes);
+    if (e == hipErrorOutOfMemory && sim->bcap != NC_BCAP_LEAST) {
+      (void)hipGetLastError();
+      fewer();
+      e = hipMalloc(&sim->arena, R.bytes);
+    }
+    H(e, "hipMalloc");
     if (st == NC_OK) {
       R.place(sim->arena);
       H(hipMemsetAsync(sim->arena, 0, cleared, sim->stream), "memset");
@@ -1324,10 +1349,29 @@ Form step_form(const nc_sim* sim, uint32_t steps) {
   return f;
 }
 
+// The step kernels of a bucket capacity: by 1, 2, 4 and 8 waves per workgroup,
+// and by 1, 2 and 4 waves per slice.
+struct StepKernels {
+  const void *neuron[4], *staged[4], *fanout[4], *step[4], *wide[3];
+};
+template <uint32_t BC>
+StepKernels step_kernels() {
+  return {{(const void*)k_neuron<1, false, BC>, (const void*)k_neuron<2, false, BC>,
+           (const void*)k_neuron<4, false, BC>, (const void*)k_neuron<8, false, BC>},
+          {(const void*)k_neuron<1, true, BC>, (const void*)k_neuron<2, true, BC>, (const void*)k_neuron<4, true, BC>,
+           (const void*)k_neuron<8, true, BC>},
+          {(const void*)k_fanout<1, BC>, (const void*)k_fanout<2, BC>, (const void*)k_fanout<4, BC>,
+           (const void*)k_fanout<8, BC>},
+          {(const void*)k_step<1, BC>, (const void*)k_step<2, BC>, (const void*)k_step<4, BC>,
+           (const void*)k_step<8, BC>},
+          {(const void*)k_neuron_wide<1, BC>, (const void*)k_neuron_wide<2, BC>, (const void*)k_neuron_wide<4, BC>}};
+}
+
 // Steps c0 .. c0 + len - 1 of a call in the workgroup-per-network form.
 template <int NSL, int W>
 nc_status launch_networks(nc_sim* sim, const nc_step_args& a, uint32_t c0, uint32_t len) {
-  const void* fn = (const void*)k_net_steps<NSL, W>;
+  const void* fn = sim->bcap == NC_BCAP_MOST ? (const void*)k_net_steps<NSL, W, NC_BCAP_MOST>
+                                             : (const void*)k_net_steps<NSL, W, NC_BCAP_LEAST>;
   const uint32_t lds = sizeof(nc_gsh<NSL, W, true>);
   const nc_net_rec* nets = sim->net_recs;
   const uint32_t* ev_step = sim->d_ev_step.p;
@@ -1557,40 +1601,23 @@ extern "C" nc_status nc_sim_step(nc_sim* sim, uint32_t n_steps) try {
   const uint32_t lds = a.tabs_in_lds ? (uint32_t)a.len_pre * 4 : 0u;
   const void* fn_neuron = nullptr;
   const void* fn_fanout = nullptr;
-  const bool tabs = a.tabs_in_lds != 0;
-  auto pick = [&](const void* plain, const void* staged, const void* fan) {
-    fn_neuron = tabs ? staged : plain;
-    fn_fanout = fan;
-  };
-  switch (wpb) {
-    case 1: pick((const void*)k_neuron<1, false>, (const void*)k_neuron<1, true>, (const void*)k_fanout<1>); break;
-    case 2: pick((const void*)k_neuron<2, false>, (const void*)k_neuron<2, true>, (const void*)k_fanout<2>); break;
-    case 8: pick((const void*)k_neuron<8, false>, (const void*)k_neuron<8, true>, (const void*)k_fanout<8>); break;
-    default: pick((const void*)k_neuron<4, false>, (const void*)k_neuron<4, true>, (const void*)k_fanout<4>); break;
-  }
+  const StepKernels K = sim->bcap == NC_BCAP_MOST ? step_kernels<NC_BCAP_MOST>() : step_kernels<NC_BCAP_LEAST>();
+  const int by_waves = wpb == 1 ? 0 : wpb == 2 ? 1 : wpb == 8 ? 3 : 2;
+  fn_neuron = (a.tabs_in_lds ? K.staged : K.neuron)[by_waves];
+  fn_fanout = K.fanout[by_waves];
   // The persistent form: one launch per step of a grid the device holds at
   // once (every workgroup resident, so that the grid barrier can end).
   const void* fn_step = nullptr;
   uint32_t pgrid = 0;
   uint32_t* const bar = sim->d_chunk_off + 32;
   if (sim->cfg.persistent) {
-    switch (wpb) {
-      case 1: fn_step = (const void*)k_step<1>; break;
-      case 2: fn_step = (const void*)k_step<2>; break;
-      case 8: fn_step = (const void*)k_step<8>; break;
-      default: fn_step = (const void*)k_step<4>; break;
-    }
+    fn_step = K.step[by_waves];
     int per_cu = 0;
     NC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn_step, (int)(64 * wpb), lds));
     pgrid = std::min<uint32_t>((uint32_t)std::max(per_cu, 0) * (uint32_t)sim->cus, std::max(grid, fan_grid));
     if (pgrid * wpb < NC_FLISTS) return fail(NC_ERR_STATE, "the device holds too few workgroups for the persistent form");
   }
-  switch (form.wide_waves) {
-    case 1: fn_neuron = (const void*)k_neuron_wide<1>; break;
-    case 2: fn_neuron = (const void*)k_neuron_wide<2>; break;
-    case 4: fn_neuron = (const void*)k_neuron_wide<4>; break;
-    default: break;
-  }
+  if (form.wide_waves) fn_neuron = K.wide[form.wide_waves == 4 ? 2 : form.wide_waves - 1];
   const uint32_t n_grid = form.wide_waves ? a.n_active_slices : grid;
   const uint32_t n_block = 64 * (form.wide_waves ? form.wide_waves : wpb);
   sim->calls = sim->calls % 0xFFFFFFFFu + 1u;
@@ -2368,7 +2395,7 @@ nc_status state_save(nc_sim* sim, StateCopy* c) {
       {sim->pend1, sim->max_slots * 4},
       {sim->pend_cnt, Q * sizeof(uint2)},
       {sim->bcnt, Q * NC_NB * 4ull},
-      {sim->bent, Q * NC_NB * NC_BCAP * sizeof(uint2)},
+      {sim->bent, Q * NC_NB * sim->bcap * sizeof(uint2)},
       {sim->acache, P * sizeof(uint4)},
       {sim->fired, (Q + NC_FLISTS * 8ull) * NC_FSPLIT * sizeof(uint4)},
       {sim->fired_cnt, 2ull * NC_FLISTS * NC_FCNT_STRIDE * 4},

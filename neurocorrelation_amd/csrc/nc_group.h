@@ -127,7 +127,7 @@ struct nc_glane {
 // owner lane's group-spike-train word; f_in, f_bg: its host-scheduled fires;
 // rec_i, soff0, b_n0: the slice's place among the active ones, its first slot
 // and its bucket's count (not resident).
-template <int NSL, int W, bool RES>
+template <int NSL, int W, bool RES, uint32_t BC>
 __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL, W, RES>& sh, const nc_netdesc& nd,
                                               uint32_t nsl, uint32_t q0, uint32_t wv, uint32_t lane, int32_t s,
                                               int32_t ci, nc_glane& L, uint32_t sm, uint32_t* mrow,
@@ -152,10 +152,10 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
   // is 0 and which does not use it.
   uint32_t b_n = b_n0;
   if constexpr (RES) b_n = sh.bcnt[xs][(uint32_t)s & (NC_NB - 1u)];
-  const uint32_t b_take = min(b_n, NC_BCAP);
+  const uint32_t b_take = min(b_n, BC);
   // (No branch around the reads: an entry whose record is not needed reads its
   // own place again.  They are first used after the fire.)
-  auto place = [&](uint32_t i) { return a.bent + (bi * NC_BCAP + min(i, NC_BCAP - 1u)); };
+  auto place = [&](uint32_t i) { return a.bent + (bi * BC + min(i, BC - 1u)); };
   auto entry_of = [&](uint32_t i, uint2 be) {
     nc_gent g;
     const uint2* const own = place(i);
@@ -193,9 +193,9 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
   g0.on = false;
   // resident counts are at hand; else the entries are read beside the count
   if constexpr (kOne) g0 = entry_of(sub * 64u + lane, be0);
-  else if (sub * 64u < (RES ? b_take : NC_BCAP)) g0 = entry(sub * 64u + lane);
+  else if (sub * 64u < (RES ? b_take : BC)) g0 = entry(sub * 64u + lane);
 
-  static_assert(NC_BCAP == 128u, "at most two entries per lane of one wave");
+  static_assert(BC <= 128u, "at most two entries per lane of one wave");
   nc_gent g1;
   g1.on = false;
   if (RES && nsub == 1u && b_take > 64u) g1 = entry(64u + lane);
@@ -550,7 +550,7 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
         const nc_slot x = a.slots[ed.j];
         const uint32_t d = ed.tq_d & 0xffu, tq = ed.tq_d >> 8;
         const int32_t arr = s + (int32_t)d, prev = x.arr_inh >> 1;
-        uint32_t at = NC_BCAP;
+        uint32_t at = BC;
         if (d <= NC_NB) at = atomicAdd(&sh.bcnt[tq - q0][(uint32_t)arr & (NC_NB - 1u)], 1u);
         nc_slot n;
         n.w = x.w;
@@ -559,8 +559,8 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
         n.arr_inh = arr * 2 + (x.arr_inh & 1);
         a.slots[ed.j] = n;
         a.edges[e].arr = arr;
-        if (at < NC_BCAP) {
-          a.bent[((size_t)tq * NC_NB + ((uint32_t)arr & (NC_NB - 1u))) * NC_BCAP + at] =
+        if (at < BC) {
+          a.bent[((size_t)tq * NC_NB + ((uint32_t)arr & (NC_NB - 1u))) * BC + at] =
               make_uint2(ed.rel | ((d - 1u) << 24) | ((uint32_t)(x.arr_inh & 1) << 31), __float_as_uint(x.w));
         } else {
           const uint32_t plist = ((uint32_t)arr >> NC_PEND_LOG_W) & 1u;
@@ -609,7 +609,7 @@ __device__ __forceinline__ void nc_group_step(const nc_step_args& a, nc_gsh<NSL,
 }
 
 // The neuron phase of one step, a workgroup of W waves per active slice.
-template <int W>
+template <int W, uint32_t BC>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6))) void k_neuron_wide(nc_step_args a) {
   __shared__ nc_gsh<1, W, false> sh;
   const uint32_t lane = threadIdx.x & 63u;
@@ -664,7 +664,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6))) voi
   // No barrier: before the step's first one, only wave 0 reads these (the
   // other waves have rec.slot_off itself).
   const uint32_t pend_n = (((uint32_t)s >> NC_PEND_LOG_W) & 1u) ? pc.y : pc.x;
-  nc_group_step<1, W, false>(a, sh, nd, 1u, q, wv, lane, s, ci, L, sm, a.amask + rec.mask_off + lane, pend_n, gword,
+  nc_group_step<1, W, false, BC>(a, sh, nd, 1u, q, wv, lane, s, ci, L, sm, a.amask + rec.mask_off + lane, pend_n, gword,
                              f_in, f_bg, a.t_pre, a.t_post, i, rec.slot_off, b_n);
   if (wv == 0 && (L.nw.x & NC_DEG_VALID)) {
     if (__float_as_uint(L.V) != __float_as_uint(L.V_in)) a.V[L.pos] = L.V;
@@ -680,7 +680,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(6))) voi
 // call; a network's are events ev0 .. ev1 - 1 of its record, ascending (in one
 // list by step for all networks every owner wave went through every network's:
 // 256 networks of 300 neurons with 15 events a step each 114 us a step, 19 so).
-template <int NSL, int W>
+template <int NSL, int W, uint32_t BC>
 __global__ __launch_bounds__(64 * W) void k_net_steps(nc_step_args a, const nc_net_rec* nets, const uint32_t* ev_step,
                                                       uint32_t c0, uint32_t len) {
   extern __shared__ __align__(16) unsigned char sh_raw[];
@@ -759,7 +759,7 @@ __global__ __launch_bounds__(64 * W) void k_net_steps(nc_step_args a, const nc_n
       }
     }
     const uint32_t pend_n = owner ? sh.pcnt[wv][((uint32_t)s >> NC_PEND_LOG_W) & 1u] : 0u;
-    nc_group_step<NSL, W, true>(a, sh, nd, nsl, q0, wv, lane, s, (int32_t)c, L, 0u, mrow, pend_n, gword, f_in, f_bg,
+    nc_group_step<NSL, W, true, BC>(a, sh, nd, nsl, q0, wv, lane, s, (int32_t)c, L, 0u, mrow, pend_n, gword, f_in, f_bg,
                                 sh.tpre, sh.tpost, 0u, 0u, 0u);
   }
   __syncthreads();

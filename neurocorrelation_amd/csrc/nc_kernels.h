@@ -41,9 +41,12 @@
 // step s holds no arrival before s nor past s + 255 (delays are 1..255).
 #define NC_PEND_LOG_W 4
 // Spikes with delays up to NC_NB steps go to an arrival bucket instead: per
-// slice, one bucket per arrival step modulo NC_NB, of up to NC_BCAP entries
-// (two per neuron: at 50 synapses per neuron and a quarter of the neurons
-// firing, a slice has 107 arrivals in a step)
+// slice, one bucket per arrival step modulo NC_NB, of up to BC entries (128, two
+// per neuron: at 50 synapses per neuron and a quarter of the neurons firing, a
+// slice has 107 arrivals in a step; or, where the 512 bytes per neuron that the
+// second 64 take are dear, 64: the kernels that touch buckets are made for
+// both, as a capacity read at run time took k_neuron two spilled registers and
+// plain-1m 0.4 us a step)
 // (slot - first slot of the slice | (delay - 1) << 24 | sign class << 31,
 // weight at the fire, whose product with 10.4 is the latched
 // depolarisation).  Fan-out takes
@@ -52,7 +55,8 @@
 // contribute -- and empties it.  A spike that finds its bucket full, or
 // whose delay exceeds NC_NB, goes to the pending list of its window.
 #define NC_NB 64u
-#define NC_BCAP 128u
+#define NC_BCAP_MOST 128u
+#define NC_BCAP_LEAST 64u
 // Slices with fired lanes go to one of NC_FLISTS lists (by wave index), so
 // that the appends of a step spread over that many counters.
 #define NC_FLISTS 64
@@ -185,8 +189,8 @@ struct nc_step_args {
   uint32_t* pend0;         // pending list 0 of every slice, at its slot range
   uint32_t* pend1;         // pending list 1
   uint2* pend_cnt;         // per slice: entries in pending list 0, in list 1
-  uint32_t* bcnt;          // per slice: NC_NB arrival-bucket counts (beyond NC_BCAP: the rest overflowed)
-  uint2* bent;             // per slice: NC_NB buckets of NC_BCAP entries {slot | delay | class, weight bits}
+  uint32_t* bcnt;          // per slice: NC_NB arrival-bucket counts (beyond BC: the rest overflowed)
+  uint2* bent;             // per slice: NC_NB buckets of BC entries {slot | delay | class, weight bits}
   uint4* acache;           // per position: (depol bits, arrival) of its first two active slots
   const uint32_t* ev_pos;  // host events of this step
   const uint8_t* ev_kind;
@@ -477,7 +481,7 @@ __global__ void k_drive(nc_step_args a) {
 // Neuron::run (src/NeuCor.cpp:619-641) for the 64 neurons of active-slice
 // record `wave` at step ci of the call (one wave of a workgroup of WPB waves;
 // blk is the workgroup's counter row).
-template <int WPB>
+template <int WPB, uint32_t BC>
 __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t blk, uint32_t wave, int32_t ci,
                                                 const float* tpre) {
   const uint32_t lane = threadIdx.x & 63;
@@ -508,7 +512,7 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
   const int32_t s = nd.base_step + ci + 1;
   const size_t bi = (size_t)q * NC_NB + ((uint32_t)s & (NC_NB - 1u));
   uint32_t b_n = a.bcnt[bi];
-  const uint2 be = a.bent[bi * NC_BCAP + lane];
+  const uint2 be = a.bent[bi * BC + lane];
   const uint32_t gword = a.gfire[(size_t)((uint32_t)ci & (NC_GRING - 1u)) * a.gwords +
                                  ((nw.x & NC_DEG_INPUT) ? (nw.y >> 5) : 0u)];
   const uint32_t plist = ((uint32_t)s >> NC_PEND_LOG_W) & 1u;
@@ -537,7 +541,7 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
   const uint32_t G = nmw <= 32 ? 1u : (nmw + 31) >> 5;  // mask words per summary bit
   uint32_t* const mrow = a.amask + rec.mask_off + lane;
   // The bucket's entries are taken up after the fire.
-  const uint32_t b_take = b_n < NC_BCAP ? b_n : NC_BCAP;
+  const uint32_t b_take = b_n < BC ? b_n : BC;
   // The weight now of the bucket entry this lane holds, read at its slot
   // record with the mask words instead of after the fire, when the target
   // fired since the source did (as of the previous step) and no host write
@@ -557,7 +561,7 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
       e_stale ? &a.slots[nc_slot_of(rec.slot_off, e_tl,
                                     ((e_rel >> (6 + NC_CHUNK_LOG)) << NC_CHUNK_LOG) | (e_rel & (NC_CHUNK - 1u)))]
                      .w
-              : reinterpret_cast<const float*>(&a.bent[bi * NC_BCAP + lane].y);
+              : reinterpret_cast<const float*>(&a.bent[bi * BC + lane].y);
   const float e_w = *e_wp;
   n_arec += e_stale ? 1u : 0u;
   // The lane's cache of (depolarisation, arrival) of its first NC_ACACHE
@@ -816,7 +820,7 @@ __device__ __forceinline__ void nc_neuron_slice(const nc_step_args& a, uint32_t 
   // (its slots have room for every spike in flight to them).
   if (b_take > 64u) {
     if (64u + lane < b_take)
-      pl[pend_n + lane] = (a.bent[bi * NC_BCAP + 64u + lane].x << 8) | ((uint32_t)s & 255u);
+      pl[pend_n + lane] = (a.bent[bi * BC + 64u + lane].x << 8) | ((uint32_t)s & 255u);
     pend_n += b_take - 64u;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -971,12 +975,12 @@ __device__ __forceinline__ const float* nc_trace_tables(const nc_step_args& a) {
 
 // The neuron phase of one step for every active slice, one wave per slice,
 // WPB waves per workgroup.
-template <int WPB, bool TABS>
+template <int WPB, bool TABS, uint32_t BC>
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) void k_neuron(nc_step_args a) {
   const uint32_t blk = nc_block_id(a.xcd_swizzle + nc_have_neuron_args(a));
   const uint32_t wave = __builtin_amdgcn_readfirstlane(blk * WPB + (threadIdx.x >> 6));
   const float* tpre = TABS ? nc_trace_tables<WPB>(a) : a.t_pre;
-  nc_neuron_slice<WPB>(a, blk, wave, (int32_t)*a.chunk_off + a.chunk_i, tpre);
+  nc_neuron_slice<WPB, BC>(a, blk, wave, (int32_t)*a.chunk_off + a.chunk_i, tpre);
 }
 
 // Synapse::fire (src/NeuCor.cpp:727-738) on every outgoing synapse of every
@@ -986,6 +990,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) v
 // source), latch permitting.  Accepted spikes latch
 // depolarisation and arrival step into the target slot and join the bucket of
 // their arrival step at the target slice (or the slice's pending list).
+template <uint32_t BC>
 __device__ __forceinline__ void nc_fire_edge(const nc_step_args& a, uint32_t e, const nc_edge& ed, int32_t s,
                                              uint32_t& n_acc) {
   // a spike still in flight or in its release window (:728)
@@ -996,7 +1001,7 @@ __device__ __forceinline__ void nc_fire_edge(const nc_step_args& a, uint32_t e, 
   // the bucket place is taken before the slot is read, so that the two round
   // trips overlap
   size_t bi = 0;
-  uint32_t at = NC_BCAP;
+  uint32_t at = BC;
   if (d <= NC_NB) {
     bi = (size_t)tq * NC_NB + ((uint32_t)arr & (NC_NB - 1u));
     at = atomicAdd(&a.bcnt[bi], 1u);
@@ -1011,8 +1016,8 @@ __device__ __forceinline__ void nc_fire_edge(const nc_step_args& a, uint32_t e, 
   n.last_arr = prev != NC_NEVER ? prev : r.last_arr;
   n.arr_inh = arr * 2 + (r.arr_inh & 1);
   a.slots[ed.j] = n;
-  if (at < NC_BCAP) {
-    a.bent[bi * NC_BCAP + at] =
+  if (at < BC) {
+    a.bent[bi * BC + at] =
         make_uint2(ed.rel | ((d - 1u) << 24) | ((uint32_t)(r.arr_inh & 1) << 31), __float_as_uint(r.w));
   } else {
     // the pending list of its window, at the target slice's slot range
@@ -1027,6 +1032,7 @@ __device__ __forceinline__ void nc_fire_edge(const nc_step_args& a, uint32_t e, 
 
 // The wave takes list lst, entries first, first + per, ... (64 per load), per
 // = the waves per list.
+template <uint32_t BC>
 __device__ __forceinline__ void nc_fanout_wave(const nc_step_args& a, uint32_t blk, uint32_t lst, uint32_t first,
                                                uint32_t per, int32_t ci) {
   const uint32_t lane = threadIdx.x & 63;
@@ -1064,7 +1070,7 @@ __device__ __forceinline__ void nc_fanout_wave(const nc_step_args& a, uint32_t b
           const uint32_t i = base + lane;
           if (i < fy) {
             const nc_edge ed = a.edges[fx + i];
-            nc_fire_edge(a, fx + i, ed, s, n_acc);
+            nc_fire_edge<BC>(a, fx + i, ed, s, n_acc);
           }
         }
         continue;
@@ -1099,7 +1105,7 @@ __device__ __forceinline__ void nc_fanout_wave(const nc_step_args& a, uint32_t b
         if (i < total) {
           const uint32_t ie = rx + (i - (ic - ry));
           const nc_edge ed = a.edges[ie];
-          nc_fire_edge(a, ie, ed, s, n_acc);
+          nc_fire_edge<BC>(a, ie, ed, s, n_acc);
         }
       }
     }
@@ -1113,7 +1119,7 @@ __device__ __forceinline__ void nc_fanout_wave(const nc_step_args& a, uint32_t b
 
 // The fan-out phase of one step: WPB waves per workgroup share the step's
 // fired-slice records.
-template <int WPB>
+template <int WPB, uint32_t BC>
 __global__ __launch_bounds__(64 * WPB) void k_fanout(nc_step_args a) {
   // the arguments in one round of reads, as in nc_have_neuron_args
   uint32_t zero = 0u;
@@ -1134,7 +1140,7 @@ __global__ __launch_bounds__(64 * WPB) void k_fanout(nc_step_args a) {
     lst = wave % NC_FLISTS;
     first = wave / NC_FLISTS;
   }
-  nc_fanout_wave(a, blk, lst, first, per, (int32_t)*a.chunk_off + a.chunk_i);
+  nc_fanout_wave<BC>(a, blk, lst, first, per, (int32_t)*a.chunk_off + a.chunk_i);
 }
 
 // Grid-wide barrier of the persistent step kernel: each workgroup adds one
@@ -1170,7 +1176,7 @@ __device__ __forceinline__ void nc_grid_barrier(uint32_t* bar, uint32_t target, 
 // the grid meets at a barrier, then all waves share the fan-out.  The
 // launch's end orders it before the next step.  bar[0] counts barrier
 // arrivals in this call (zeroed at its start).
-template <int WPB>
+template <int WPB, uint32_t BC>
 __global__ __launch_bounds__(64 * WPB) void k_step(nc_step_args a, uint32_t* bar) {
   const uint32_t blk = blockIdx.x;
   const uint32_t nwaves = gridDim.x * WPB;
@@ -1178,7 +1184,7 @@ __global__ __launch_bounds__(64 * WPB) void k_step(nc_step_args a, uint32_t* bar
   const int32_t ci = (int32_t)*a.chunk_off + a.chunk_i;
   const float* tpre = nc_trace_tables<WPB>(a);
   // every wave of the grid runs the same number of slice passes
-  for (uint32_t b = 0; b < a.n_active_slices; b += nwaves) nc_neuron_slice<WPB>(a, blk, b + w0, ci, tpre);
+  for (uint32_t b = 0; b < a.n_active_slices; b += nwaves) nc_neuron_slice<WPB, BC>(a, blk, b + w0, ci, tpre);
   nc_grid_barrier(bar, ((uint32_t)ci + 1u) * gridDim.x, a.host_words + 1);
-  nc_fanout_wave(a, blk, w0 % NC_FLISTS, w0 / NC_FLISTS, nwaves / NC_FLISTS, ci);
+  nc_fanout_wave<BC>(a, blk, w0 % NC_FLISTS, w0 / NC_FLISTS, nwaves / NC_FLISTS, ci);
 }
