@@ -34,12 +34,14 @@ def timing_every(steps):
     return min(TIMING_EVERY, max(1, steps // 5))
 
 
-# Launch shapes that the live tuner chose for a plain workload on MI355X, used
-# by runs too short to tune (under 1000 timed steps). plain-1m: 1 slice per
-# workgroup with the XCD-ordered remap, 1.367 ms per 16-step trial after the
-# warm-up against 1.421 ms for the engine's default (4 slices per workgroup, no
-# remap); 20 timed steps from step 6, three runs each: 73.1 against 75.6 us per
-# step (an earlier build).
+# Launch shapes that the live tuner chooses for a plain workload's first steps on
+# MI355X, used by runs too short to tune (under 1000 timed steps). plain-1m: 1
+# slice per workgroup with the XCD-ordered remap (k_neuron), 1.038 ms per
+# 16-step trial behind 5 steps against 1.053 for the engine's default (which
+# takes k_neuron_wide of one wave in XCD order here); 20 timed steps from step
+# 6, three runs each: 69.6 against 71.5 us per step. As activity grows the
+# default is the faster one (2000 steps: 78.9 against 83.7), and what the tuner
+# chooses behind 200 steps.
 TUNED_LAUNCH = {"plain-1m": {"waves_per_block": 1, "xcd_swizzle": 1}}
 
 
@@ -258,33 +260,43 @@ def bench_batched(args):
 
     sim.synchronize()
     tune_table, tune_s = None, 0.0
-    if args.tune_steps:
+
+    def tune():
         # the engine's 38 candidate shapes, each timed from the same saved
         # state over 3 rounds (tuning takes no simulated step)
-        t_tune = time.perf_counter()
         gs = (0, min(args.tune_steps, 1024))
         cands = [dict(waves_per_block=w, xcd_swizzle=x & 1, graph_steps=g, stage_tables=x >> 1)
                  for g in gs for w in (1, 2, 4, 8) for x in range(4)]
         cands += [dict(waves_per_block=w, graph_steps=g, persistent=1) for g in gs for w in (2, 4, 8)]
         chosen, ms = sim.tune_list(cands, steps_per_trial=args.tune_steps, rounds=3)
-        tune_s = time.perf_counter() - t_tune
-        tune_table = [dict(c, median_ms=float(m)) for c, m in zip(cands, ms)]
-        for row in tune_table:
+        table = [dict(c, median_ms=float(m)) for c, m in zip(cands, ms)]
+        for row in table:
             print("[bench] tune %s" % row, file=sys.stderr, flush=True)
-        print("[bench] tuned launch %s (%.2fs)" % (chosen, tune_s), file=sys.stderr, flush=True)
-    else:
+        print("[bench] tuned launch %s" % chosen, file=sys.stderr, flush=True)
+        return table
+
+    if not args.tune_steps:
         sim.set_launch(args.waves_per_block)
-        chosen = sim.launch()
     done = 0
     t_start = time.perf_counter()
     while done < steps:
         k = min(args.chunk, steps - done)
         sim.step(k)
         done += k
+        if tune_table is None and args.tune_steps and done < steps:
+            # Behind the first chunk, at the activity that the networks keep: in
+            # their first steps little fires, and the best shape is another.
+            # The time it takes is not the run's (tune_s).
+            sim.synchronize()
+            t_tune = time.perf_counter()
+            tune_table = tune()
+            tune_s = time.perf_counter() - t_tune
+            t_start += tune_s
         if done % 5000 < args.chunk:
             sim.synchronize()
             print("[bench] batched step %d (%.1fs)" % (done, time.perf_counter() - t_start), file=sys.stderr,
                   flush=True)
+    chosen = sim.launch()
     sim.synchronize()
     elapsed = time.perf_counter() - t_start
     assert all(sim.progress(i)[1] == 0 for i in ids)
@@ -618,7 +630,11 @@ def main():
     traffic = None
     tpath = os.path.join(ROOT, "profiles", "traffic_%s.json" % args.workload)
     if os.path.exists(tpath):
-        traffic = json.load(open(tpath)).get("%s_bytes_per_launch" % dom)
+        # (of these steps in this shape only: others run other kernels at
+        # another activity)
+        for r in json.load(open(tpath))["runs"]:
+            if r["launch"] == launch_used and r["steps"] == args.steps and r["warmup"] == args.warmup:
+                traffic = r["%s_bytes_per_launch" % dom.replace("k_step", "k_neuron")]
     rate = ev["F"] / N if ev["F"] is not None else None
 
     cpu = None
