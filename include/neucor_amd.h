@@ -401,7 +401,9 @@ nc_status nc_sim_synchronize(nc_sim* sim);
  * step, 3 fan-out; 0 = off): start/stop events carried by the dispatch of
  * every `every`-th step (1 = all steps; the events cost the queue a little
  * time per timed launch).  nc_read_kernel_timing returns the timed launches
- * and their total milliseconds since the last nc_set_kernel_timing call. */
+ * and their total milliseconds since the last nc_set_kernel_timing call.
+ * While it is on, the default launch shape takes no workgroup-per-network form
+ * and makes no captured chunks: small networks run other kernels than without. */
 nc_status nc_set_kernel_timing(nc_sim* sim, int kernel_mask, uint32_t every);
 nc_status nc_read_kernel_timing(nc_sim* sim, uint32_t kernel, uint64_t* launches,
                                 double* total_ms);

@@ -209,8 +209,8 @@ struct NetMaps {
 
 // A network's device image in network-local coordinates: every array
 // nc_sim_add uploads, with slot, slice and edge indices relative to the
-// network's own first slot, slice and out-edge.  nc_sim_add relocates it
-// (host offsets for the per-neuron rows, k_relocate_edges for the edges).
+// network's own first slot, slice and out-edge.  The placing kernels
+// (k_place_net, k_place_slots, k_place_edges) relocate it.
 struct NetImage {
   uint32_t nq = 0, max_mw = 0;  // slices; most active-mask words of a lane
   uint64_t S = 0, nslots = 0, nmwords = 0, mwords_step = 0;
@@ -532,7 +532,6 @@ struct nc_sim {
   std::vector<uint32_t> slice_off_host, slice_moff_host;
   bool active_dirty = true;
   std::vector<uint32_t> slice_net_host;
-  uint64_t raster_read = 0;
   bool act_identity = false;  // active record i is slice act_q0 + i
   uint32_t act_q0 = 0;
   uint32_t net_all = ~0u;  // the only live network, or ~0u

@@ -191,7 +191,7 @@ struct nc_step_args {
   uint2* pend_cnt;         // per slice: entries in pending list 0, in list 1
   uint32_t* bcnt;          // per slice: NC_NB arrival-bucket counts (beyond BC: the rest overflowed)
   uint2* bent;             // per slice: NC_NB buckets of BC entries {slot | delay | class, weight bits}
-  uint4* acache;           // per position: (depol bits, arrival) of its first two active slots
+  uint4* acache;           // per position: its first NC_ACACHE active slots' depolarisations and arrivals' low bytes
   const uint32_t* ev_pos;  // host events of this step
   const uint8_t* ev_kind;
   uint32_t n_ev;
@@ -330,7 +330,8 @@ __device__ __forceinline__ uint32_t nc_have_neuron_args(const nc_step_args& a) {
 }
 
 // Advances the device-side chunk offset by the chunk's step count (the last
-// node of a captured chunk); k_set_u32 clears it at the start of a call.
+// node of a captured chunk, or behind a run of direct launches); k_begin clears
+// it at the start of a call.
 __global__ void k_advance(uint32_t* chunk_off, uint32_t steps) {
   if (threadIdx.x == 0) *chunk_off += steps;
 }
@@ -366,9 +367,8 @@ NC_HD uint32_t nc_slot_of(uint32_t slot_off, uint32_t l, uint32_t k) {
 
 // A network's out-edges from their uploaded network-local form (target slot,
 // target slice << 8 | delay): target slot moved by the network's first slot,
-// target slice by its first slice, the slot's active-mask word and bit from
-// the target slice's first slot and first mask word (already in place), no
-// spike latched.
+// target slice by its first slice, the slot's place in its slice from the
+// slice's first slot (already in place), no spike latched.
 __global__ __launch_bounds__(256) void k_place_edges(nc_edge* e, const uint2* jq, uint64_t n, uint32_t slot0,
                                                      uint32_t q0, const uint32_t* slice_off) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
